@@ -113,6 +113,9 @@ struct fxg_job {
   std::vector<long long> pbw_off; // per datastream: offset of its weights in d_pbw (-1: none)
   // per-subint
   DBuf d_ss, d_flags, d_ftab, d_blocks, d_weights, d_results, d_ct;
+  DBuf d_rotgroups, d_rots;       // rotations of the bands, and of each block (k_prologue)
+  DBuf d_cdesc, d_base, d_quad;   // tables of the F stage with linear rotation (fx_fstage.hip)
+  bool fstage_lin = false;        // that F stage runs: real samples, orders 0 and 1, up to kFStageMaxL points
   DBuf d_bandlist;                // global bands grouped by sample size
   int nb2 = 0, nb8 = 0;           // bands of 2-bit and 8-bit datastreams
   std::vector<DBuf> d_raw;        // staged host data per datastream
@@ -544,7 +547,8 @@ static void job_free(fxg_job* j) {
                   &j->d_ss, &j->d_flags, &j->d_ftab, &j->d_blocks, &j->d_weights, &j->d_results,
                   &j->d_spec, &j->d_V, &j->d_ct, &j->d_bandlist, &j->d_iota, &j->d_zero, &j->d_z, &j->d_rtab,
                   &j->d_pcal, &j->d_pcalaux, &j->d_pcaltone, &j->d_pcalpart, &j->d_vpart, &j->d_cexp,
-                  &j->d_eoff, &j->d_kurt, &j->d_kurtout, &j->d_kurtnz};
+                  &j->d_eoff, &j->d_kurt, &j->d_kurtout, &j->d_kurtnz, &j->d_rotgroups, &j->d_rots, &j->d_cdesc,
+                  &j->d_base, &j->d_quad};
   for (DBuf* b : bufs) b->release();
   for (DBuf& b : j->d_raw) b.release();
   if (j->copy_stream) { (void)hipStreamSynchronize(j->copy_stream); (void)hipStreamDestroy(j->copy_stream); j->copy_stream = nullptr; }
@@ -724,6 +728,25 @@ int fxg_job_create(fxg_ctx* c, const fxg_job_desc* desc, fxg_job** out) {
     if (hipMemcpy(j->d_cexp.p, ex.data(), ex.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(j->d_eoff.p, eoff.data(), sizeof(int) * eoff.size(), hipMemcpyHostToDevice) != hipSuccess)
       return fail(set_err(FXG_EHIP, "scale table upload failed"));
+  }
+  j->fstage_lin = !P.st[0].cplx && P.st[0].order != 2 && P.L <= kFStageMaxL;
+  if (j->fstage_lin) {
+    std::vector<float4> cdesc, quad(512);
+    std::vector<float2> base;
+    const float vdif[4] = {-kHiMag, -1.0f, 1.0f, kHiMag}, mark5b[4] = {-kHiMag, 1.0f, -1.0f, kHiMag};
+    fstage_quad_levels(vdif, quad.data());
+    fstage_quad_levels(mark5b, quad.data() + 256);
+    if (!fstage_lin_tables(P.L, &cdesc, &base)) return fail(set_err(FXG_EUNSUPPORTED, "FFT length"));
+    if ((rc = j->d_rotgroups.ensure(sizeof(DevRotGroup) * P.rots.size())) ||
+        (rc = j->d_rots.ensure(sizeof(DevRot) * P.rots.size() * (size_t)desc->blockspersend)) ||
+        (rc = j->d_cdesc.ensure(sizeof(float4) * cdesc.size())) ||
+        (rc = j->d_base.ensure(sizeof(float2) * base.size())) || (rc = j->d_quad.ensure(sizeof(float4) * quad.size())))
+      return fail(rc);
+    if (hipMemcpy(j->d_rotgroups.p, P.rots.data(), sizeof(DevRotGroup) * P.rots.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(j->d_cdesc.p, cdesc.data(), sizeof(float4) * cdesc.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(j->d_base.p, base.data(), sizeof(float2) * base.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(j->d_quad.p, quad.data(), sizeof(float4) * quad.size(), hipMemcpyHostToDevice) != hipSuccess)
+      return fail(set_err(FXG_EHIP, "F-stage table upload failed"));
   }
   if (P.vpart_elems > 0) {
     if ((rc = j->d_vpart.ensure(sizeof(float2) * (size_t)P.vpart_elems))) return fail(rc);
@@ -1044,7 +1067,8 @@ static int launch_front(fxg_job* j, const LaunchShape& sh, hipStream_t s) {
   if ((rc = j->ev_end())) return rc;
   if ((rc = j->ev_begin(FXG_STAGE_PROLOGUE))) return rc;
   HIPCHK(launch_prologue(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_flags.as<int>(),
-                         j->d_ftab.as<int2>(), j->desc.blockspersend, j->d_blocks.as<DevBlock>(), P.nds, s));
+                         j->d_ftab.as<int2>(), j->desc.blockspersend, j->d_blocks.as<DevBlock>(), P.nds,
+                         j->d_rotgroups.as<DevRotGroup>(), j->fstage_lin ? j->d_rots.as<DevRot>() : nullptr, s));
   if ((rc = j->ev_end())) return rc;
   return 0;
 }
@@ -1079,6 +1103,18 @@ static void fill_fstage_args(fxg_job* j, FStageArgs* fa) {
   fa->cexp = j->d_cexp.p ? j->d_cexp.as<signed char>() : nullptr;
   fa->gstride = j->gstride;
   fa->bstride = j->bstride;
+  fa->rots = j->d_rots.as<DevRot>();
+  fa->cdesc = j->d_cdesc.as<float4>();
+  fa->base = j->d_base.as<float2>();
+  fa->quad = j->d_quad.as<float4>();
+}
+
+// the F stage of nbands bands (fa.bandlist) of nbits-bit samples over nblocks blocks from fa.chunk0
+static hipError_t launch_job_fstage(const fxg_job* j, int nbits, const FStageArgs& fa, int nbands, int nblocks,
+                                    hipStream_t s) {
+  const Plan& P = j->plan;
+  if (j->fstage_lin) return launch_fstage_lin(P.L, nbits, fa, nbands, nblocks, s);
+  return launch_fstage(P.L, nbits, P.st[0].cplx, fa, nbands, nblocks, s);
 }
 
 // identity of a subintegration's inputs: the prepared state is reused while it matches
@@ -1125,11 +1161,11 @@ static int launch_back(fxg_job* j, float* dres, hipStream_t s) {
     if ((rc = j->ev_begin(FXG_STAGE_FSTAGE))) return rc;
     if (j->nb2) {
       fa.bandlist = j->d_bandlist.as<int>();
-      HIPCHK(launch_fstage(P.L, 2, P.st[0].cplx, fa, j->nb2, cn, s));
+      HIPCHK(launch_job_fstage(j, 2, fa, j->nb2, cn, s));
     }
     if (j->nb8) {
       fa.bandlist = j->d_bandlist.as<int>() + j->nb2;
-      HIPCHK(launch_fstage(P.L, 8, P.st[0].cplx, fa, j->nb8, cn, s));
+      HIPCHK(launch_job_fstage(j, 8, fa, j->nb8, cn, s));
     }
     if ((rc = j->ev_end())) return rc;
     if (j->kurt_on) {
@@ -1667,7 +1703,7 @@ int fxg_station_process_block(fxg_job* j, const fxg_subint_desc* sub, const fxg_
   fill_fstage_args(j, &fa);
   fa.chunk0 = block;
   fa.bandlist = j->d_iota.as<int>() + P.st[ds].band0;
-  HIPCHK(launch_fstage(P.L, P.st[ds].nbits, P.st[ds].cplx, fa, P.st[ds].nchan, 1, j->stream));
+  HIPCHK(launch_job_fstage(j, P.st[ds].nbits, fa, P.st[ds].nchan, 1, j->stream));
   HIPCHK(hipStreamSynchronize(j->stream));
   j->ev_collect();
   j->have_subint = 1;

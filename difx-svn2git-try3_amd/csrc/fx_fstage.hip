@@ -1,0 +1,472 @@
+// fx_fstage.hip — the F stage of real-sampled data with linear (or post-F)
+// fringe rotation, transforms up to 16384 points (mode.cpp:909-1310): level
+// decoding, fringe rotation, FFT, sideband select, fractional-sample rotation.
+#include <hip/hip_runtime.h>
+#include "fx_kernels.h"
+#include "fx_device.h"
+#include "fx_fft.h"
+#include "fx_spectra.h"
+#include <cmath>
+#include <vector>
+
+namespace fxg {
+
+// The passes of one length: R1 = 16 P in the first, 16 in a middle one from
+// 2048 points on, RL = 16 or 8 in the last; NTF threads and NB blocks per
+// workgroup of NT threads; the per-block table (pass 1: CP entries for each
+// of the P thread sets; the last pass's four powers and the eight channel
+// steps; eight twiddles for each bin of the middle pass).
+template <int L> struct FsShape {
+  static constexpr int LOG = L == 128 ? 7 : L == 256 ? 8 : L == 512 ? 9 : L == 1024 ? 10 : L == 2048 ? 11
+                           : L == 4096 ? 12 : L == 8192 ? 13 : 14;
+  static constexpr int P = LOG % 4 == 1 ? 2 : LOG % 4 == 2 ? 4 : 1;
+  static constexpr int R1 = 16 * P, J1 = L / R1, RL = LOG % 4 == 3 ? 8 : 16;
+  static constexpr bool MID = LOG >= 11;
+  static constexpr int J2 = MID ? J1 / 16 : 16;
+  static constexpr int NTF = L / 16, NB = NTF >= 128 ? 1 : 256 / NTF, NT = NTF * NB;
+  static constexpr int CP = P == 1 ? 8 : P == 2 ? 10 : 12, LAST = P * CP, MIDOFF = LAST + 12;
+  static constexpr int NE = MIDOFF + (MID ? 8 * R1 : 0);
+};
+
+// Validity of the 32 / BITS consecutive samples from t of one band, one bit
+// each (the rule of sample_value: frames by their valid byte range, blanked
+// bands, validend, the end of the data)
+template <int COUNT>
+__device__ __forceinline__ unsigned valid_samples(const DevStation& S, const DevStationSub& Q,
+                                                  const int2* __restrict__ ftab, long long t, long long validend,
+                                                  int band) {
+  unsigned m = 0u;
+  const long long end = min(t + COUNT, validend);
+  long long u = t < 0 ? 0 : t;
+  while (u < end) {
+    const long long f = u / S.framesamples;
+    if (f >= Q.nframes) break;
+    const long long base = f * (long long)S.framesamples;
+    const long long fe = min(end, base + S.framesamples);
+    const int2 z = ftab[Q.fbase + f];
+    const bool blank = Q.fblank && ((Q.fblank[f] >> band) & 1ull);
+    if (z.x < z.y && !blank) {
+      const long long g0 = ((long long)z.x + S.groupbytes - 1) / S.groupbytes;
+      const long long g1 = ((long long)z.y + S.groupbytes - 1) / S.groupbytes;
+      const long long a = max(u, base + g0 * S.groupsamples), b = min(fe, base + g1 * S.groupsamples);
+      if (b > a) m |= (((1u << (int)(b - a)) - 1u) << (int)(a - t));
+    }
+    u = fe;
+  }
+  return m;
+}
+
+// 16 bits to 16 two-bit fields (each bit doubled)
+__device__ __forceinline__ unsigned double_bits16(unsigned m) {
+  m = (m | (m << 8)) & 0x00FF00FFu;
+  m = (m | (m << 4)) & 0x0F0F0F0Fu;
+  m = (m | (m << 2)) & 0x33333333u;
+  m = (m | (m << 1)) & 0x55555555u;
+  return m * 3u;
+}
+
+// Four rows of 16 two-bit samples to quads: byte m of a[t] becomes the four
+// rows' sample 4 m + t, row 0 in the low bits.
+__device__ __forceinline__ void quads2(unsigned* a) {
+  unsigned t;
+  t = ((a[0] >> 2) ^ a[1]) & 0x33333333u; a[1] ^= t; a[0] ^= t << 2;
+  t = ((a[2] >> 2) ^ a[3]) & 0x33333333u; a[3] ^= t; a[2] ^= t << 2;
+  t = ((a[0] >> 4) ^ a[2]) & 0x0F0F0F0Fu; a[2] ^= t; a[0] ^= t << 4;
+  t = ((a[1] >> 4) ^ a[3]) & 0x0F0F0F0Fu; a[3] ^= t; a[1] ^= t << 4;
+}
+// Four rows of four bytes to quads: byte i of a[t] becomes row i's byte t.
+__device__ __forceinline__ void quads8(unsigned* a) {
+  const unsigned lo01 = __builtin_amdgcn_perm(a[1], a[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(a[1], a[0], 0x07030602u);
+  const unsigned lo23 = __builtin_amdgcn_perm(a[3], a[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(a[3], a[2], 0x07030602u);
+  a[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+  a[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+  a[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+  a[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+}
+
+// ---------------------------------------------------------------------------
+// k_fstage_lin<L, NBITS>: L = R1 x (16) x RL points, 16 per thread.
+//
+// What bounds it: FP32 VALU issue (wave64, four cycles an instruction), so it
+// is built for few instructions:
+//   - the fringe rotation is in the twiddles (fx_fft.h), whose per-block
+//     values are two dozen to 60 sines of FP64 phases, one per thread;
+//   - the first pass reads samples as quads, the four samples a quarter of
+//     the block apart, whose first two butterfly stages have real inputs: one
+//     LDS byte and one 16-byte lookup decode four samples;
+//   - R1 = 16 P: pass 1 has radix 32 or 64 where L is an odd power of two or
+//     four times a power of 16, P threads sharing one input set (each forms
+//     the outputs q = P q' + p), so that no length but 8 x 16^n needs a pass
+//     of smaller radix: two LDS exchanges at 2048 points and more, one below;
+//   - the last pass forms only the sideband's half of the outputs (the lower
+//     sideband's sign rides on w).
+// Exchanges are laid out so that both sides hit all banks with immediate
+// offsets: the one into the middle pass by exchanging pieces of J2 values
+// between neighbouring rows, the one into the last pass by a row pad.
+// Against the kernel with rotator tables, padded twiddle products and one
+// radix-2 pass more (rocprofv3, ms): 32 stations, 8192 points, 16.8 Gsamples
+// 33.4 -> 26.2; 16384 points, 8.2 Gsamples 24.0 -> 18.4; 2048 points, 1.34
+// Gsamples 3.23 -> 2.80; 512 points, 8-bit, 0.92 Gsamples 3.53 -> 1.37.
+// ---------------------------------------------------------------------------
+template <int L, int NBITS>
+__global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) {
+  using Sh = FsShape<L>;
+  constexpr int P = Sh::P, R1 = Sh::R1, J1 = Sh::J1, J2 = Sh::J2, RL = Sh::RL, NTF = Sh::NTF, NB = Sh::NB, NT = Sh::NT;
+  constexpr bool MID = Sh::MID;
+  constexpr int QW = NBITS == 8 ? L / 4 : L / 16;         // staged quad words of one block
+  constexpr int NL = L / RL, LPAD = 32 / RL;               // bins entering the last pass, and its row pad
+  // a block within one wavefront: its quads lie in the exchange buffer, read
+  // before that wavefront's first exchange write
+  constexpr bool RAWOWN = NTF > 64 || NTF < 32;
+  struct Smem {
+    float2 tab[NB][Sh::NE];
+    float4 quad[NBITS == 2 ? 256 : 0];
+    unsigned raw_own[RAWOWN ? NB * QW : 0];
+    unsigned ok_own[RAWOWN && NBITS == 2 ? NB * QW : 0];
+    float2 buf[NB][L + 32 + (NTF < 32 ? 1 : 0)];
+  };
+  __shared__ __align__(16) Smem sm;
+
+  const int tid = threadIdx.x;
+  const int fi = NB == 1 ? 0 : tid / NTF, t = NB == 1 ? tid : tid % NTF;
+  unsigned* const raw = RAWOWN ? sm.raw_own + fi * QW : (unsigned*)sm.buf[fi];
+  unsigned* const ok = RAWOWN ? sm.ok_own + fi * QW : (unsigned*)sm.buf[fi] + QW;
+  // block groups within the chunk: workgroups are dealt to the 8 XCDs
+  // round-robin, so consecutive blocks go to one XCD (its L2 merges the
+  // halves of the lines that neighbouring blocks write in the grouped layout)
+  const int grp = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  if (grp * NB >= A.nchunk) return;
+  const int cbx = grp * NB + fi;
+  const bool mine = NB == 1 || cbx < A.nchunk;
+  const int cb = mine ? cbx : A.nchunk - 1;
+  const int gband = A.bandlist ? A.bandlist[blockIdx.y] : blockIdx.y;
+  const DevBand& B = A.bands[gband];
+  const DevStationSub& Q = A.ss[B.station];
+  const DevRot& R = A.rots[(long long)B.rot * A.nblocks_subint + A.chunk0 + cb];
+  constexpr int C = L / 2;
+  const long long outbase = B.specoff + (long long)cb * A.bstride;
+  const bool dead = R.status != 0;
+  if (NB == 1 && dead) {
+    zero_spec(A.spectra, A.prec, outbase, C, A.gstride, tid, NT);
+    return;
+  }
+
+  // ---- the block's samples of this band: four rows a quarter block apart
+  constexpr int GROUPS = NBITS == 8 ? L / 16 : L / 64;
+  unsigned a[4];
+  if (t < GROUPS) {
+    const long long bit0 = (long long)(dead ? 0 : R.t0) * NBITS;
+    const unsigned* src = (const unsigned*)(A.ct + Q.ctbase + (long long)B.band * Q.ctstride);
+    const long long nwords = Q.ctstride >> 2;
+    const long long w0 = (bit0 >> 5) + t;
+    const int sh = (int)(bit0 & 31);
+    unsigned lo[4], hi[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      const long long w = w0 + m * GROUPS;
+      lo[m] = w < nwords ? src[w] : 0u;
+      hi[m] = w + 1 < nwords ? src[w + 1] : 0u;
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++) a[m] = __builtin_amdgcn_alignbit(hi[m], lo[m], sh);
+  }
+  // ---- this block's twiddles and fractional-sample steps
+  {
+    const double delta = R.delta, theta = R.theta;
+    for (int i = NTF - 1 - t; i < Sh::NE; i += NTF) {
+      const float4 d = A.cdesc[i];
+      double ph = theta * (double)d.y - (delta * (double)d.x + (double)d.z);
+      if (i == Sh::LAST + 3 && B.lsb) ph += 0.5;           // the lower sideband keeps a - w b
+      sm.tab[fi][i] = exact_rotator(ph);
+    }
+  }
+  if (NBITS == 2)
+    for (int i = tid; i < 256; i += NT) sm.quad[i] = A.quad[B.levels * 256 + i];
+  const bool fast = R.allvalid != 0 || dead;
+  if (t < GROUPS) {
+    if (NBITS == 8) {
+#pragma unroll
+      for (int m = 0; m < 4; m++) a[m] ^= 0x80808080u;     // signed levels, 0 = none
+    }
+    if (!fast) {
+      // a blanked sample has no 2-bit code: its validity is staged beside it;
+      // 8-bit samples are cleared
+      const DevStation& S = A.st[B.station];
+      unsigned v[4];
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        const long long ts = R.t0 + (long long)(m * GROUPS + t) * (32 / NBITS);
+        v[m] = valid_samples<32 / NBITS>(S, Q, A.ftab, ts, R.validend, B.band);
+        if (NBITS == 2) {
+          v[m] = double_bits16(v[m]);
+        } else {
+          const unsigned by = ((v[m] & 1u) | ((v[m] & 2u) << 7) | ((v[m] & 4u) << 14) | ((v[m] & 8u) << 21)) * 255u;
+          a[m] &= by;
+        }
+      }
+      if (NBITS == 2) {
+        quads2(v);
+        *(uint4*)&ok[4 * t] = make_uint4(v[0], v[1], v[2], v[3]);
+      }
+    }
+    if (NBITS == 8) quads8(a); else quads2(a);
+    *(uint4*)&raw[4 * t] = make_uint4(a[0], a[1], a[2], a[3]);
+  }
+  __syncthreads();
+
+  // workgroup barrier, or (a block's threads within one wavefront) only an
+  // order for the compiler: LDS accesses of a wavefront complete in order
+  auto sync = [] {
+    if (NTF > 64) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  };
+  float2* const buf = sm.buf[fi];
+  const float2* const tab = sm.tab[fi];
+
+  // ---- pass 1: decode, radix R1 (this thread's 16 of the R1 outputs)
+  {
+    const int p = t / J1, j = t % J1;
+    const float2* c = tab + p * Sh::CP;
+    Tw16 w;
+    w.w8 = c[0]; w.w4 = c[1]; w.w2 = c[2]; w.w2h = c[3]; w.w1 = c[4]; w.w1a = c[5]; w.w1b = c[6]; w.w1c = c[7];
+    // Quads of samples j + r J1, QN at a time, all their LDS reads in flight
+    // together: bytes within a group of 16 in the order of quads2.
+    constexpr int NQ = R1 / 4, QN = NQ > 8 ? 8 : NQ;
+    auto quads_at = [&](int r0, float4* x) {
+      if (NBITS == 8) {
+        unsigned q[QN];
+#pragma unroll
+        for (int r = 0; r < QN; r++) q[r] = raw[j + (r0 + r) * J1];
+#pragma unroll
+        for (int r = 0; r < QN; r++)
+          x[r] = make_float4((float)(signed char)(q[r] & 0xFFu), (float)(signed char)((q[r] >> 8) & 0xFFu),
+                             (float)(signed char)((q[r] >> 16) & 0xFFu), (float)(signed char)(q[r] >> 24));
+      } else {
+        const int at0 = J1 >= 16 ? (j & ~15) + ((j & 3) << 2) + ((j >> 2) & 3) : ((j & 3) << 2) + (j >> 2);
+        auto at = [&](int r) { return at0 + (J1 >= 16 ? r * J1 : 16 * (r >> 1) + 2 * (r & 1)); };
+        unsigned q[QN];
+#pragma unroll
+        for (int r = 0; r < QN; r++) q[r] = ((const unsigned char*)raw)[at(r0 + r)];
+#pragma unroll
+        for (int r = 0; r < QN; r++) x[r] = sm.quad[q[r]];
+        if (!fast) {
+#pragma unroll
+          for (int r = 0; r < QN; r++) {
+            const unsigned m = ((const unsigned char*)ok)[at(r0 + r)];
+            x[r].x = m & 1u ? x[r].x : 0.0f;
+            x[r].y = m & 4u ? x[r].y : 0.0f;
+            x[r].z = m & 16u ? x[r].z : 0.0f;
+            x[r].w = m & 64u ? x[r].w : 0.0f;
+          }
+        }
+      }
+    };
+    float2 v[16];
+    if (P == 1) {
+      // samples r, r + 4, r + 8, r + 12
+      float4 xq[QN];
+      quads_at(0, xq);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float4 x = xq[r];
+        const float s0 = w.w8.y * x.z, s1 = w.w8.y * x.w;
+        v[r] = make_float2(__builtin_fmaf(w.w8.x, x.z, x.x), s0);
+        v[r + 8] = make_float2(__builtin_fmaf(-w.w8.x, x.z, x.x), -s0);
+        v[r + 4] = make_float2(__builtin_fmaf(w.w8.x, x.w, x.y), s1);
+        v[r + 12] = make_float2(__builtin_fmaf(-w.w8.x, x.w, x.y), -s1);
+      }
+    } else if (P == 2) {
+      // samples r, r + 8, r + 16, r + 24 of 32
+      const float2 g2 = c[8], g3 = c[9];
+      float4 xq[QN];
+      quads_at(0, xq);
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        const float4 x = xq[r];
+        const float2 e = make_float2(__builtin_fmaf(g2.x, x.z, x.x), g2.y * x.z);
+        const float2 s = make_float2(__builtin_fmaf(g3.x, x.w, __builtin_fmaf(w.w8.x, x.y, e.x)),
+                                     __builtin_fmaf(g3.y, x.w, __builtin_fmaf(w.w8.y, x.y, e.y)));
+        v[r] = s;
+        v[r + 8] = make_float2(__builtin_fmaf(2.0f, e.x, -s.x), __builtin_fmaf(2.0f, e.y, -s.y));
+      }
+    } else {
+      // samples r, r + 16, r + 32, r + 48 of 64
+      const float2 g1 = c[8], g2 = c[9], g3 = c[10];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        float4 xq[QN];
+        quads_at(8 * h, xq);
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+          const float4 x = xq[r];
+          v[8 * h + r] = make_float2(__builtin_fmaf(g3.x, x.w, __builtin_fmaf(g2.x, x.z, __builtin_fmaf(g1.x, x.y, x.x))),
+                                     __builtin_fmaf(g3.y, x.w, __builtin_fmaf(g2.y, x.z, g1.y * x.y)));
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 8; r++) bfly(v[r], v[r + 8], w.w8);
+    }
+    dft16_stage2(v, w);
+    dft16_stage3(v, w);
+    dft16_stage4<false>(v, w);
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int k = P * q + p;
+      const int slot = MID ? k * J1 + (j ^ (J2 * (k % (32 / J2)))) : j * (NL + LPAD) + k;
+      buf[slot] = v[bitrev4(q)];
+    }
+  }
+
+  // ---- middle pass: radix 16 from R1 to 16 R1 bins
+  if (MID) {
+    sync();
+    const int j = t % J2, k = t / J2;
+    Tw16 w;
+    const float2* c = tab + Sh::MIDOFF + 8 * k;
+    w.w8 = c[0]; w.w4 = c[1]; w.w2 = c[2]; w.w2h = c[3]; w.w1 = c[4]; w.w1a = c[5]; w.w1b = c[6]; w.w1c = c[7];
+    constexpr int NX = 32 / J2;
+    int off[NX];
+#pragma unroll
+    for (int i = 0; i < NX; i++) off[i] = k * J1 + j + J2 * (i ^ (k % NX));
+    float2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = buf[off[r % NX] + J2 * (r - r % NX)];
+    dft16_tw<false>(v, w);
+    sync();
+    float2* op = buf + j * (NL + LPAD) + k;
+#pragma unroll
+    for (int q = 0; q < 16; q++) op[R1 * q] = v[bitrev4(q)];
+  }
+
+  // ---- last pass (radix RL), the sideband's half; fractional-sample rotation
+  float2 w[RL == 16 ? 4 : 6];
+#pragma unroll
+  for (int i = 0; i < (RL == 16 ? 4 : 6); i++) w[i] = A.base[i * NTF + t];
+  // channel t + e L/16: this thread's phase (FP64, in turns) times E[e]
+  float2 F;
+  {
+    const float s = dead ? 0.0f : (NBITS == 8 ? A.scale * (float)(1.0 / 3.3) : A.scale);
+    F = cmulx(exact_rotator(R.phase + R.theta * (double)t), make_float2(B.polre * s, B.polim * s));
+  }
+  sync();
+  float2 x[8];                                             // channel t + e L/16
+  const float2* cl = tab + Sh::LAST;
+  if (RL == 16) {
+    Tw16 tw;
+    tw.w8 = cmulx(w[0], cl[0]); tw.w4 = cmulx(w[1], cl[1]); tw.w2 = cmulx(w[2], cl[2]); tw.w1 = cmulx(w[3], cl[3]);
+    tw16_multiples(tw);
+    float2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = buf[r * (NL + LPAD) + t];
+    dft16_tw<true>(v, tw);
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[e] = v[bitrev4(e)];
+  } else {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      float2 v[8];
+#pragma unroll
+      for (int r = 0; r < 8; r++) v[r] = buf[r * (NL + LPAD) + t + u * NTF];
+      dft8_tw<true>(v, cmulx(w[u], cl[1]), cmulx(w[2 + u], cl[2]), cmulx(w[4 + u], cl[3]));
+#pragma unroll
+      for (int q = 0; q < 4; q++) x[u + 2 * q] = v[bitrev3(q)];
+    }
+  }
+  if (!mine) return;
+  const float2* E = tab + Sh::LAST + 4;
+  const long long c0 = cidx(t, A.gstride), cstep = (NTF / 16) * A.gstride;
+  auto store = [&](auto out) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const long long at = NTF % 16 == 0 ? c0 + e * cstep : cidx(t + e * NTF, A.gstride);
+      put_spec(out, at, t + e * NTF, cmulx(x[e], cmulx(F, E[e])));
+    }
+  };
+  if (A.prec == FXG_XMAC_FP32) store((float2*)A.spectra + outbase);
+  else if (A.prec == FXG_XMAC_FP16) store((__half2*)A.spectra + outbase);
+  else if (A.prec == FXG_XMAC_FP8) store(Fp8Out{(unsigned short*)A.spectra + outbase, A.cexp + (long long)gband * C});
+  else store((__hip_bfloat162*)A.spectra + outbase);
+}
+
+// ---------------------------------------------------------------------------
+// host side: the tables of one length
+// ---------------------------------------------------------------------------
+template <int L>
+static void fill_tables(std::vector<float4>* cdesc, std::vector<float2>* base) {
+  using Sh = FsShape<L>;
+  cdesc->assign(Sh::NE, make_float4(0.f, 0.f, 0.f, 0.f));
+  // entry = e^{2 pi i (theta y - delta x - z)}
+  auto set = [&](int i, double x, double z, double y = 0.0) {
+    (*cdesc)[i] = make_float4((float)x, (float)y, (float)(z - std::floor(z)), 0.f);
+  };
+  // the eight twiddles of a radix-16 pass to N bins at bin k (w = e^{-2 pi i (k + d)/N})
+  auto tw16 = [&](int i, int N, double k) {
+    const int m[8] = {8, 4, 2, 2, 1, 1, 1, 1};
+    const double add[8] = {0, 0, 0, 1.0 / 8, 0, 1.0 / 16, 2.0 / 16, 3.0 / 16};
+    for (int e = 0; e < 8; e++) set(i + e, (double)(L / N) * m[e], k * m[e] / N + add[e]);
+  };
+  for (int p = 0; p < Sh::P; p++) {
+    tw16(p * Sh::CP, 16 * Sh::P, p);
+    for (int m = 1; m < 4 && Sh::P > 1; m++) {
+      // samples a quarter of the block apart (m = 1 is w^8 where P = 2)
+      if (Sh::P == 2 && m == 1) continue;
+      set(p * Sh::CP + (Sh::P == 2 ? 6 + m : 7 + m), (double)(L / 4) * m, 0.25 * p * m);
+    }
+  }
+  const int ml[4] = {8, 4, 2, 1};
+  for (int i = 0; i < 4; i++) set(Sh::LAST + i, ml[i], 0.0);
+  for (int e = 0; e < 8; e++) set(Sh::LAST + 4 + e, 0.0, 0.0, (double)(L / 16) * e);
+  if (Sh::MID)
+    for (int k = 0; k < Sh::R1; k++) tw16(Sh::MIDOFF + 8 * k, 16 * Sh::R1, k);
+  // last pass at d = 0: powers 8, 4, 2, 1 (radix 16) or 4, 2, 1 of its two
+  // butterflies (radix 8), one entry per thread
+  base->clear();
+  const int nb = Sh::RL == 16 ? 4 : 3, nu = Sh::RL == 16 ? 1 : 2;
+  for (int i = 0; i < nb; i++)
+    for (int k = 0; k < nu * Sh::NTF; k++) {
+      const double ang = -kTwoPi * (double)k * (1 << (nb - 1 - i)) / L;
+      base->push_back(make_float2((float)std::cos(ang), (float)std::sin(ang)));
+    }
+}
+
+#define FX_LENGTHS(X) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192) X(16384)
+
+bool fstage_lin_tables(int L, std::vector<float4>* cdesc, std::vector<float2>* base) {
+  switch (L) {
+#define X(Lv) case Lv: fill_tables<Lv>(cdesc, base); return true;
+    FX_LENGTHS(X)
+#undef X
+  }
+  return false;
+}
+
+void fstage_quad_levels(const float* lut, float4* out) {
+  for (int b = 0; b < 256; b++)
+    out[b] = make_float4(lut[b & 3], lut[(b >> 2) & 3], lut[(b >> 4) & 3], lut[(b >> 6) & 3]);
+}
+
+hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream) {
+  if (nbits != 2 && nbits != 8) return hipErrorInvalidValue;
+  FStageArgs b = a;
+  b.nchunk = nblocks;
+  switch (L) {
+#define X(Lv)                                                                                                       \
+    case Lv: {                                                                                                      \
+      const dim3 grid((unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8), nbands);         \
+      if (nbits == 2) hipLaunchKernelGGL((k_fstage_lin<Lv, 2>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);         \
+      else hipLaunchKernelGGL((k_fstage_lin<Lv, 8>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);                    \
+      break;                                                                                                        \
+    }
+    FX_LENGTHS(X)
+#undef X
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+}  // namespace fxg

@@ -27,6 +27,7 @@ struct DevStation {
   int cplx;             // complex samples (real part in the low nbits of each unit)
   int unitbits;         // bits of one band's sample: nbits, or 2 nbits if complex
   int edv4;             // INTERLACEDVDIF: EDV4 per-band validity and weights
+  int rot0, nrot;       // the datastream's rotations (DevRotGroup) in the job's list
   int pad0;
   double sampletime, bw;
   float lut[4];         // 2-bit level table (VDIF or Mark5B order)
@@ -40,6 +41,25 @@ struct DevBand {
   double lofreq, clock, clockdelta, looffset;   // lofreq: the fringe rotator's LO
   long long specoff;    // element offset of this band in the spectra buffer
   float polre, polim;   // polarisation phase correction of the band's spectrum (1, 0: none)
+  int rot;              // the band's rotation (DevRotGroup) in the job's list
+  int levels;           // 2-bit level order: 0 VDIF, 1 Mark5B
+};
+
+// ---- the distinct rotations of a datastream's bands: the bands of one
+// recorded frequency share theirs (with a polarisation clock offset, those of
+// the same sign do)
+struct DevRotGroup {
+  double lofreq, clock, clockdelta, looffset;
+  int useB, lsb, dsb, pad;
+};
+
+// ---- rotation of one (DevRotGroup, block), what the F stage with linear or
+// post-F rotation reads of a block: sample n turns by -(phase0 + delta n),
+// channel c by theta c + theta0, in turns; phase = theta0 - phase0
+struct DevRot {
+  double delta, phase, theta;
+  long long validend;   // samples at or after this index decode as zero
+  int t0, status, allvalid, pad;
 };
 
 // ---- per subintegration, per datastream ----------------------------------
@@ -140,6 +160,7 @@ struct Plan {
   int nbands_total = 0;                                // recorded bands over all datastreams
   std::vector<DevStation> st;
   std::vector<DevBand> bands;
+  std::vector<DevRotGroup> rots;
   std::vector<XmacFreq> xf;                            // XMAC frequencies
   std::vector<int> xf_of_freq;                         // freq -> index in xf or -1
   long long vsize = 0;                                 // complex elements of V

@@ -3,6 +3,7 @@
 // fx_pcal.hip, fx_mux.hip and fx_kurtosis.hip).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <vector>
 #include "fx_internal.h"
 
 namespace fxg {
@@ -47,6 +48,12 @@ struct FStageArgs {
   const signed char* cexp;    // fp8: power-of-two scale exponent per [global band][channel]
   long long gstride;          // spectra layout (cidx)
   int bstride;
+  // linear and post-F rotation, transforms up to kFStageMaxL points:
+  const DevRot* rots;         // [rotation][block of the subintegration]
+  const float4* cdesc;        // per-block table entries e^{2 pi i (theta y - delta x - z)}
+  const float2* base;         // last-pass twiddles at d = 0, per thread
+  const float4* quad;         // levels of four 2-bit samples by their byte: VDIF, Mark5B
+  int nchunk;                 // blocks of the launch
 };
 
 struct XmacArgs {
@@ -127,9 +134,15 @@ hipError_t launch_cornerturn(const DevStation* st, const DevStationSub* ss, unsi
                              long long maxframes, int maxdatabytes, int fastW, long long maxsamples,
                              hipStream_t stream);
 hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const int* flags,
-                           const int2* ftab, int nblocks, DevBlock* out, int nst, hipStream_t stream);
+                           const int2* ftab, int nblocks, DevBlock* out, int nst, const DevRotGroup* groups,
+                           DevRot* rots, hipStream_t stream);
 // cplx: complex samples (L = nchan, every output of the transform kept)
 hipError_t launch_fstage(int L, int nbits, int cplx, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
+// linear and post-F rotation of real samples, L <= kFStageMaxL; its tables for
+// one length, and the levels of four 2-bit samples by their byte (256 entries)
+hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
+bool fstage_lin_tables(int L, std::vector<float4>* cdesc, std::vector<float2>* base);
+void fstage_quad_levels(const float* lut, float4* out);
 hipError_t launch_unpack(const DevStation* st, const DevStationSub* ss, const int2* ftab, const float* lut8,
                          long long first, int nsamp, int nchan, long long validend, float* out,
                          hipStream_t stream);

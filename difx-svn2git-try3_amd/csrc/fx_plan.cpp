@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cmath>
 #include <numeric>
+#include <cstring>
 #include <map>
 #include <array>
 
@@ -448,6 +449,7 @@ int build_plan(const fxg_job_desc* d, Plan* p, std::string* err) {
       if (ds.recfreq_clockoffsetdelta_us[i] != 0.0) st.deltapol = 1;
     }
     st.band0 = band;
+    st.rot0 = (int)P.rots.size();
     if (st.format == FXG_FORMAT_VDIF) { st.lut[0] = -kHiMag; st.lut[1] = -1.0f; st.lut[2] = 1.0f; st.lut[3] = kHiMag; }
     else { st.lut[0] = -kHiMag; st.lut[1] = 1.0f; st.lut[2] = -1.0f; st.lut[3] = kHiMag; }
     P.st.push_back(st);
@@ -483,9 +485,16 @@ int build_plan(const fxg_job_desc* d, Plan* p, std::string* err) {
           b.polim = (float)-std::sin(degphase * M_PI / 180.0);
         }
       }
+      b.levels = st.format == FXG_FORMAT_VDIF ? 0 : 1;
+      // the band's rotation: one of this datastream's, or a new one
+      DevRotGroup rg{b.lofreq, b.clock, b.clockdelta, b.looffset, b.useB, b.lsb, b.dsb, 0};
+      b.rot = st.rot0;
+      while (b.rot < (int)P.rots.size() && std::memcmp(&P.rots[b.rot], &rg, sizeof rg) != 0) b.rot++;
+      if (b.rot == (int)P.rots.size()) P.rots.push_back(rg);
       P.bands.push_back(b);
       band++;
     }
+    P.st[s].nrot = (int)P.rots.size() - P.st[s].rot0;
   }
   P.nbands_total = band;
 
@@ -770,7 +779,8 @@ int64_t plan_device_bytes(const Plan& p, const fxg_job_desc* d) {
   long long spec = (long long)p.nbands_total * p.C * p.chunk_blocks * spectrum_bytes(d->xmac_precision);
   if (d->xmac_precision == FXG_XMAC_FP8) spec += (long long)p.nbands_total * p.C;   // the scale exponents
   long long v = p.vsize * 8;
-  long long blocks = (long long)p.nds * d->blockspersend * (long long)sizeof(DevBlock);
+  long long blocks = ((long long)p.nds * (long long)sizeof(DevBlock) + (long long)p.rots.size() * (long long)sizeof(DevRot)) *
+                     d->blockspersend;
   long long res = p.info.result_length * 8;
   long long tables = (long long)p.segs.size() * sizeof(DevSeg) + p.bands.size() * sizeof(DevBand) + (1 << 20);
   long long z = p.L > 16384 ? (long long)p.nbands_total * p.zcap * ((long long)p.L + p.rtabn) * 8 : 0;

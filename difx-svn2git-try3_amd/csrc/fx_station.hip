@@ -3,9 +3,11 @@
 //               format_vdif.c:4009-4060, blanker_mark5.c:53-165, 282-312)
 //   k_prologue  FP64 block geometry + data weight      (mode.cpp:649-813,
 //               mk5mode.cpp:104-177)
-//   k_fstage<L> LUT unpack -> fringe rotation -> L-point FP32 Stockham FFT
-//               -> sideband select -> fractional-sample rotation -> spectra
-//               (mode.cpp:909-1310)
+//   k_fstage<L> LUT unpack -> quadratic fringe rotation -> L-point FP32
+//               Stockham FFT -> sideband select -> fractional-sample rotation
+//               -> spectra (mode.cpp:909-1310); k_fstage_c complex samples;
+//               k_bigfft_a/b transforms above 16384 points.  Real samples
+//               with linear or post-F rotation: fx_fstage.hip
 //   k_unpack    standalone Mk5Mode::unpack equivalent
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -13,6 +15,7 @@
 #include "fx_kernels.h"
 #include "fx_bits.h"
 #include "fx_device.h"
+#include "fx_spectra.h"
 #include <type_traits>
 
 namespace fxg {
@@ -152,15 +155,10 @@ __device__ __forceinline__ long long nonzero_in_frame(const DevStation& S, const
 // order is the reference's, with FMA contraction off, so nearestsample and
 // integerdelay are the same integers the CPU computes.
 // ---------------------------------------------------------------------------
-__global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSub* __restrict__ ss,
-                           const int* __restrict__ flags, const int2* __restrict__ ftab,
-                           int nblocks, DevBlock* __restrict__ out) {
+__device__ __forceinline__ DevBlock block_geometry(const DevStation& S, const DevStationSub& Q,
+                                                   const int* __restrict__ flags, const int2* __restrict__ ftab,
+                                                   int index) {
 #pragma clang fp contract(off)
-  const int s = blockIdx.y;
-  const int index = blockIdx.x * blockDim.x + threadIdx.x;
-  if (index >= nblocks) return;
-  const DevStation S = st[s];
-  const DevStationSub Q = ss[s];
   DevBlock g;
   g.status = 0; g.nearestsample = 0; g.integerdelay = 0; g.intwall = 0; g.allvalid = 0; g.pad = 0;
   g.weight = 0.0f; g.fse = 0.0f; g.validend = 0x7fffffffffffffffLL; g.a = 0; g.b = 0; g.fracwall = 0;
@@ -173,7 +171,7 @@ __global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSu
   // INTERLACEDVDIF band weights stay zero unless the block unpacks (mode.cpp:661-668)
   if (Q.pbw)
     for (int b = 0; b < S.nchan; b++) Q.pbw[(long long)index * S.nchan + b] = 0.0f;
-  if (!ok) { g.status = 1; out[(long long)s * nblocks + index] = g; return; }
+  if (!ok) { g.status = 1; return g; }
   const double* ip = Q.interp;
   const int fftchannels = S.L;
   double fftcentre = index + 0.5;
@@ -189,7 +187,7 @@ __global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSu
   g.nearestsample = nearestsample;
   if (nearestsample < -1 ||
       ((((long long)nearestsample + fftchannels) / 1) * S.bpbnum) / S.bpbden > Q.nbytes) {
-    g.status = 2; out[(long long)s * nblocks + index] = g; return;
+    g.status = 2; return g;
   }
   if (nearestsample == -1) nearestsample = 0;
   g.nearestsample = nearestsample;
@@ -268,7 +266,7 @@ __global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSu
     g.weight = gs / (float)S.L;
     if (blanked) g.allvalid = 0;
   }
-  if (!(g.weight > 0.0f)) { g.status = 3; out[(long long)s * nblocks + index] = g; return; }
+  if (!(g.weight > 0.0f)) { g.status = 3; return g; }
   double nearestsampletime = nearestsample * S.sampletime;
   g.fse = (float)(starttime - nearestsampletime);
   if (S.order == 0) {                        // post-F (mode.cpp:791-793)
@@ -291,7 +289,61 @@ __global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSu
     c -= integerdelay;
     g.a = a; g.b = b; g.c = c; g.integerdelay = integerdelay;
   }
+  return g;
+}
+
+// The rotation of one block by one DevRotGroup (orders 0 and 1).  Order 1: the
+// rotator e^{-2 pi i ((a n/L + b) LO - LO offset terms)} (mode.cpp:909-978) as
+// phase0 + delta n; order 0: the phase of the block at its centre delay
+// (mode.cpp:1064-1073), no rotation of the samples.  The fractional-sample
+// rotator e^{2 pi i f_c (fse - clock)} (mode.cpp:1054-1097) as theta0 + theta c.
+__device__ __forceinline__ DevRot block_rotation(const DevStation& S, const DevRotGroup& B, const DevBlock& G) {
+#pragma clang fp contract(off)
+  DevRot r;
+  r.delta = 0.0; r.phase = 0.0; r.theta = 0.0;
+  r.validend = G.validend; r.t0 = G.nearestsample; r.status = G.status; r.allvalid = G.allvalid; r.pad = 0;
+  if (G.status != 0) return r;
+  const double looffset = B.looffset;
+  double ph;
+  if (S.order == 0) {
+    ph = (G.c - G.integerdelay) * B.lofreq;
+    if (S.fractionalLo) ph += G.integerdelay * (B.lofreq - (int)B.lofreq);
+    ph -= G.wall * looffset;
+  } else {
+    r.delta = G.a * B.lofreq / S.L;
+    ph = G.b * B.lofreq;
+    if (S.fractionalLo) ph += (B.lofreq - (int)B.lofreq) * (double)G.integerdelay;
+    if (looffset > 0.0 || looffset < 0.0) {
+      double fraclooffset = fabs(looffset) - (int)fabs(looffset);
+      const bool isfrac = fraclooffset > kTiny;
+      if (looffset < 0) fraclooffset = -fraclooffset;
+      r.delta += (S.sampletime / 1e6) * (-looffset);
+      ph += -looffset * G.fracwall;
+      if (isfrac) ph += -fraclooffset * G.intwall;
+    }
+  }
+  const double sign = B.useB ? -1.0 : 1.0;
+  const float val = (float)((double)G.fse - B.clock + sign * B.clockdelta / 2);
+  r.theta = (double)val * S.bw / S.C;
+  const double theta0 = B.dsb ? -0.5 * (double)val * S.bw : B.lsb ? -(double)val * S.bw : 0.0;
+  const double q = theta0 - (ph - rint(ph));
+  r.phase = q - rint(q);
+  return r;
+}
+
+__global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSub* __restrict__ ss,
+                           const int* __restrict__ flags, const int2* __restrict__ ftab, int nblocks,
+                           DevBlock* __restrict__ out, const DevRotGroup* __restrict__ groups,
+                           DevRot* __restrict__ rots) {
+  const int s = blockIdx.y;
+  const int index = blockIdx.x * blockDim.x + threadIdx.x;
+  if (index >= nblocks) return;
+  const DevStation S = st[s];
+  const DevStationSub Q = ss[s];
+  const DevBlock g = block_geometry(S, Q, flags, ftab, index);
   out[(long long)s * nblocks + index] = g;
+  if (rots)
+    for (int k = 0; k < S.nrot; k++) rots[(long long)(S.rot0 + k) * nblocks + index] = block_rotation(S, groups[S.rot0 + k], g);
 }
 
 // ---------------------------------------------------------------------------
@@ -677,39 +729,6 @@ __device__ __forceinline__ void rotator_tables(const DevBand& B, const DevStatio
   }
 }
 
-// fp8 e4m3 pair (re low byte, im high byte) of y * 2^e, saturated at the
-// largest finite value 448
-__device__ __forceinline__ unsigned short fp8_pair(float2 y, int e) {
-  const float a = fminf(fmaxf(ldexpf(y.x, e), -448.0f), 448.0f);
-  const float b = fminf(fmaxf(ldexpf(y.y, e), -448.0f), 448.0f);
-  return (unsigned short)(__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) & 0xFFFF);
-}
-struct Fp8Out {
-  unsigned short* p;          // the band's spectrum of this block
-  const signed char* e;       // the band's channel exponents
-};
-
-// channel c's value y stored at element i of the spectrum (i = cidx(c))
-__device__ __forceinline__ void put_spec(float2* o, long long i, int c, float2 y) { o[i] = y; }
-__device__ __forceinline__ void put_spec(__half2* o, long long i, int c, float2 y) { o[i] = __floats2half2_rn(y.x, y.y); }
-__device__ __forceinline__ void put_spec(__hip_bfloat162* o, long long i, int c, float2 y) { o[i] = __float22bfloat162_rn(y); }
-__device__ __forceinline__ void put_spec(const Fp8Out& o, long long i, int c, float2 y) { o.p[i] = fp8_pair(y, o.e[c]); }
-
-// zero spectrum of one (band, block): C values of the job's spectrum type
-__device__ __forceinline__ void zero_spec(void* spectra, int prec, long long outbase, int C, long long gs, int tid,
-                                          int nt) {
-  if (prec == FXG_XMAC_FP32) {
-    float2* o = (float2*)spectra + outbase;
-    for (int c = tid; c < C; c += nt) o[cidx(c, gs)] = make_float2(0.f, 0.f);
-  } else if (prec == FXG_XMAC_FP8) {
-    unsigned short* o = (unsigned short*)spectra + outbase;
-    for (int c = tid; c < C; c += nt) o[cidx(c, gs)] = 0;
-  } else {
-    unsigned* o = (unsigned*)spectra + outbase;
-    for (int c = tid; c < C; c += nt) o[cidx(c, gs)] = 0u;
-  }
-}
-
 // The block-independent LDS tables of a single-workgroup F stage (split
 // twiddles, the second pass's 256 twiddles, the 8-bit level table), loaded
 // into registers at the start of the kernel: their loads then overlap the
@@ -780,6 +799,8 @@ __device__ __forceinline__ void last_pass_r2(const float2* buf, const float2* tw
   }
 }
 
+// The F stage of real samples with quadratic fringe rotation (order 2), whose
+// rotator has no shifted-grid form (linear and post-F rotation: fx_fstage.hip)
 template <int L, int NBITS>
 __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage(FStageArgs A) {
   using Sh = FftShape<L>;
@@ -882,41 +903,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage(FStageArgs A) {
   float2 v[16];
   if (tid < NTF) {
     const int j = tid;
-    bool transformed = false;                  // the branch ran the 16-point DFT itself
-    if (kWordStep && fast && rotfast && S.order == 1) {
-      const int bp = bitoff + NBITS * j;
-      const unsigned* wp = raw + (bp >> 5);
-      const int sh = bp & 31;
-      const float2 r0 = rsub[j & (s - 1)];
-      const float2* stp = rstep + (j >> slog);
-      const int sstep = NTF >> slog;
-      // x[r] rot[r] and x[r + 8] rot[r + 8] go straight into the first
-      // butterflies: sum and difference as two FMAs on the first product
-      float2 sm[8], df[8];
-#pragma unroll
-      for (int r = 0; r < 8; r++) {
-        const unsigned c0 = (wp[r * WSTEP] >> sh) & ((1u << NBITS) - 1u);
-        const unsigned c8 = (wp[(r + 8) * WSTEP] >> sh) & ((1u << NBITS) - 1u);
-        const float x0 = lut8s[c0], x8 = lut8s[c8];
-        const float2 q0 = cmulf(r0, stp[r * sstep]);         // sub[k] * step[j], mode.cpp:975-977
-        const float2 q8 = cmulf(r0, stp[(r + 8) * sstep]);
-        const float2 p = make_float2(x0 * q0.x, x0 * q0.y);
-        sm[r] = make_float2(__builtin_fmaf(x8, q8.x, p.x), __builtin_fmaf(x8, q8.y, p.y));
-        df[r] = make_float2(__builtin_fmaf(-x8, q8.x, p.x), __builtin_fmaf(-x8, q8.y, p.y));
-      }
-      dft16_from_halves(sm, df, v);
-      transformed = true;
-    } else if (kWordStep && fast && S.order == 0) {
-      // post-F fringe rotation: the samples are transformed unrotated
-      const int bp = bitoff + NBITS * j;
-      const unsigned* wp = raw + (bp >> 5);
-      const int sh = bp & 31;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const unsigned code = (wp[r * WSTEP] >> sh) & ((1u << NBITS) - 1u);
-        v[r] = make_float2(lut8s[code], 0.0f);
-      }
-    } else if (kWordStep && fast && rotfast && S.order == 2) {
+    if (kWordStep && fast && rotfast) {
       // piecewise quadratic rotator: rot[j s + k] = piece_j[k] step[j] with
       // piece_0 = sub[k], piece_{j+1} = piece_j quad[k] (mode.cpp:1043-1049);
       // this thread's points all have the same k and step index q0 + r sstep
@@ -950,24 +937,16 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage(FStageArgs A) {
         } else {
           x = sample_value(S, Q, A.ftab, NBITS == 8 ? lut8s : A.lut8, lut2, t0 + n, G.validend, B.band);
         }
-        float2 rot;
-        if (S.order == 0) {
-          rot = make_float2(1.0f, 0.0f);
-        } else if (S.order == 1) {
-          if (slog >= 0) rot = n < s ? rsub[n] : cmulf(rsub[n & (s - 1)], rstep[n >> slog]);
-          else rot = n < s ? rsub[n] : cmulf(rsub[n % s], rstep[n / s]);
-        } else {
-          const int kk = slog >= 0 ? (n & (s - 1)) : n % s;
-          const int jj = slog >= 0 ? (n >> slog) : n / s;
-          const float2 qd = rquad[kk];
-          float2 piece = rsub[kk];
-          for (int i = 0; i < jj; i++) piece = cmulf(piece, qd);
-          rot = cmulf(piece, rstep[jj]);
-        }
-        v[r] = S.order == 0 ? make_float2(x, 0.0f) : make_float2(x * rot.x, x * rot.y);
+        const int kk = slog >= 0 ? (n & (s - 1)) : n % s;
+        const int jj = slog >= 0 ? (n >> slog) : n / s;
+        const float2 qd = rquad[kk];
+        float2 piece = rsub[kk];
+        for (int i = 0; i < jj; i++) piece = cmulf(piece, qd);
+        const float2 rot = cmulf(piece, rstep[jj]);
+        v[r] = make_float2(x * rot.x, x * rot.y);
       }
     }
-    if (!transformed) DFT<16>::run(v);
+    DFT<16>::run(v);
   }
   if (kAliasRaw) __syncthreads();            // every stream word read before buf is written
   if (tid < NTF) {
@@ -1660,9 +1639,10 @@ hipError_t launch_frames(const DevStation* st, const DevStationSub* ss, int2* ft
 }
 
 hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const int* flags,
-                           const int2* ftab, int nblocks, DevBlock* out, int nst, hipStream_t stream) {
+                           const int2* ftab, int nblocks, DevBlock* out, int nst, const DevRotGroup* groups,
+                           DevRot* rots, hipStream_t stream) {
   dim3 grid((unsigned)((nblocks + 127) / 128), nst);
-  hipLaunchKernelGGL(k_prologue, grid, dim3(128), 0, stream, st, ss, flags, ftab, nblocks, out);
+  hipLaunchKernelGGL(k_prologue, grid, dim3(128), 0, stream, st, ss, flags, ftab, nblocks, out, groups, rots);
   return hipGetLastError();
 }
 
