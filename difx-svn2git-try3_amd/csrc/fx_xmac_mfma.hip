@@ -303,26 +303,190 @@ __global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_dl(XmacArgs A,
 }
 
 // ---------------------------------------------------------------------------
-// FP32 on the matrix cores: v_mfma_f32_32x32x2_f32 takes one block per
-// instruction (K = 2: lanes 0-31 give the real part of their row's input,
-// lanes 32-63 the imaginary part), so with the same tiles as above
+// FP32 on the matrix cores, up to 64 inputs (and the diagonal chunks of more):
+// v_mfma_f32_16x16x4_f32, K = four blocks, T x T tiles of 16 inputs, I <= J.
+// A lane holds one input's complex value of one block (one 8-byte LDS read
+// per 16 inputs and four blocks), so with A = its real or imaginary part
+//     Re V = Ar Br^T + Ai Bi^T,   Im V = Ai Br^T - Ar Bi^T,
+// four instructions a tile; on a diagonal tile Ar Bi^T is the transpose of
+// Ai Br^T, formed once at the end, so three.  32x32 tiles cost 2 x 64 cycles
+// a block and channel for up to 32 inputs and 6 x 64 for up to 64; these
+// 24 (16 inputs), 80 (32), 168 (48), 288 (64).
+// Rows past the last input are neither loaded nor read back (a row of A or B
+// only reaches its own row or column of the tile); blocks past the last read
+// a 16-byte zero buffer.  LDS is a ring of stages of 8 blocks x 16 channels x
+// 16 T rows, filled by global_load_lds, as deep as leaves two workgroups on a
+// CU for one and two tiles: there the load stream is the bound, above it the
+// matrix cores.
+// 4 stations, 256 channels, 62500 blocks 1109 -> 320 us; 10 stations, 1024
+// channels, 4096 blocks 327 -> 249 us a frequency; 32 stations, 4096
+// channels, 500 blocks 494 -> 485 us.
+// ---------------------------------------------------------------------------
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// waits until at most N of this wavefront's vector-memory operations are in
+// flight, and for its LDS reads (expcnt left at its maximum)
+template <int N> __device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (((N >> 4) & 3) << 14) | (7 << 4));
+}
+
+template <int T>
+__global__ __launch_bounds__(1024, T <= 2 ? 8 : 4) void k_xmac_f32_t16(XmacArgs A, const uint4* __restrict__ zero16) {
+  constexpr int CG = 16;                 // channels (wavefronts) per workgroup
+  constexpr int TT = 8;                  // blocks per stage
+  constexpr int NBUF = T == 1 ? 4 : T == 3 ? 3 : 2;
+  constexpr int NTILE = T * (T + 1) / 2;
+  constexpr int RBW = 2 * CG;            // dwords per (row, block)
+  constexpr int SDW = TT * RBW + 4;      // dwords per row per stage
+  constexpr int STAGE = 16 * T * SDW;
+  __shared__ __align__(16) unsigned lds[NBUF * STAGE];
+  static_assert(NBUF * STAGE >= CG * 16 * 17, "the ring holds the wavefronts' transposes");
+
+  const char* spec = (const char*)A.spec;
+  const int tid = threadIdx.x;
+  const int w = tid >> 6, l = tid & 63;
+  const int nwg = gridDim.x;
+  const int bid = blockIdx.x;
+  const int grp = (nwg % 8 == 0) ? (bid % 8) * (nwg / 8) + bid / 8 : bid;   // XCD-aware groups
+  const int c0 = grp * CG;
+  const int row = l & 15, kk = l >> 4;
+  const int lt = l >> 3, lp = l & 7;                // load lane: block and 2-channel piece
+  const int sb0 = blockIdx.y * A.split_blocks;
+  const int nb = min(A.nblocks - sb0, A.split_blocks);
+  float2* const Vout = A.V + (long long)blockIdx.y * A.vsplit;
+  const int in0 = 64 * blockIdx.z;                  // this chunk's first input
+  // the rows this wavefront loads: w, w + 16, ... (the valid ones come first)
+  const int wu = __builtin_amdgcn_readfirstlane(w);
+  long long ioff[T];
+  int nv = 0;
+#pragma unroll
+  for (int u = 0; u < T; u++) {
+    const int a = in0 + 16 * u + wu;
+    ioff[u] = a < A.nin ? A.in_off[a] + c0 : 0;
+    if (a < A.nin) nv = u + 1;
+  }
+  auto issue = [&](int stage, int buf) {
+    const int t = stage * TT + lt;
+#pragma unroll
+    for (int u = 0; u < T; u++) {
+      if (u >= nv) break;
+      const void* src = zero16;
+      if (t < nb) src = spec + 8 * (ioff[u] + (long long)(sb0 + t) * A.block_stride + 2 * lp);
+      __builtin_amdgcn_global_load_lds(
+          src, (__attribute__((address_space(3))) void*)(lds + buf * STAGE + (16 * u + wu) * SDW), 16, 0, 0);
+    }
+  };
+  // all but the newest NBUF - 2 stages of this wavefront's loads have landed
+  auto landed = [&] {
+    if (nv == 1) wait_vm<(NBUF - 2) * 1>();
+    else if (nv == 2) wait_vm<(NBUF - 2) * 2>();
+    else if (nv == 3) wait_vm<(NBUF - 2) * 3>();
+    else if (nv == 4) wait_vm<(NBUF - 2) * 4>();
+    else wait_vm<0>();
+  };
+  auto barrier = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  f32x4_t accR[NTILE], accI[NTILE];
+#pragma unroll
+  for (int k = 0; k < NTILE; k++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) { accR[k][e] = 0.0f; accI[k][e] = 0.0f; }
+
+  const int nstage = (nb + TT - 1) / TT;
+#pragma unroll
+  for (int st = 0; st < NBUF - 1; st++) issue(st, st);
+  landed();
+  barrier();
+  int buf = 0;
+  for (int sg = 0; sg < nstage; sg++) {
+    issue(sg + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
+    const float* base = (const float*)(lds + buf * STAGE) + row * SDW + kk * RBW + 2 * w;
+#pragma unroll
+    for (int ks = 0; ks < TT / 4; ks++) {
+      float2 f[T];
+      float n[T];
+#pragma unroll
+      for (int I = 0; I < T; I++) {
+        f[I] = *(const float2*)(base + 16 * I * SDW + 4 * ks * RBW);
+        n[I] = -f[I].x;
+      }
+      int k = 0;
+#pragma unroll
+      for (int I = 0; I < T; I++)
+#pragma unroll
+        for (int J = I; J < T; J++, k++) {
+          accR[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[I].x, f[J].x, accR[k], 0, 0, 0);
+          accI[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[I].y, f[J].x, accI[k], 0, 0, 0);
+          accR[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[I].y, f[J].y, accR[k], 0, 0, 0);
+          if (J > I) accI[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(n[I], f[J].y, accI[k], 0, 0, 0);
+        }
+    }
+    landed();                            // this wavefront's loads of the next stage
+    barrier();                           // everyone's, and nobody still reads this stage
+    buf = buf + 1 == NBUF ? 0 : buf + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(0);         // the stages past the end have landed
+  barrier();                             // before the ring is reused for the transposes
+
+  const int c = c0 + w;
+  float* const tr = (float*)lds + w * 16 * 17;
+  int k = 0;
+#pragma unroll
+  for (int I = 0; I < T; I++)
+#pragma unroll
+    for (int J = I; J < T; J++, k++) {
+      f32x4_t im = accI[k];
+      if (I == J) {
+        // Im V[a][b] = Q[a][b] - Q[b][a], within this wavefront
+#pragma unroll
+        for (int r = 0; r < 4; r++) tr[(4 * kk + r) * 17 + row] = im[r];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int r = 0; r < 4; r++) im[r] -= tr[row * 17 + 4 * kk + r];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+      const int b = in0 + 16 * J + row;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int a = in0 + 16 * I + 4 * kk + r;
+        if (a >= A.nin || b >= A.nin || c >= A.nchan) continue;
+        float2* ptr = Vout + ((long long)a * A.nin + b) * A.nchan + c;
+        float2 v = make_float2(accR[k][r], im[r]);
+        if (A.accumulate) { float2 o = *ptr; v.x += o.x; v.y += o.y; }
+        *ptr = v;
+      }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// FP32, the products between two chunks of 64 inputs: v_mfma_f32_32x32x2_f32
+// takes one block per instruction (K = 2: lanes 0-31 give the real part of
+// their row's input, lanes 32-63 the imaginary part), so with the same tiles
+// as the streamed kernel above
 //     Re V += A A^T, Im V += Ah A^T,  Ah = (im, -re)
 // in FP32 products and FP32 accumulation.  The spectra are row-major
-// [band][block][channel] float2; a stage holds 8 blocks of CG channels of
-// every row in LDS ([row][block][CG float2], rows padded by 4 dwords),
-// filled by global_load_lds (one 16-byte piece, two channels, per lane) and
+// [band][block][channel] float2; a stage holds 8 blocks of 8 channels of
+// every row in LDS ([row][block][8 float2], rows padded by 4 dwords), filled
+// by global_load_lds (one 16-byte piece, two channels, per lane) and
 // double-buffered: the matrix cores need ~5 us per stage, the loads of the
 // next one far less.  Rows and chunk pairs as in k_xmac_mfma_dl.
 // ---------------------------------------------------------------------------
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-template <int T, bool CROSS>
-__global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_f32(XmacArgs A, const uint4* __restrict__ zero16) {
-  static_assert(!CROSS || T == 4, "a cross workgroup holds two 64-input chunks");
-  constexpr int CG = CROSS ? 8 : 16;     // channels (wavefronts) per workgroup
+__global__ __launch_bounds__(512) void k_xmac_f32_cross(XmacArgs A, const uint4* __restrict__ zero16) {
+  constexpr int T = 4;                   // tiles of 32 rows: two chunks of 64 inputs
+  constexpr int CG = 8;                  // channels (wavefronts) per workgroup
   constexpr int TT = 8;                  // blocks per stage
   constexpr int NR = 32 * T;
-  using TL = DlTiles<T, CROSS>;
+  using TL = DlTiles<T, true>;
   constexpr int NTILE = TL::N;
   constexpr int RBW = 2 * CG;            // dwords per (row, block)
   constexpr int SDW = TT * RBW + 4;      // dwords per row per stage
@@ -343,14 +507,10 @@ __global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_f32(XmacArgs A
   const int sb0 = blockIdx.y * A.split_blocks;
   const int nb = min(A.nblocks - sb0, A.split_blocks);
   float2* const Vout = A.V + (long long)blockIdx.y * A.vsplit;
-  int p = blockIdx.z, q = blockIdx.z;
-  if (CROSS) {
-    const int nch = (A.nin + 63) >> 6;
-    int rem = blockIdx.z;
-    p = 0;
-    while (rem >= nch - 1 - p) { rem -= nch - 1 - p; p++; }
-    q = p + 1 + rem;
-  }
+  int p = 0, rem = blockIdx.z;
+  const int nch = (A.nin + 63) >> 6;
+  while (rem >= nch - 1 - p) { rem -= nch - 1 - p; p++; }
+  const int q = p + 1 + rem;
   auto input_of = [&](int r) { return r < 64 ? 64 * p + r : 64 * q + r - 64; };
   const int wu = __builtin_amdgcn_readfirstlane(w);
   long long ioff[LPW];
@@ -624,16 +784,15 @@ bool xmac_mfma_f32_ok(const XmacArgs& a, const long long* in_off_host) {
 hipError_t launch_xmac_mfma_f32(const XmacArgs& a, const void* zero16, hipStream_t stream) {
   const unsigned gx = (unsigned)(a.nchan / 16), gy = (unsigned)((a.nblocks + a.split_blocks - 1) / a.split_blocks);
   const uint4* z = (const uint4*)zero16;
-  if (a.nin <= 32) {
-    hipLaunchKernelGGL((k_xmac_mfma_f32<1, false>), dim3(gx, gy), dim3(1024), 0, stream, a, z);
-  } else if (a.nin <= 64) {
-    hipLaunchKernelGGL((k_xmac_mfma_f32<2, false>), dim3(gx, gy), dim3(1024), 0, stream, a, z);
-  } else {
-    const unsigned nch = (unsigned)((a.nin + 63) / 64);
-    hipLaunchKernelGGL((k_xmac_mfma_f32<2, false>), dim3(gx, gy, nch), dim3(1024), 0, stream, a, z);
-    hipLaunchKernelGGL((k_xmac_mfma_f32<4, true>), dim3(2 * gx, gy, nch * (nch - 1) / 2), dim3(512), 0, stream, a,
-                       z);
-  }
+  const unsigned nch = (unsigned)((a.nin + 63) / 64);
+  const dim3 grid(gx, gy, nch), block(1024);
+  if (a.nin <= 16) hipLaunchKernelGGL(k_xmac_f32_t16<1>, grid, block, 0, stream, a, z);
+  else if (a.nin <= 32) hipLaunchKernelGGL(k_xmac_f32_t16<2>, grid, block, 0, stream, a, z);
+  else if (a.nin <= 48) hipLaunchKernelGGL(k_xmac_f32_t16<3>, grid, block, 0, stream, a, z);
+  else hipLaunchKernelGGL(k_xmac_f32_t16<4>, grid, block, 0, stream, a, z);
+  // more than 64 inputs: every pair of chunks (8 channels per workgroup)
+  if (nch > 1)
+    hipLaunchKernelGGL(k_xmac_f32_cross, dim3(2 * gx, gy, nch * (nch - 1) / 2), dim3(512), 0, stream, a, z);
   return hipGetLastError();
 }
 

@@ -1,0 +1,37 @@
+"""The FP32 cross-multiply in 16-input tiles on the matrix cores, against the
+FP64 oracle: input counts either side of the tile and chunk edges (16, 32, 48
+and 64 inputs), block counts around its stages of 8 blocks.
+
+Tolerance: twice the spectra's bound ((3 log2 L + 8) half ulps) for the two
+factors of a product, and half an ulp for each of the blocks added up."""
+import numpy as np
+import pytest
+
+from fxcorr import JobSpec
+from fxsynth import make_subint
+from fxtestlib import GpuJob, oracle_results, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nstations,npol,blocks", [(1, 2, 3), (2, 1, 8), (8, 2, 7), (17, 1, 9), (16, 2, 16), (33, 1, 5),
+                                                   (24, 2, 17), (49, 1, 8), (32, 2, 1), (33, 2, 9)])
+def test_tiles(gpu, oracle, nstations, npol, blocks):
+    lib, ctx = gpu
+    spec = JobSpec(nstations=nstations, nsubbands=1, npol=npol, bw_mhz=16.0, nchan=64, blockspersend=blocks,
+                   crosspol=npol == 2)
+    job, keep = spec.build()
+    rng = np.random.default_rng(nstations)
+    sd = make_subint(spec, seed=nstations + blocks, rho=0.3, delays_us=rng.uniform(-5, 5, nstations),
+                     rates_us_per_s=rng.uniform(-1, 1, nstations))
+    g = GpuJob(lib, ctx, job)
+    got = g.process(sd)
+    ref = oracle_results(oracle, job, sd, fp64=True, nthreads=8)
+    tol = 2 * (3 * np.log2(spec.fftchannels) + 8) * 2.0 ** -25 + blocks * 2.0 ** -25
+    assert rel_err(got, ref) < tol, (rel_err(got, ref), tol)
+    # every product by itself: none hides behind the autocorrelations
+    nprod = nstations * (nstations - 1) // 2 * npol * npol
+    for k in range(nprod):
+        a, b = got[k * 64:(k + 1) * 64], ref[k * 64:(k + 1) * 64]
+        assert np.linalg.norm(a - b) < tol * np.sqrt(64.0) * blocks * spec.fftchannels * 4.4 * 2, k
+    g.close()
