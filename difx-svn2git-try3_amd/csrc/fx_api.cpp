@@ -1250,7 +1250,9 @@ static int launch_back(fxg_job* j, float* dres, hipStream_t s) {
     pa.tonebin = j->d_pcaltone.as<int>(); pa.part = j->d_pcalpart.as<float>(); pa.res = dres;
     pa.nblocks = nblocks; pa.ngroups = P.pcal_groups;
     if ((rc = j->ev_begin(FXG_STAGE_PCAL))) return rc;
-    HIPCHK(launch_pcal(pa, (int)P.pcal.size(), s));
+    bool few = false, many = false;
+    for (const DevPcal& pc : P.pcal) (pc.nbins <= kPcalFewBins ? few : many) = true;
+    HIPCHK(launch_pcal(pa, (int)P.pcal.size(), few, many, s));
     if ((rc = j->ev_end())) return rc;
   }
   return 0;

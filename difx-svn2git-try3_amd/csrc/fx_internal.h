@@ -191,6 +191,8 @@ inline int spectrum_bytes(int prec) { return prec == FXG_XMAC_FP32 ? 8 : prec ==
 
 // the largest accumulation of one band's phase-cal bins (LDS floats)
 constexpr int kPcalMaxFloats = 32768;
+// bands of at most this many bins keep them in registers, a thread each
+constexpr int kPcalFewBins = 256;
 
 int build_plan(const fxg_job_desc* d, Plan* p, std::string* err);
 // the library's error string (fxg_last_error) and code

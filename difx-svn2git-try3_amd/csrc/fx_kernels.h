@@ -166,7 +166,8 @@ hipError_t launch_xmac_reduce(const float2* P, int nsplit, long long vsplit, flo
                               hipStream_t stream);
 hipError_t launch_weights(const DevStation* st, const DevStationSub* ss, const DevBlock* blocks, int nblocks,
                           const DevWTerm* terms, int nterms, float* w, hipStream_t stream);
-hipError_t launch_pcal(const PcalArgs& a, int npcal, hipStream_t stream);
+// few / many: some band has at most kPcalFewBins bins / more
+hipError_t launch_pcal(const PcalArgs& a, int npcal, bool few, bool many, hipStream_t stream);
 // p[0, n) = 0 with a kernel (graph-safe clearing)
 hipError_t launch_zero(float* p, long long n, hipStream_t stream);
 hipError_t launch_scatter(const DevSeg* segs, int nseg, int maxlen, const float2* V, const float* w,
