@@ -115,7 +115,7 @@ struct fxg_job {
   DBuf d_ss, d_flags, d_ftab, d_blocks, d_weights, d_results, d_ct;
   DBuf d_rotgroups, d_rots;       // rotations of the bands, and of each block (k_prologue)
   DBuf d_cdesc, d_base, d_quad;   // tables of the F stage with linear rotation (fx_fstage.hip)
-  bool fstage_lin = false;        // that F stage runs: real samples, orders 0 and 1, up to kFStageMaxL points
+  bool fstage_lin = false;        // that F stage runs: real samples, fringe orders 0 and 1
   DBuf d_bandlist;                // global bands grouped by sample size
   int nb2 = 0, nb8 = 0;           // bands of 2-bit and 8-bit datastreams
   std::vector<DBuf> d_raw;        // staged host data per datastream
@@ -616,6 +616,7 @@ int fxg_job_create(fxg_ctx* c, const fxg_job_desc* desc, fxg_job** out) {
   if (hipStreamCreateWithFlags(&j->copy_stream, hipStreamNonBlocking) != hipSuccess)
     return fail(set_err(FXG_EHIP, "copy stream"));
 
+  j->fstage_lin = !P.st[0].cplx && P.st[0].order != 2;
   const int prec = desc->xmac_precision;
   // spectrum scale for reduced precision: 2^-round(log2(sqrt(L)))
   // (fp8: per-channel exponents instead, below)
@@ -629,9 +630,10 @@ int fxg_job_create(fxg_ctx* c, const fxg_job_desc* desc, fxg_job** out) {
   const long long chunk = P.chunk_blocks;
   for (size_t g = 0; g < P.bands.size(); g++) P.bands[g].specoff = (long long)g * chunk * P.C;
   {
-    // (FFTs above 16384 points write their channels from a separate pass
-    // whose scattered 64-byte pieces cost more than the grouped reads save)
-    bool grouped = prec != FXG_XMAC_FP32 && P.C % 16 == 0 && P.L <= kFStageMaxL;
+    // (with quadratic rotation, FFTs above 16384 points write their channels
+    // from a separate pass whose scattered 64-byte pieces cost more than the
+    // grouped reads save)
+    bool grouped = prec != FXG_XMAC_FP32 && P.C % 16 == 0 && (j->fstage_lin || P.L <= kFStageMaxL);
     for (const XmacFreq& x : P.xf) {
       if (!xmac_mfma_streaming_supported((int)x.in_station.size(), x.nchan)) grouped = false;
       for (long long o : x.in_off) if (o % 16) grouped = false;     // zoom channel offsets
@@ -729,7 +731,6 @@ int fxg_job_create(fxg_ctx* c, const fxg_job_desc* desc, fxg_job** out) {
         hipMemcpy(j->d_eoff.p, eoff.data(), sizeof(int) * eoff.size(), hipMemcpyHostToDevice) != hipSuccess)
       return fail(set_err(FXG_EHIP, "scale table upload failed"));
   }
-  j->fstage_lin = !P.st[0].cplx && P.st[0].order != 2 && P.L <= kFStageMaxL;
   if (j->fstage_lin) {
     std::vector<float4> cdesc, quad(512);
     std::vector<float2> base;

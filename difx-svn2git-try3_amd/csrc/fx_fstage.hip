@@ -1,6 +1,5 @@
 // fx_fstage.hip — the F stage of real-sampled data with linear (or post-F)
-// fringe rotation, transforms up to 16384 points (mode.cpp:909-1310): level
-// decoding, fringe rotation, FFT, sideband select, fractional-sample rotation.
+// fringe rotation (mode.cpp:909-1310): level decoding, fringe rotation, FFT, sideband select, fractional-sample rotation.
 #include <hip/hip_runtime.h>
 #include "fx_kernels.h"
 #include "fx_device.h"
@@ -11,21 +10,26 @@
 
 namespace fxg {
 
-// The passes of one length: R1 = 16 P in the first, 16 in a middle one from
-// 2048 points on, RL = 16 or 8 in the last; NTF threads and NB blocks per
-// workgroup of NT threads; the per-block table (pass 1: CP entries for each
-// of the P thread sets; the last pass's four powers and the eight channel
-// steps; eight twiddles for each bin of the middle pass).
+// The passes of one length L = PW x M: PW workgroups share a block above 8192
+// points, each transforming M points to the bins k = PW k' + pw.  M = R1 x
+// (16) x RL: R1 = 16 P in the first pass, 16 in a middle one from 2048 points
+// on, RL = 16 or 8 in the last; NTF threads a block and NB blocks per
+// workgroup of NT threads; the per-block table (pass 1: CP entries for each of
+// the P thread sets; the last pass's four powers and the eight channel steps;
+// eight twiddles for each bin of the middle pass).
 template <int L> struct FsShape {
-  static constexpr int LOG = L == 128 ? 7 : L == 256 ? 8 : L == 512 ? 9 : L == 1024 ? 10 : L == 2048 ? 11
-                           : L == 4096 ? 12 : L == 8192 ? 13 : 14;
+  static constexpr int M = L > 8192 ? 8192 : L, PW = L / M;
+  static constexpr int LOG = M == 128 ? 7 : M == 256 ? 8 : M == 512 ? 9 : M == 1024 ? 10 : M == 2048 ? 11
+                           : M == 4096 ? 12 : 13;
   static constexpr int P = LOG % 4 == 1 ? 2 : LOG % 4 == 2 ? 4 : 1;
-  static constexpr int R1 = 16 * P, J1 = L / R1, RL = LOG % 4 == 3 ? 8 : 16;
+  static constexpr int R1 = 16 * P, J1 = M / R1, RL = LOG % 4 == 3 ? 8 : 16;
   static constexpr bool MID = LOG >= 11;
   static constexpr int J2 = MID ? J1 / 16 : 16;
-  static constexpr int NTF = L / 16, NB = NTF >= 128 ? 1 : 256 / NTF, NT = NTF * NB;
-  static constexpr int CP = P == 1 ? 8 : P == 2 ? 10 : 12, LAST = P * CP, MIDOFF = LAST + 12;
+  static constexpr int NTF = M / 16, NB = NTF >= 128 ? 1 : 256 / NTF, NT = NTF * NB;
+  static constexpr int CP = PW > 1 || P == 4 ? 12 : P == 2 ? 10 : 8, LAST = P * CP, MIDOFF = LAST + 12;
   static constexpr int NE = MIDOFF + (MID ? 8 * R1 : 0);
+  // PW > 1: quads of one first-pass input, and tables of quad sums
+  static constexpr int QSUM = P * PW / 4, NSUM = PW == 1 ? 0 : PW == 2 ? 2 : 1;
 };
 
 // Validity of the 32 / BITS consecutive samples from t of one band, one bit
@@ -84,8 +88,14 @@ __device__ __forceinline__ void quads8(unsigned* a) {
   a[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
 }
 
+// x0 + g1 x1 + g2 x2 + g3 x3
+__device__ __forceinline__ float2 quad_sum(const float4& x, float2 g1, float2 g2, float2 g3) {
+  return make_float2(__builtin_fmaf(g3.x, x.w, __builtin_fmaf(g2.x, x.z, __builtin_fmaf(g1.x, x.y, x.x))),
+                     __builtin_fmaf(g3.y, x.w, __builtin_fmaf(g2.y, x.z, g1.y * x.y)));
+}
+
 // ---------------------------------------------------------------------------
-// k_fstage_lin<L, NBITS>: L = R1 x (16) x RL points, 16 per thread.
+// k_fstage_lin<L, NBITS>: 16 points per thread in every pass.
 //
 // What bounds it: FP32 VALU issue (wave64, four cycles an instruction), so it
 // is built for few instructions:
@@ -99,31 +109,46 @@ __device__ __forceinline__ void quads8(unsigned* a) {
 //     the outputs q = P q' + p), so that no length but 8 x 16^n needs a pass
 //     of smaller radix: two LDS exchanges at 2048 points and more, one below;
 //   - the last pass forms only the sideband's half of the outputs (the lower
-//     sideband's sign rides on w).
+//     sideband's sign rides on w);
+//   - above 8192 points PW workgroups share a block, so that two still fit a
+//     CU and one's LDS phases run under the other's arithmetic.  A thread's
+//     first-pass inputs are then sums of QSUM quads with fixed weights, x0 +
+//     g x1 + g^2 x2 + g^3 x3 by the quad's byte from a table that the
+//     workgroup forms once (g is the same for all its threads, or for every
+//     other set).  Every workgroup decodes the whole block, and nothing goes
+//     through memory between the passes.  The PW workgroups of a block run
+//     side by side on one XCD, whose L2 merges their interleaved channels
+//     into lines.  One workgroup of 1024 threads and 16384 points a CU instead
+//     left the VALU idle half of the time (16384 points 18.4 ms, 65536 points
+//     28.0 ms on the workloads below).
 // Exchanges are laid out so that both sides hit all banks with immediate
 // offsets: the one into the middle pass by exchanging pieces of J2 values
 // between neighbouring rows, the one into the last pass by a row pad.
-// Against the kernel with rotator tables, padded twiddle products and one
-// radix-2 pass more (rocprofv3, ms): 32 stations, 8192 points, 16.8 Gsamples
-// 33.4 -> 26.2; 16384 points, 8.2 Gsamples 24.0 -> 18.4; 2048 points, 1.34
-// Gsamples 3.23 -> 2.80; 512 points, 8-bit, 0.92 Gsamples 3.53 -> 1.37.
+// Against the kernels with rotator tables and padded twiddle products, one
+// radix-2 pass more, and from 32768 points a scratch in HBM between two kernels
+// (rocprofv3, ms): 8192 points, 16.8 Gsamples 33.4 -> 25.9; 16384 points, 8.2
+// Gsamples 24.0 -> 14.5; 65536 points, 7.9 Gsamples 37.5 -> 23.2; 2048 points,
+// 1.34 Gsamples 3.23 -> 2.80; 512 points, 8-bit, 0.92 Gsamples 3.53 -> 1.37.
 // ---------------------------------------------------------------------------
 template <int L, int NBITS>
 __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) {
   using Sh = FsShape<L>;
+  constexpr int M = Sh::M, PW = Sh::PW;
   constexpr int P = Sh::P, R1 = Sh::R1, J1 = Sh::J1, J2 = Sh::J2, RL = Sh::RL, NTF = Sh::NTF, NB = Sh::NB, NT = Sh::NT;
   constexpr bool MID = Sh::MID;
   constexpr int QW = NBITS == 8 ? L / 4 : L / 16;         // staged quad words of one block
-  constexpr int NL = L / RL, LPAD = 32 / RL;               // bins entering the last pass, and its row pad
-  // a block within one wavefront: its quads lie in the exchange buffer, read
-  // before that wavefront's first exchange write
-  constexpr bool RAWOWN = NTF > 64 || NTF < 32;
+  constexpr int NL = M / RL, LPAD = 32 / RL;               // bins entering the last pass, and its row pad
+  // The quads lie in the exchange buffer where a block is within one
+  // wavefront (read before that wavefront's first exchange write) and where
+  // PW workgroups share a block (a barrier between).
+  constexpr bool RAWOWN = PW == 1 && (NTF > 64 || NTF < 32);
   struct Smem {
     float2 tab[NB][Sh::NE];
-    float4 quad[NBITS == 2 ? 256 : 0];
+    float4 quad[NBITS == 2 && PW == 1 ? 256 : 0];
+    float2 sums[NBITS == 2 ? 256 * Sh::NSUM : 0];
     unsigned raw_own[RAWOWN ? NB * QW : 0];
     unsigned ok_own[RAWOWN && NBITS == 2 ? NB * QW : 0];
-    float2 buf[NB][L + 32 + (NTF < 32 ? 1 : 0)];
+    float2 buf[NB][M + 32 + (NTF < 32 ? 1 : 0)];
   };
   __shared__ __align__(16) Smem sm;
 
@@ -134,7 +159,8 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
   // block groups within the chunk: workgroups are dealt to the 8 XCDs
   // round-robin, so consecutive blocks go to one XCD (its L2 merges the
   // halves of the lines that neighbouring blocks write in the grouped layout)
-  const int grp = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  const int grp = (blockIdx.x % 8) * (gridDim.x / (8 * PW)) + blockIdx.x / (8 * PW);
+  const int pw = PW == 1 ? 0 : (blockIdx.x / 8) % PW;
   if (grp * NB >= A.nchunk) return;
   const int cbx = grp * NB + fi;
   const bool mine = NB == 1 || cbx < A.nchunk;
@@ -147,46 +173,34 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
   const long long outbase = B.specoff + (long long)cb * A.bstride;
   const bool dead = R.status != 0;
   if (NB == 1 && dead) {
-    zero_spec(A.spectra, A.prec, outbase, C, A.gstride, tid, NT);
+    if (pw == 0) zero_spec(A.spectra, A.prec, outbase, C, A.gstride, tid, NT);
     return;
   }
 
-  // ---- the block's samples of this band: four rows a quarter block apart
+  // ---- the block's samples of this band: four rows a quarter block apart,
+  // their first loads in flight under the tables' sines
   constexpr int GROUPS = NBITS == 8 ? L / 16 : L / 64;
-  unsigned a[4];
-  if (t < GROUPS) {
-    const long long bit0 = (long long)(dead ? 0 : R.t0) * NBITS;
-    const unsigned* src = (const unsigned*)(A.ct + Q.ctbase + (long long)B.band * Q.ctstride);
-    const long long nwords = Q.ctstride >> 2;
-    const long long w0 = (bit0 >> 5) + t;
-    const int sh = (int)(bit0 & 31);
-    unsigned lo[4], hi[4];
+  const bool fast = R.allvalid != 0 || dead;
+  const long long bit0 = (long long)(dead ? 0 : R.t0) * NBITS;
+  const unsigned* src = (const unsigned*)(A.ct + Q.ctbase + (long long)B.band * Q.ctstride);
+  const long long nwords = Q.ctstride >> 2;
+  constexpr int NIT = (GROUPS + NTF - 1) / NTF, AHEAD = NIT > 2 ? 2 : NIT;
+  unsigned lo[AHEAD][4], hi[AHEAD][4];
+  auto load_rows = [&](int g, unsigned (&lo)[4], unsigned (&hi)[4]) {
+    const long long w0 = (bit0 >> 5) + g;
 #pragma unroll
     for (int m = 0; m < 4; m++) {
       const long long w = w0 + m * GROUPS;
       lo[m] = w < nwords ? src[w] : 0u;
       hi[m] = w + 1 < nwords ? src[w + 1] : 0u;
     }
+  };
+  auto store_quads = [&](int g, const unsigned (&lo)[4], const unsigned (&hi)[4]) {
+    unsigned a[4];
 #pragma unroll
-    for (int m = 0; m < 4; m++) a[m] = __builtin_amdgcn_alignbit(hi[m], lo[m], sh);
-  }
-  // ---- this block's twiddles and fractional-sample steps
-  {
-    const double delta = R.delta, theta = R.theta;
-    for (int i = NTF - 1 - t; i < Sh::NE; i += NTF) {
-      const float4 d = A.cdesc[i];
-      double ph = theta * (double)d.y - (delta * (double)d.x + (double)d.z);
-      if (i == Sh::LAST + 3 && B.lsb) ph += 0.5;           // the lower sideband keeps a - w b
-      sm.tab[fi][i] = exact_rotator(ph);
-    }
-  }
-  if (NBITS == 2)
-    for (int i = tid; i < 256; i += NT) sm.quad[i] = A.quad[B.levels * 256 + i];
-  const bool fast = R.allvalid != 0 || dead;
-  if (t < GROUPS) {
-    if (NBITS == 8) {
-#pragma unroll
-      for (int m = 0; m < 4; m++) a[m] ^= 0x80808080u;     // signed levels, 0 = none
+    for (int m = 0; m < 4; m++) {
+      a[m] = __builtin_amdgcn_alignbit(hi[m], lo[m], (int)(bit0 & 31));
+      if (NBITS == 8) a[m] ^= 0x80808080u;                 // signed levels, 0 = none
     }
     if (!fast) {
       // a blanked sample has no 2-bit code: its validity is staged beside it;
@@ -195,7 +209,7 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
       unsigned v[4];
 #pragma unroll
       for (int m = 0; m < 4; m++) {
-        const long long ts = R.t0 + (long long)(m * GROUPS + t) * (32 / NBITS);
+        const long long ts = R.t0 + (long long)(m * GROUPS + g) * (32 / NBITS);
         v[m] = valid_samples<32 / NBITS>(S, Q, A.ftab, ts, R.validend, B.band);
         if (NBITS == 2) {
           v[m] = double_bits16(v[m]);
@@ -206,13 +220,49 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
       }
       if (NBITS == 2) {
         quads2(v);
-        *(uint4*)&ok[4 * t] = make_uint4(v[0], v[1], v[2], v[3]);
+        *(uint4*)&ok[4 * g] = make_uint4(v[0], v[1], v[2], v[3]);
       }
     }
     if (NBITS == 8) quads8(a); else quads2(a);
-    *(uint4*)&raw[4 * t] = make_uint4(a[0], a[1], a[2], a[3]);
+    *(uint4*)&raw[4 * g] = make_uint4(a[0], a[1], a[2], a[3]);
+  };
+#pragma unroll
+  for (int i = 0; i < AHEAD; i++)
+    if (t + i * NTF < GROUPS) load_rows(t + i * NTF, lo[i], hi[i]);
+  float4 level;                                            // PW > 1: the levels of quad byte tid % 256
+  if (NBITS == 2 && PW > 1) level = A.quad[B.levels * 256 + (tid & 255)];
+  // ---- this block's twiddles and fractional-sample steps
+  {
+    const double delta = R.delta, theta = R.theta;
+    for (int i = NTF - 1 - t; i < Sh::NE; i += NTF) {
+      const float4 d = A.cdesc[i];
+      double ph = theta * (double)d.y - (delta * (double)d.x + (double)d.z);
+      if (PW > 1) ph -= (double)pw * (double)d.w;
+      if (i == Sh::LAST + 3 && B.lsb) ph += 0.5;           // the lower sideband keeps a - w b
+      sm.tab[fi][i] = exact_rotator(ph);
+    }
+  }
+  if (NBITS == 2 && PW == 1)
+    for (int i = tid; i < 256; i += NT) sm.quad[i] = A.quad[B.levels * 256 + i];
+#pragma unroll
+  for (int i0 = 0; i0 < NIT; i0 += AHEAD) {
+    if (i0 > 0) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; i++)
+        if (t + (i0 + i) * NTF < GROUPS) load_rows(t + (i0 + i) * NTF, lo[i], hi[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++)
+      if (t + (i0 + i) * NTF < GROUPS) store_quads(t + (i0 + i) * NTF, lo[i], hi[i]);
   }
   __syncthreads();
+  if (NBITS == 2 && PW > 1) {
+    if (tid < 256 * Sh::NSUM) {
+      const float2* g = sm.tab[0] + (tid >> 8) * Sh::CP + 9;
+      sm.sums[tid] = quad_sum(level, g[0], g[1], g[2]);
+    }
+    __syncthreads();
+  }
 
   // workgroup barrier, or (a block's threads within one wavefront) only an
   // order for the compiler: LDS accesses of a wavefront complete in order
@@ -236,8 +286,8 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
     w.w8 = c[0]; w.w4 = c[1]; w.w2 = c[2]; w.w2h = c[3]; w.w1 = c[4]; w.w1a = c[5]; w.w1b = c[6]; w.w1c = c[7];
     // Quads of samples j + r J1, QN at a time, all their LDS reads in flight
     // together: bytes within a group of 16 in the order of quads2.
-    constexpr int NQ = R1 / 4, QN = NQ > 8 ? 8 : NQ;
-    auto quads_at = [&](int r0, float4* x) {
+    constexpr int QN = P == 1 && PW == 1 ? 4 : 8;
+    auto quads_at = [&](int r0, float4* x) {                // r0 + r counts J1 samples
       if (NBITS == 8) {
         unsigned q[QN];
 #pragma unroll
@@ -253,7 +303,7 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
 #pragma unroll
         for (int r = 0; r < QN; r++) q[r] = ((const unsigned char*)raw)[at(r0 + r)];
 #pragma unroll
-        for (int r = 0; r < QN; r++) x[r] = sm.quad[q[r]];
+        for (int r = 0; r < QN; r++) x[r] = PW == 1 ? sm.quad[q[r]] : A.quad[B.levels * 256 + q[r]];
         if (!fast) {
 #pragma unroll
           for (int r = 0; r < QN; r++) {
@@ -267,7 +317,43 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
       }
     };
     float2 v[16];
-    if (P == 1) {
+    if (PW > 1) {
+      // QSUM quads 16 J1 samples apart, the later ones times powers of c[8]
+      constexpr int QS = PW > 1 ? Sh::QSUM : 1;
+      const float2 g1 = c[9], g2 = c[10], g3 = c[11], w1 = c[8];
+      if (NBITS == 2 && fast) {
+        const float2* sums = sm.sums + (p % (PW > 1 ? Sh::NSUM : 1)) * 256;
+        const unsigned char* q0 = (const unsigned char*)raw + (j & ~15) + ((j & 3) << 2) + ((j >> 2) & 3);
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+          unsigned q[4 * QS];
+#pragma unroll
+          for (int i = 0; i < 4 * QS; i++) q[i] = q0[(4 * h + i / QS + 16 * (i % QS)) * J1];
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            float2 x = sums[q[r * QS + QS - 1]];
+#pragma unroll
+            for (int m = QS - 2; m >= 0; m--) x = bfly_plus(sums[q[r * QS + m]], x, w1);
+            v[4 * h + r] = x;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int m = QS - 1; m >= 0; m--)
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            float4 xq[QN];
+            quads_at(8 * h + 16 * m, xq);
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+              const float2 x = quad_sum(xq[r], g1, g2, g3);
+              v[8 * h + r] = m == QS - 1 ? x : bfly_plus(x, v[8 * h + r], w1);
+            }
+          }
+      }
+#pragma unroll
+      for (int r = 0; r < 8; r++) bfly(v[r], v[r + 8], w.w8);
+    } else if (P == 1) {
       // samples r, r + 4, r + 8, r + 12
       float4 xq[QN];
       quads_at(0, xq);
@@ -302,11 +388,7 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
         float4 xq[QN];
         quads_at(8 * h, xq);
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
-          const float4 x = xq[r];
-          v[8 * h + r] = make_float2(__builtin_fmaf(g3.x, x.w, __builtin_fmaf(g2.x, x.z, __builtin_fmaf(g1.x, x.y, x.x))),
-                                     __builtin_fmaf(g3.y, x.w, __builtin_fmaf(g2.y, x.z, g1.y * x.y)));
-        }
+        for (int r = 0; r < 8; r++) v[8 * h + r] = quad_sum(xq[r], g1, g2, g3);
       }
 #pragma unroll
       for (int r = 0; r < 8; r++) bfly(v[r], v[r + 8], w.w8);
@@ -314,6 +396,7 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
     dft16_stage2(v, w);
     dft16_stage3(v, w);
     dft16_stage4<false>(v, w);
+    if (PW > 1) __syncthreads();                           // every quad read before the buffer is written
 #pragma unroll
     for (int q = 0; q < 16; q++) {
       const int k = P * q + p;
@@ -347,14 +430,14 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
   float2 w[RL == 16 ? 4 : 6];
 #pragma unroll
   for (int i = 0; i < (RL == 16 ? 4 : 6); i++) w[i] = A.base[i * NTF + t];
-  // channel t + e L/16: this thread's phase (FP64, in turns) times E[e]
+  // channel PW (t + e M/16) + pw: this thread's phase (FP64, in turns) times E[e]
   float2 F;
   {
     const float s = dead ? 0.0f : (NBITS == 8 ? A.scale * (float)(1.0 / 3.3) : A.scale);
-    F = cmulx(exact_rotator(R.phase + R.theta * (double)t), make_float2(B.polre * s, B.polim * s));
+    F = cmulx(exact_rotator(R.phase + R.theta * (double)(PW * t + pw)), make_float2(B.polre * s, B.polim * s));
   }
   sync();
-  float2 x[8];                                             // channel t + e L/16
+  float2 x[8];                                             // bin t + e M/16
   const float2* cl = tab + Sh::LAST;
   if (RL == 16) {
     Tw16 tw;
@@ -379,12 +462,12 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
   }
   if (!mine) return;
   const float2* E = tab + Sh::LAST + 4;
-  const long long c0 = cidx(t, A.gstride), cstep = (NTF / 16) * A.gstride;
+  const long long c0 = cidx(PW * t + pw, A.gstride), cstep = (PW * NTF / 16) * A.gstride;
   auto store = [&](auto out) {
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       const long long at = NTF % 16 == 0 ? c0 + e * cstep : cidx(t + e * NTF, A.gstride);
-      put_spec(out, at, t + e * NTF, cmulx(x[e], cmulx(F, E[e])));
+      put_spec(out, at, PW * (t + e * NTF) + pw, cmulx(x[e], cmulx(F, E[e])));
     }
   };
   if (A.prec == FXG_XMAC_FP32) store((float2*)A.spectra + outbase);
@@ -399,28 +482,34 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
 template <int L>
 static void fill_tables(std::vector<float4>* cdesc, std::vector<float2>* base) {
   using Sh = FsShape<L>;
+  constexpr int M = Sh::M, PW = Sh::PW, P = Sh::P;
   cdesc->assign(Sh::NE, make_float4(0.f, 0.f, 0.f, 0.f));
-  // entry = e^{2 pi i (theta y - delta x - z)}
-  auto set = [&](int i, double x, double z, double y = 0.0) {
-    (*cdesc)[i] = make_float4((float)x, (float)y, (float)(z - std::floor(z)), 0.f);
+  // entry = e^{2 pi i (theta y - delta x - z - pw w)}
+  auto set = [&](int i, double x, double z, double w, double y = 0.0) {
+    (*cdesc)[i] = make_float4((float)x, (float)y, (float)(z - std::floor(z)), (float)w);
   };
-  // the eight twiddles of a radix-16 pass to N bins at bin k (w = e^{-2 pi i (k + d)/N})
+  // the eight twiddles of a radix-16 pass to N bins at bin k: powers of
+  // e^{-2 pi i (k + d)/N}, d = (pw + delta L)/PW
   auto tw16 = [&](int i, int N, double k) {
     const int m[8] = {8, 4, 2, 2, 1, 1, 1, 1};
     const double add[8] = {0, 0, 0, 1.0 / 8, 0, 1.0 / 16, 2.0 / 16, 3.0 / 16};
-    for (int e = 0; e < 8; e++) set(i + e, (double)(L / N) * m[e], k * m[e] / N + add[e]);
+    for (int e = 0; e < 8; e++) set(i + e, (double)(M / N) * m[e], k * m[e] / N + add[e], (double)m[e] / (PW * N));
   };
-  for (int p = 0; p < Sh::P; p++) {
-    tw16(p * Sh::CP, 16 * Sh::P, p);
-    for (int m = 1; m < 4 && Sh::P > 1; m++) {
+  for (int p = 0; p < P; p++) {
+    const int i = p * Sh::CP;
+    tw16(i, 16 * P, p);
+    if (PW > 1) {
+      // samples 16 J1 apart, then a quarter of the block apart
+      set(i + 8, L / (P * PW), (double)p / P, 1.0 / (P * PW));
+      for (int e = 1; e < 4; e++) set(i + 8 + e, (double)(L / 4) * e, 0.25 * PW * p * e, 0.25 * e);
+    } else if (P > 1) {
       // samples a quarter of the block apart (m = 1 is w^8 where P = 2)
-      if (Sh::P == 2 && m == 1) continue;
-      set(p * Sh::CP + (Sh::P == 2 ? 6 + m : 7 + m), (double)(L / 4) * m, 0.25 * p * m);
+      for (int m = P == 2 ? 2 : 1; m < 4; m++) set(i + (P == 2 ? 6 + m : 7 + m), (double)(L / 4) * m, 0.25 * p * m, 0.0);
     }
   }
   const int ml[4] = {8, 4, 2, 1};
-  for (int i = 0; i < 4; i++) set(Sh::LAST + i, ml[i], 0.0);
-  for (int e = 0; e < 8; e++) set(Sh::LAST + 4 + e, 0.0, 0.0, (double)(L / 16) * e);
+  for (int i = 0; i < 4; i++) set(Sh::LAST + i, ml[i], 0.0, (double)ml[i] / L);
+  for (int e = 0; e < 8; e++) set(Sh::LAST + 4 + e, 0.0, 0.0, 0.0, (double)(L / 16) * e);
   if (Sh::MID)
     for (int k = 0; k < Sh::R1; k++) tw16(Sh::MIDOFF + 8 * k, 16 * Sh::R1, k);
   // last pass at d = 0: powers 8, 4, 2, 1 (radix 16) or 4, 2, 1 of its two
@@ -429,12 +518,13 @@ static void fill_tables(std::vector<float4>* cdesc, std::vector<float2>* base) {
   const int nb = Sh::RL == 16 ? 4 : 3, nu = Sh::RL == 16 ? 1 : 2;
   for (int i = 0; i < nb; i++)
     for (int k = 0; k < nu * Sh::NTF; k++) {
-      const double ang = -kTwoPi * (double)k * (1 << (nb - 1 - i)) / L;
+      const double ang = -kTwoPi * (double)k * (1 << (nb - 1 - i)) / M;
       base->push_back(make_float2((float)std::cos(ang), (float)std::sin(ang)));
     }
 }
 
-#define FX_LENGTHS(X) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192) X(16384)
+#define FX_LENGTHS(X) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192) X(16384) \
+  X(32768) X(65536)
 
 bool fstage_lin_tables(int L, std::vector<float4>* cdesc, std::vector<float2>* base) {
   switch (L) {
@@ -457,7 +547,7 @@ hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, int nbands, 
   switch (L) {
 #define X(Lv)                                                                                                       \
     case Lv: {                                                                                                      \
-      const dim3 grid((unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8), nbands);         \
+      const dim3 grid((unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8 * FsShape<Lv>::PW), nbands); \
       if (nbits == 2) hipLaunchKernelGGL((k_fstage_lin<Lv, 2>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);         \
       else hipLaunchKernelGGL((k_fstage_lin<Lv, 8>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);                    \
       break;                                                                                                        \

@@ -11,8 +11,8 @@ namespace fxg {
 // LDS entries for an F-stage workgroup's rotator tables (sub, step,
 // fractional sub and step, quadratic pieces) at FFT length L
 constexpr int fxg_rotator_table_entries(int L) { return L >= 16384 ? 768 : 512; }
-// the largest FFT length of the single-workgroup F stage; longer ones (to
-// 65536) take the two-kernel path
+// the largest FFT length of one workgroup; longer ones (to 65536) take
+// several (linear and post-F rotation) or the two-kernel path (quadratic)
 constexpr int kFStageMaxL = 16384;
 
 // Spectra layout.  Channel c of the spectrum of one (band, pass block) sits
@@ -39,7 +39,7 @@ struct FStageArgs {
   float scale;                // applied before reduced-precision stores
   int nblocks_subint;
   int chunk0;                 // first block of the chunk
-  // FFTs above 16384 points run zcap blocks of the chunk at a time:
+  // quadratic rotation above 16384 points runs zcap blocks of the chunk at a time:
   float2* zbuf;               // sub-FFT scratch [band][zcap][16][L/16]
   float2* rtab;               // rotator tables [band][zcap][rtabn] (sub, step, quad, frac sub, frac step)
   int zcap;                   // blocks per sub-chunk
@@ -48,9 +48,9 @@ struct FStageArgs {
   const signed char* cexp;    // fp8: power-of-two scale exponent per [global band][channel]
   long long gstride;          // spectra layout (cidx)
   int bstride;
-  // linear and post-F rotation, transforms up to kFStageMaxL points:
+  // linear and post-F rotation:
   const DevRot* rots;         // [rotation][block of the subintegration]
-  const float4* cdesc;        // per-block table entries e^{2 pi i (theta y - delta x - z)}
+  const float4* cdesc;        // per-block table entries e^{2 pi i (theta y - delta x - z - pw w)}
   const float2* base;         // last-pass twiddles at d = 0, per thread
   const float4* quad;         // levels of four 2-bit samples by their byte: VDIF, Mark5B
   int nchunk;                 // blocks of the launch
@@ -138,7 +138,7 @@ hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const 
                            DevRot* rots, hipStream_t stream);
 // cplx: complex samples (L = nchan, every output of the transform kept)
 hipError_t launch_fstage(int L, int nbits, int cplx, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
-// linear and post-F rotation of real samples, L <= kFStageMaxL; its tables for
+// linear and post-F rotation of real samples; its tables for
 // one length, and the levels of four 2-bit samples by their byte (256 entries)
 hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
 bool fstage_lin_tables(int L, std::vector<float4>* cdesc, std::vector<float2>* base);

@@ -752,12 +752,12 @@ int build_plan(const fxg_job_desc* d, Plan* p, std::string* err) {
   chunk = std::min(chunk, d->blockspersend);
   P.chunk_blocks = chunk;
   P.info.chunk_blocks = chunk;
-  // FFTs above 16384 points: a scratch of about 160 MiB takes zcap blocks of
+  // quadratic rotation above 16384 points: a scratch of about 160 MiB takes zcap blocks of
   // the chunk at a time, with their rotator tables; at that size the second
   // kernel reads back what the first wrote from the 256 MB Infinity Cache
   // rather than from HBM (measured: the 65536-point job of the uneven mix
   // 54.0 -> 51.5 ms per subint against a 2 GiB scratch)
-  if (P.L > 16384) {
+  if (P.L > 16384 && d->fringe_order == 2) {
     P.zcap = (int)std::max(1LL, std::min<long long>(chunk, (160LL << 20) / ((long long)P.nbands_total * P.L * 8)));
     for (const DevStation& st : P.st) P.rtabn = std::max(P.rtabn, 3 * st.s + st.nfrsteps + st.nfracsteps);
   }
@@ -783,7 +783,7 @@ int64_t plan_device_bytes(const Plan& p, const fxg_job_desc* d) {
                      d->blockspersend;
   long long res = p.info.result_length * 8;
   long long tables = (long long)p.segs.size() * sizeof(DevSeg) + p.bands.size() * sizeof(DevBand) + (1 << 20);
-  long long z = p.L > 16384 ? (long long)p.nbands_total * p.zcap * ((long long)p.L + p.rtabn) * 8 : 0;
+  long long z = p.zcap > 0 ? (long long)p.nbands_total * p.zcap * ((long long)p.L + p.rtabn) * 8 : 0;
   long long vpart = p.vpart_elems * 8;
   long long pcal = p.pcal_partfloats * 4 + (long long)p.pcal_aux.size() * 4 +
                    (long long)p.pcal.size() * sizeof(DevPcal) + (long long)p.pcal_tonebin.size() * 4;

@@ -1296,7 +1296,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
 }
 
 // ---------------------------------------------------------------------------
-// FFT lengths above 16384: L = 16 M and
+// FFT lengths above 16384 with quadratic fringe rotation: L = 16 M and
 //     X[k2 + M k1] = sum_n1 W_16^(n1 k1) W_L^(n1 k2) Y_n1[k2],
 // Y_n1 the M-point FFT of x[n1 + 16 n2], n2 < M.  k_bigfft_a: one workgroup
 // per (block, band, n1) decodes and fringe-rotates its decimated samples,
@@ -1353,7 +1353,7 @@ __global__ __launch_bounds__(FftShape<M>::NT) void k_bigfft_a(FStageArgs A) {
     // the rotator table entries, all loads in flight before the LDS stores
     constexpr int NROT = (fxg_rotator_table_entries(L) + NT - 1) / NT;
     const float2* rt = A.rtab + ((long long)gband * A.zcap + cbl) * A.rtabn;
-    const int nrot = S.order == 0 ? 0 : (S.order == 2 ? 2 * S.s : S.s) + S.nfrsteps;
+    const int nrot = 2 * S.s + S.nfrsteps;
     float2 rr[NROT];
 #pragma unroll
     for (int q = 0; q < NROT; q++) {
@@ -1390,21 +1390,9 @@ __global__ __launch_bounds__(FftShape<M>::NT) void k_bigfft_a(FStageArgs A) {
     const long long bq = bit0 + (long long)NBITS * n0;
     const long long wq = bq >> 5;
     const int sh = (int)(bq & 31);
-    const bool wordfast = fast && (S.order == 1 || S.order == 2) && slog >= 0 && ((16 * NTF) & (s - 1)) == 0 &&
+    const bool wordfast = fast && slog >= 0 && ((16 * NTF) & (s - 1)) == 0 &&
                           wq + 15LL * WSTEP < nwords;
-    if (wordfast && S.order == 1) {
-      const float2 r0 = rsub[n0 & (s - 1)];
-      const float2* stp = rstep + (n0 >> slog);
-      const int sstep = (16 * NTF) >> slog;
-      const unsigned* wp = stream + wq;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const float x = lut8s[(wp[r * WSTEP] >> sh) & ((1u << NBITS) - 1u)];
-        const float2 rot = cmulf(r0, *stp);     // sub[k] * step[j], mode.cpp:975-977
-        stp += sstep;
-        v[r] = make_float2(x * rot.x, x * rot.y);
-      }
-    } else if (wordfast) {
+    if (wordfast) {
       // piecewise quadratic rotator: piece_q[k] = sub[k] quad[k]^q, one
       // product chain per thread carried from point to point (the same
       // products, in the same order, as rebuilding it for each point)
@@ -1435,20 +1423,13 @@ __global__ __launch_bounds__(FftShape<M>::NT) void k_bigfft_a(FStageArgs A) {
       } else {
         x = sample_value(S, Q, A.ftab, NBITS == 8 ? lut8s : A.lut8, lut2, t0 + n, G.validend, B.band);
       }
-      float2 rot = make_float2(1.0f, 0.0f);
-      if (S.order != 0) {
-        const int kk = slog >= 0 ? (n & (s - 1)) : n % s;
-        const int jj = slog >= 0 ? (n >> slog) : n / s;
-        if (S.order == 1) {
-          rot = n < s ? rsub[n] : cmulf(rsub[kk], rstep[jj]);
-        } else {
-          const float2 qd = rquad[kk];
-          float2 piece = rsub[kk];
-          for (int i = 0; i < jj; i++) piece = cmulf(piece, qd);
-          rot = cmulf(piece, rstep[jj]);
-        }
-      }
-      v[r] = S.order == 0 ? make_float2(x, 0.0f) : make_float2(x * rot.x, x * rot.y);
+      const int kk = slog >= 0 ? (n & (s - 1)) : n % s;
+      const int jj = slog >= 0 ? (n >> slog) : n / s;
+      const float2 qd = rquad[kk];
+      float2 piece = rsub[kk];
+      for (int i = 0; i < jj; i++) piece = cmulf(piece, qd);
+      const float2 rot = cmulf(piece, rstep[jj]);
+      v[r] = make_float2(x * rot.x, x * rot.y);
     }
     }
     DFT<16>::run(v);

@@ -17,8 +17,10 @@ from fxtestlib import GpuJob, oracle_spectra, rel_err
 
 pytestmark = pytest.mark.gpu
 
-# (channels, blocks): lengths 128..16384; one workgroup holds 32, 16, 8, 4 or 1 blocks
-SHAPES = [(64, 1), (64, 33), (128, 17), (256, 7), (256, 9), (512, 5), (1024, 3), (2048, 2), (4096, 2), (8192, 2)]
+# (channels, blocks): lengths 128..65536; one workgroup holds 32, 16, 8, 4 or 1 blocks, and above 16384 points a half
+# or a quarter
+SHAPES = [(64, 1), (64, 33), (128, 17), (256, 7), (256, 9), (512, 5), (1024, 3), (2048, 2), (4096, 2), (8192, 2),
+          (16384, 2), (32768, 2)]
 
 
 @pytest.mark.parametrize("order", [0, 1])
