@@ -926,10 +926,9 @@ static void xmac_shape(int nin, int nchan, XmacArgs* a, int ct_req = 0, int tb_r
 // buffers: a graph captured for one shape replays for every subintegration of
 // the same shape.
 struct LaunchShape {
-  long long maxframes = 0, maxsamples = 0;
-  int maxdatabytes = 0;
-  int fastW = 0;        // 2-bit register corner turn: W words per sample-time, else 0
+  CornerTurn ct;
 };
+static_assert(sizeof(CornerTurn) == 3 * sizeof(long long) + 6 * sizeof(int), "graph_key compares its bytes");
 
 // Raw data (host inputs), the per-datastream subint table and the valid
 // flags of one subintegration, copied to the device on stream s.  With
@@ -956,9 +955,9 @@ static int upload_subint(fxg_job* j, const fxg_subint_desc* sub, const fxg_stati
   }
   std::vector<DevStationSub> ss(P.nds);
   std::vector<int> flags;
-  long long fbase = 0, maxframes = 0, ctbytes = 0, maxsamples = 0;
-  int maxdatabytes = 0;
-  int fastW = -1;
+  long long fbase = 0, ctbytes = 0;
+  CornerTurn turn;
+  int fastW = -1, unit = -1;
   for (int d = 0; d < P.nds; d++) {
     const fxg_station_input& in = st[d];
     DevStationSub& q = ss[d];
@@ -986,16 +985,26 @@ static int upload_subint(fxg_job* j, const fxg_subint_desc* sub, const fxg_stati
     q.ctbase = ctbytes;
     q.ctstride = ((q.nframes * P.st[d].bpf + 3) / 4) * 4;
     ctbytes += q.ctstride * P.st[d].nchan;
-    maxdatabytes = std::max(maxdatabytes, P.st[d].databytes);
-    maxframes = std::max(maxframes, q.nframes);
+    turn.maxdatabytes = std::max(turn.maxdatabytes, P.st[d].databytes);
+    turn.maxframes = std::max(turn.maxframes, q.nframes);
     {
       const DevStation& S = P.st[d];
+      const uintptr_t align = (uintptr_t)q.data | (uintptr_t)S.framebytes | (uintptr_t)S.headerbytes | (uintptr_t)S.databytes;
       const int W = S.nbits == 2 && !S.cplx && S.nchan % 16 == 0 ? S.nchan / 16 : 0;
-      const bool ok = (W == 1 || W == 2 || W == 4) &&
-                      (((uintptr_t)q.data | (uintptr_t)S.framebytes | (uintptr_t)S.headerbytes |
-                        (uintptr_t)S.databytes) % (4 * W)) == 0;
+      const bool ok = (W == 1 || W == 2 || W == 4) && align % (4 * W) == 0;
       if (q.nframes > 0) fastW = (ok && (fastW < 0 || fastW == W)) ? W : 0;
-      if (W) maxsamples = std::max(maxsamples, q.nframes * (S.databytes / (4 * W)));
+      if (W) turn.maxsamples = std::max(turn.maxsamples, q.nframes * (S.databytes / (4 * W)));
+      // the register kernel for any unit size and band count: one shape for
+      // every datastream, the loads as wide as the least aligned one allows
+      int logn = 0;
+      while ((1 << logn) < S.nchan) logn++;
+      const int vec = logn >= 2 && logn <= 5 && align % 16 == 0 ? 4 : logn >= 1 && align % 8 == 0 ? 2 : logn == 0 && align % 4 == 0 ? 1 : 0;
+      if (q.nframes > 0) {
+        if (unit < 0 && vec) { unit = S.unitbits; turn.logn = logn; turn.vec = vec; }
+        else if (!vec || unit != S.unitbits || turn.logn != logn) unit = 0;
+        else turn.vec = std::min(turn.vec, vec);
+        turn.maxgroups = std::max(turn.maxgroups, (q.nframes * (S.databytes / 4) + S.nchan - 1) / S.nchan);
+      }
     }
     q.datasec = in.sec; q.datans = in.ns;
     q.datasamples = static_cast<int>(in.ns / (P.st[d].sampletime * 1e3) + 0.5);   // mode.cpp:1572
@@ -1048,10 +1057,9 @@ static int upload_subint(fxg_job* j, const fxg_subint_desc* sub, const fxg_stati
   if (!flags.empty()) HIPCHK(hipMemcpyAsync(j->d_flags.p, hs.flags, sizeof(int) * flags.size(), hipMemcpyHostToDevice, s));
   HIPCHK(hipEventRecord(hs.done, s));
   hs.queued = true;
-  sh->maxframes = maxframes;
-  sh->maxsamples = maxsamples;
-  sh->maxdatabytes = maxdatabytes;
-  sh->fastW = fastW > 0 ? fastW : 0;
+  turn.fastW = fastW > 0 ? fastW : 0;
+  turn.unit = unit > 0 ? unit : 0;
+  sh->ct = turn;
   return 0;
 }
 
@@ -1062,9 +1070,9 @@ static int launch_front(fxg_job* j, const LaunchShape& sh, hipStream_t s) {
   int rc;
   if ((rc = j->ev_begin(FXG_STAGE_FRAMES))) return rc;
   HIPCHK(launch_frames(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_ftab.as<int2>(), P.nds,
-                       sh.maxframes, s));
+                       sh.ct.maxframes, s));
   HIPCHK(launch_cornerturn(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_ct.as<unsigned char>(),
-                           P.nds, sh.maxframes, sh.maxdatabytes, sh.fastW, sh.maxsamples, s));
+                           P.nds, sh.ct, s));
   if ((rc = j->ev_end())) return rc;
   if ((rc = j->ev_begin(FXG_STAGE_PROLOGUE))) return rc;
   HIPCHK(launch_prologue(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_flags.as<int>(),

@@ -130,9 +130,18 @@ hipError_t launch_frame_digest(const unsigned char* data, long long f0, long lon
 unsigned long long host_frame_digest(const unsigned char* p, int n);
 hipError_t launch_frames(const DevStation* st, const DevStationSub* ss, int2* ftab, int nst,
                          long long maxframes, hipStream_t stream);
+// The corner turn of one subintegration: its largest station, and the
+// register kernel that every datastream's shape and alignment allow
+struct CornerTurn {
+  long long maxframes = 0, maxsamples = 0, maxgroups = 0;
+  int maxdatabytes = 0;
+  int fastW = 0;        // k_cornerturn2: 2-bit frames of W whole words per sample-time, else 0
+  int unit = 0;         // k_cornerturn_u: bits per unit, log2 of the bands, words per load; unit 0: the
+  int logn = 0, vec = 0;   // general kernel
+  int pad = 0;          // (compared byte by byte: no gaps)
+};
 hipError_t launch_cornerturn(const DevStation* st, const DevStationSub* ss, unsigned char* ct, int nst,
-                             long long maxframes, int maxdatabytes, int fastW, long long maxsamples,
-                             hipStream_t stream);
+                             const CornerTurn& c, hipStream_t stream);
 hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const int* flags,
                            const int2* ftab, int nblocks, DevBlock* out, int nst, const DevRotGroup* groups,
                            DevRot* rots, hipStream_t stream);

@@ -13,7 +13,6 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_bf16.h>
 #include "fx_kernels.h"
-#include "fx_bits.h"
 #include "fx_device.h"
 #include "fx_spectra.h"
 #include <type_traits>
@@ -501,135 +500,6 @@ __device__ __forceinline__ void twiddlesR(const float2* lo, const float2* hi, in
 // LDS index with one pad slot per 16 complex values: spreads the strided
 // Stockham writes of the early passes over the banks
 __device__ __forceinline__ int pidx(int a) { return a + (a >> 4); }
-
-// ---------------------------------------------------------------------------
-// k_cornerturn: one workgroup per (frame, datastream).  De-interleaves the
-// frame payload (sample-time major, channel minor) into one contiguous
-// sample stream per band, unitbits per sample (nbits, or 2 nbits for complex
-// samples), LSB first, so that the F-stage of one band reads L*unitbits/8
-// contiguous bytes per FFT block.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_cornerturn(const DevStation* __restrict__ st,
-                                                    const DevStationSub* __restrict__ ss,
-                                                    unsigned char* __restrict__ ct) {
-  extern __shared__ unsigned char pay[];
-  const int s = blockIdx.y;
-  const DevStation S = st[s];
-  const DevStationSub Q = ss[s];
-  const long long f = blockIdx.x;
-  if (f >= Q.nframes) return;
-  const unsigned char* src = Q.data + f * S.framebytes + S.headerbytes;
-  if ((((unsigned long long)Q.data | (unsigned long long)S.framebytes | (unsigned long long)S.headerbytes) & 3) == 0) {
-    // eight words per thread in flight before their LDS stores
-    const unsigned* s32 = (const unsigned*)src;
-    unsigned* p32 = (unsigned*)pay;
-    const int nw = S.databytes / 4;
-    for (int i0 = threadIdx.x; i0 < nw; i0 += 8 * blockDim.x) {
-      unsigned w[8];
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        const int i = i0 + q * blockDim.x;
-        if (i < nw) w[q] = s32[i];
-      }
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        const int i = i0 + q * blockDim.x;
-        if (i < nw) p32[i] = w[q];
-      }
-    }
-  } else {
-    for (int i = threadIdx.x; i < S.databytes; i += blockDim.x) pay[i] = src[i];
-  }
-  __syncthreads();
-  const int nbits = S.unitbits, nchan = S.nchan, bpf = S.bpf;
-  if (nbits >= 8) {
-    // units of whole bytes (complex 8-bit: two bytes per unit)
-    const int bpu = nbits / 8;
-    for (int ob = threadIdx.x; ob < nchan * bpf; ob += blockDim.x) {
-      const int c = ob / bpf, i = ob - c * bpf;
-      const int u = i / bpu;
-      ct[Q.ctbase + (long long)c * Q.ctstride + f * bpf + i] = pay[(u * nchan + c) * bpu + (i - u * bpu)];
-    }
-    return;
-  }
-  const int per = 8 / nbits;                   // samples per output byte
-  const unsigned mask = (1u << nbits) - 1u;
-  for (int ob = threadIdx.x; ob < nchan * bpf; ob += blockDim.x) {
-    const int c = ob / bpf, i = ob - c * bpf;
-    unsigned v = 0;
-    for (int k = 0; k < per; k++) {
-      const int bit = ((i * per + k) * nchan + c) * nbits;
-      v |= ((pay[bit >> 3] >> (bit & 7)) & mask) << (k * nbits);
-    }
-    ct[Q.ctbase + (long long)c * Q.ctstride + f * bpf + i] = (unsigned char)v;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// k_cornerturn2<W>: the same corner turn for 2-bit frames whose sample-times
-// are W whole 32-bit words (16 W bands), used when every datastream has that
-// shape and 4W-byte aligned frames.  A workgroup stages 4096 consecutive
-// sample-times through LDS with coalesced loads; each thread then turns 16
-// of them for all bands with a 2-bit transpose in registers and stores one
-// coalesced word per band.
-// ---------------------------------------------------------------------------
-template <int W>
-__global__ __launch_bounds__(256) void k_cornerturn2(const DevStation* __restrict__ st,
-                                                     const DevStationSub* __restrict__ ss,
-                                                     unsigned char* __restrict__ ct) {
-  using VW = typename std::conditional<W == 1, unsigned, typename std::conditional<W == 2, uint2, uint4>::type>::type;
-  constexpr int TPW = 16 * 256;                        // sample-times per workgroup
-  __shared__ VW buf[TPW + TPW / 16];                   // element i at i + i/16
-  const int s = blockIdx.y;
-  const DevStation S = st[s];
-  const DevStationSub Q = ss[s];
-  const long long spf = S.databytes / (4 * W);          // sample-times per frame
-  const long long total = Q.nframes * spf;
-  const long long base = (long long)blockIdx.x * TPW;
-  if (base >= total) return;                            // the whole workgroup
-  // frame f and sample-time r within it of this thread's sample-time, kept
-  // up to date as it steps by 256 (one division per workgroup)
-  const long long fw = base / spf;
-  long long f = fw;
-  long long r = base - fw * spf + threadIdx.x;
-  while (r >= spf) { r -= spf; f++; }
-  // all 16 loads in flight before the first LDS store
-  VW v[16];
-#pragma unroll
-  for (int k = 0; k < 16; k++) {
-    const long long tau = base + threadIdx.x + k * 256;
-    if (tau < total) {
-      v[k] = ((const VW*)(Q.data + f * S.framebytes + S.headerbytes))[r];
-    } else {
-      memset(&v[k], 0, sizeof v[k]);
-    }
-    r += 256;
-    while (r >= spf) { r -= spf; f++; }
-  }
-#pragma unroll
-  for (int k = 0; k < 16; k++) {
-    const int i = threadIdx.x + k * 256;
-    buf[i + (i >> 4)] = v[k];
-  }
-  __syncthreads();
-  const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (g * 16 >= total) return;
-  uint32_t w[W][16];
-#pragma unroll
-  for (int t = 0; t < 16; t++) {
-    const VW v = buf[threadIdx.x * 17 + t];
-    const uint32_t* pv = (const uint32_t*)&v;
-#pragma unroll
-    for (int c = 0; c < W; c++) w[c][t] = pv[c];
-  }
-#pragma unroll
-  for (int c = 0; c < W; c++) {
-    transpose16x2(w[c]);
-#pragma unroll
-    for (int k = 0; k < 16; k++)
-      ((uint32_t*)(ct + Q.ctbase + (long long)(16 * c + k) * Q.ctstride))[g] = w[c][k];
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Rotator tables of one (band, block) at FFT length L, by the threads tid of
@@ -1666,23 +1536,6 @@ hipError_t launch_fstage(int L, int nbits, int cplx, const FStageArgs& a, int nb
 #undef BIG
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
-}
-
-hipError_t launch_cornerturn(const DevStation* st, const DevStationSub* ss, unsigned char* ct, int nst,
-                             long long maxframes, int maxdatabytes, int fastW, long long maxsamples,
-                             hipStream_t stream) {
-  if (maxframes <= 0) return hipSuccess;
-  if (fastW) {
-    const long long groups = (maxsamples + 15) / 16;
-    dim3 grid((unsigned)((groups + 255) / 256), nst);
-    if (fastW == 1) hipLaunchKernelGGL(k_cornerturn2<1>, grid, dim3(256), 0, stream, st, ss, ct);
-    else if (fastW == 2) hipLaunchKernelGGL(k_cornerturn2<2>, grid, dim3(256), 0, stream, st, ss, ct);
-    else hipLaunchKernelGGL(k_cornerturn2<4>, grid, dim3(256), 0, stream, st, ss, ct);
-    return hipGetLastError();
-  }
-  dim3 grid((unsigned)maxframes, nst);
-  hipLaunchKernelGGL(k_cornerturn, grid, dim3(256), (size_t)maxdatabytes, stream, st, ss, ct);
   return hipGetLastError();
 }
 
