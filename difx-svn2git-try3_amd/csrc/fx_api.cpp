@@ -114,6 +114,8 @@ struct fxg_job {
   // per-subint
   DBuf d_ss, d_flags, d_ftab, d_blocks, d_weights, d_results, d_ct;
   DBuf d_rotgroups, d_rots;       // rotations of the bands, and of each block (k_prologue)
+  DBuf d_pairs;                   // band lists of that F stage
+  BandLists lists2, lists8;       // its 2-bit and 8-bit bands
   DBuf d_cdesc, d_base, d_quad;   // tables of the F stage with linear rotation (fx_fstage.hip)
   bool fstage_lin = false;        // that F stage runs: real samples, fringe orders 0 and 1
   DBuf d_bandlist;                // global bands grouped by sample size
@@ -548,7 +550,7 @@ static void job_free(fxg_job* j) {
                   &j->d_spec, &j->d_V, &j->d_ct, &j->d_bandlist, &j->d_iota, &j->d_zero, &j->d_z, &j->d_rtab,
                   &j->d_pcal, &j->d_pcalaux, &j->d_pcaltone, &j->d_pcalpart, &j->d_vpart, &j->d_cexp,
                   &j->d_eoff, &j->d_kurt, &j->d_kurtout, &j->d_kurtnz, &j->d_rotgroups, &j->d_rots, &j->d_cdesc,
-                  &j->d_base, &j->d_quad};
+                  &j->d_base, &j->d_quad, &j->d_pairs};
   for (DBuf* b : bufs) b->release();
   for (DBuf& b : j->d_raw) b.release();
   if (j->copy_stream) { (void)hipStreamSynchronize(j->copy_stream); (void)hipStreamDestroy(j->copy_stream); j->copy_stream = nullptr; }
@@ -748,6 +750,30 @@ int fxg_job_create(fxg_ctx* c, const fxg_job_desc* desc, fxg_job** out) {
         hipMemcpy(j->d_base.p, base.data(), sizeof(float2) * base.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(j->d_quad.p, quad.data(), sizeof(float4) * quad.size(), hipMemcpyHostToDevice) != hipSuccess)
       return fail(set_err(FXG_EHIP, "F-stage table upload failed"));
+    // [pairs of 2-bit bands][of 8-bit][single 2-bit bands][8-bit][every band by itself]
+    std::vector<int2> pl, single[2];
+    int npair[2] = {0, 0};
+    for (int b8 = 0; b8 < 2; b8++) {
+      std::vector<char> used(P.bands.size(), 0);
+      for (size_t g = 0; g < P.bands.size(); g++) {
+        if ((P.st[P.bands[g].station].nbits == 8) != (b8 == 1)) continue;
+        single[b8].push_back(make_int2((int)g, -1));
+        if (used[g]) continue;
+        int other = -1;
+        for (size_t h = g + 1; h < P.bands.size() && P.bands[h].station == P.bands[g].station && other < 0; h++)
+          if (!used[h] && P.bands[h].rot == P.bands[g].rot) { other = (int)h; used[h] = 1; }
+        pl.push_back(make_int2((int)g, other));
+        npair[b8]++;
+      }
+    }
+    for (int b8 = 0; b8 < 2; b8++) pl.insert(pl.end(), single[b8].begin(), single[b8].end());
+    for (size_t g = 0; g < P.bands.size(); g++) pl.push_back(make_int2((int)g, -1));
+    if ((rc = j->d_pairs.ensure(sizeof(int2) * pl.size()))) return fail(rc);
+    if (hipMemcpy(j->d_pairs.p, pl.data(), sizeof(int2) * pl.size(), hipMemcpyHostToDevice) != hipSuccess)
+      return fail(set_err(FXG_EHIP, "band list upload failed"));
+    const int2* dp = j->d_pairs.as<int2>();
+    j->lists2 = BandLists{dp, dp + npair[0] + npair[1], npair[0], (int)single[0].size()};
+    j->lists8 = BandLists{dp + npair[0], dp + npair[0] + npair[1] + single[0].size(), npair[1], (int)single[1].size()};
   }
   if (P.vpart_elems > 0) {
     if ((rc = j->d_vpart.ensure(sizeof(float2) * (size_t)P.vpart_elems))) return fail(rc);
@@ -1118,12 +1144,27 @@ static void fill_fstage_args(fxg_job* j, FStageArgs* fa) {
   fa->quad = j->d_quad.as<float4>();
 }
 
-// the F stage of nbands bands (fa.bandlist) of nbits-bit samples over nblocks blocks from fa.chunk0
-static hipError_t launch_job_fstage(const fxg_job* j, int nbits, const FStageArgs& fa, int nbands, int nblocks,
-                                    hipStream_t s) {
+// the F stage of every nbits-bit band over nblocks blocks from fa.chunk0
+static hipError_t launch_job_fstage(const fxg_job* j, int nbits, FStageArgs& fa, int nblocks, hipStream_t s) {
   const Plan& P = j->plan;
-  if (j->fstage_lin) return launch_fstage_lin(P.L, nbits, fa, nbands, nblocks, s);
-  return launch_fstage(P.L, nbits, P.st[0].cplx, fa, nbands, nblocks, s);
+  if (j->fstage_lin) return launch_fstage_lin(P.L, nbits, fa, nbits == 8 ? j->lists8 : j->lists2, nblocks, s);
+  fa.bandlist = j->d_bandlist.as<int>() + (nbits == 8 ? j->nb2 : 0);
+  return launch_fstage(P.L, nbits, P.st[0].cplx, fa, nbits == 8 ? j->nb8 : j->nb2, nblocks, s);
+}
+
+// and of the bands of datastream ds in block fa.chunk0
+static hipError_t launch_block_fstage(const fxg_job* j, int ds, FStageArgs& fa, hipStream_t s) {
+  const Plan& P = j->plan;
+  const DevStation& S = P.st[ds];
+  if (j->fstage_lin) {
+    BandLists l;
+    // the list of every band by itself, after the pairs and the lists by sample size
+    l.singles = j->lists8.singles + j->lists8.nsingles + S.band0;
+    l.nsingles = S.nchan;
+    return launch_fstage_lin(P.L, S.nbits, fa, l, 1, s);
+  }
+  fa.bandlist = j->d_iota.as<int>() + S.band0;
+  return launch_fstage(P.L, S.nbits, S.cplx, fa, S.nchan, 1, s);
 }
 
 // identity of a subintegration's inputs: the prepared state is reused while it matches
@@ -1168,14 +1209,8 @@ static int launch_back(fxg_job* j, float* dres, hipStream_t s) {
     int cn = std::min(chunk, nblocks - c0);
     fa.chunk0 = c0;
     if ((rc = j->ev_begin(FXG_STAGE_FSTAGE))) return rc;
-    if (j->nb2) {
-      fa.bandlist = j->d_bandlist.as<int>();
-      HIPCHK(launch_job_fstage(j, 2, fa, j->nb2, cn, s));
-    }
-    if (j->nb8) {
-      fa.bandlist = j->d_bandlist.as<int>() + j->nb2;
-      HIPCHK(launch_job_fstage(j, 8, fa, j->nb8, cn, s));
-    }
+    if (j->nb2) HIPCHK(launch_job_fstage(j, 2, fa, cn, s));
+    if (j->nb8) HIPCHK(launch_job_fstage(j, 8, fa, cn, s));
     if ((rc = j->ev_end())) return rc;
     if (j->kurt_on) {
       ka.chunk0 = c0; ka.nchunk = cn;
@@ -1713,8 +1748,7 @@ int fxg_station_process_block(fxg_job* j, const fxg_subint_desc* sub, const fxg_
   FStageArgs fa;
   fill_fstage_args(j, &fa);
   fa.chunk0 = block;
-  fa.bandlist = j->d_iota.as<int>() + P.st[ds].band0;
-  HIPCHK(launch_job_fstage(j, P.st[ds].nbits, fa, P.st[ds].nchan, 1, j->stream));
+  HIPCHK(launch_block_fstage(j, ds, fa, j->stream));
   HIPCHK(hipStreamSynchronize(j->stream));
   j->ev_collect();
   j->have_subint = 1;

@@ -28,6 +28,7 @@ template <int L> struct FsShape {
   static constexpr int NTF = M / 16, NB = NTF >= 128 ? 1 : 256 / NTF, NT = NTF * NB;
   static constexpr int CP = PW > 1 || P == 4 ? 12 : P == 2 ? 10 : 8, LAST = P * CP, MIDOFF = LAST + 12;
   static constexpr int NE = MIDOFF + (MID ? 8 * R1 : 0);
+  static constexpr bool TWO = MID && PW == 1;                  // takes two bands of one rotation
   // PW > 1: quads of one first-pass input, and tables of quad sums
   static constexpr int QSUM = P * PW / 4, NSUM = PW == 1 ? 0 : PW == 2 ? 2 : 1;
 };
@@ -121,14 +122,22 @@ __device__ __forceinline__ float2 quad_sum(const float4& x, float2 g1, float2 g2
 //     into lines.  One workgroup of 1024 threads and 16384 points a CU instead
 //     left the VALU idle half of the time (16384 points 18.4 ms, 65536 points
 //     28.0 ms on the workloads below).
+//   - from 2048 to 8192 points a workgroup takes both polarisations of a
+//     frequency, which share the rotation: its table, the last pass's twiddles
+//     and the channel rotators are formed once, and the second band's samples
+//     are in registers when the first is done.
+// (Tried and dropped: the first-stage outputs by the quad's byte from a table
+// per workgroup, 8192 points: 803 -> 746 VALU instructions a band, 25.2 -> 25.0
+// ms, the VALU 84 % busy instead of 90 %: what is left is the barriers that two
+// workgroups a CU do not cover.)
 // Exchanges are laid out so that both sides hit all banks with immediate
 // offsets: the one into the middle pass by exchanging pieces of J2 values
 // between neighbouring rows, the one into the last pass by a row pad.
 // Against the kernels with rotator tables and padded twiddle products, one
 // radix-2 pass more, and from 32768 points a scratch in HBM between two kernels
-// (rocprofv3, ms): 8192 points, 16.8 Gsamples 33.4 -> 25.9; 16384 points, 8.2
+// (rocprofv3, ms): 8192 points, 16.8 Gsamples 33.4 -> 25.2; 16384 points, 8.2
 // Gsamples 24.0 -> 14.5; 65536 points, 7.9 Gsamples 37.5 -> 23.2; 2048 points,
-// 1.34 Gsamples 3.23 -> 2.80; 512 points, 8-bit, 0.92 Gsamples 3.53 -> 1.37.
+// 1.34 Gsamples 3.23 -> 2.40; 512 points, 8-bit, 0.92 Gsamples 3.53 -> 1.29.
 // ---------------------------------------------------------------------------
 template <int L, int NBITS>
 __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) {
@@ -165,28 +174,31 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
   const int cbx = grp * NB + fi;
   const bool mine = NB == 1 || cbx < A.nchunk;
   const int cb = mine ? cbx : A.nchunk - 1;
-  const int gband = A.bandlist ? A.bandlist[blockIdx.y] : blockIdx.y;
-  const DevBand& B = A.bands[gband];
-  const DevStationSub& Q = A.ss[B.station];
-  const DevRot& R = A.rots[(long long)B.rot * A.nblocks_subint + A.chunk0 + cb];
+  // one band, or two that share a rotation (the polarisations of a frequency)
+  const int2 pair = A.pairs[blockIdx.y];
+  const int nband = Sh::TWO && pair.y >= 0 ? 2 : 1;
+  const DevBand& B0 = A.bands[pair.x];
+  const DevBand& B1 = A.bands[nband == 2 ? pair.y : pair.x];
+  const DevStationSub& Q = A.ss[B0.station];
+  const DevRot& R = A.rots[(long long)B0.rot * A.nblocks_subint + A.chunk0 + cb];
   constexpr int C = L / 2;
-  const long long outbase = B.specoff + (long long)cb * A.bstride;
   const bool dead = R.status != 0;
   if (NB == 1 && dead) {
-    if (pw == 0) zero_spec(A.spectra, A.prec, outbase, C, A.gstride, tid, NT);
+    for (int b = 0; b < nband && pw == 0; b++)
+      zero_spec(A.spectra, A.prec, (b ? B1 : B0).specoff + (long long)cb * A.bstride, C, A.gstride, tid, NT);
     return;
   }
 
-  // ---- the block's samples of this band: four rows a quarter block apart,
-  // their first loads in flight under the tables' sines
+  // ---- the block's samples of a band: four rows a quarter block apart, their
+  // first loads (and the second band's) in flight under the tables' sines
   constexpr int GROUPS = NBITS == 8 ? L / 16 : L / 64;
   const bool fast = R.allvalid != 0 || dead;
   const long long bit0 = (long long)(dead ? 0 : R.t0) * NBITS;
-  const unsigned* src = (const unsigned*)(A.ct + Q.ctbase + (long long)B.band * Q.ctstride);
   const long long nwords = Q.ctstride >> 2;
   constexpr int NIT = (GROUPS + NTF - 1) / NTF, AHEAD = NIT > 2 ? 2 : NIT;
-  unsigned lo[AHEAD][4], hi[AHEAD][4];
-  auto load_rows = [&](int g, unsigned (&lo)[4], unsigned (&hi)[4]) {
+  unsigned lo[AHEAD][4], hi[AHEAD][4], lo1[4], hi1[4];
+  auto load_rows = [&](const DevBand& B, int g, unsigned (&lo)[4], unsigned (&hi)[4]) {
+    const unsigned* src = (const unsigned*)(A.ct + Q.ctbase + (long long)B.band * Q.ctstride);
     const long long w0 = (bit0 >> 5) + g;
 #pragma unroll
     for (int m = 0; m < 4; m++) {
@@ -195,7 +207,7 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
       hi[m] = w + 1 < nwords ? src[w + 1] : 0u;
     }
   };
-  auto store_quads = [&](int g, const unsigned (&lo)[4], const unsigned (&hi)[4]) {
+  auto store_quads = [&](const DevBand& B, int g, const unsigned (&lo)[4], const unsigned (&hi)[4]) {
     unsigned a[4];
 #pragma unroll
     for (int m = 0; m < 4; m++) {
@@ -226,11 +238,26 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
     if (NBITS == 8) quads8(a); else quads2(a);
     *(uint4*)&raw[4 * g] = make_uint4(a[0], a[1], a[2], a[3]);
   };
+  auto load_ahead = [&](const DevBand& B, int i0) {
 #pragma unroll
-  for (int i = 0; i < AHEAD; i++)
-    if (t + i * NTF < GROUPS) load_rows(t + i * NTF, lo[i], hi[i]);
-  float4 level;                                            // PW > 1: the levels of quad byte tid % 256
-  if (NBITS == 2 && PW > 1) level = A.quad[B.levels * 256 + (tid & 255)];
+    for (int i = 0; i < AHEAD; i++)
+      if (t + (i0 + i) * NTF < GROUPS) load_rows(B, t + (i0 + i) * NTF, lo[i], hi[i]);
+  };
+  // the quads of a band whose first loads are in lo, hi
+  auto stage = [&](const DevBand& B) {
+#pragma unroll
+    for (int i0 = 0; i0 < NIT; i0 += AHEAD) {
+      if (i0 > 0) load_ahead(B, i0);
+#pragma unroll
+      for (int i = 0; i < AHEAD; i++)
+        if (t + (i0 + i) * NTF < GROUPS) store_quads(B, t + (i0 + i) * NTF, lo[i], hi[i]);
+    }
+  };
+  static_assert(!Sh::TWO || (NIT == 1 && RAWOWN), "the second band's rows are one round, into the first's place");
+  load_ahead(B0, 0);
+  if (Sh::TWO && t < GROUPS) load_rows(B1, t, lo1, hi1);
+  float4 level;                                            // of quad byte tid % 256, for the tables below
+  if (NBITS == 2 && PW > 1) level = A.quad[B0.levels * 256 + (tid & 255)];
   // ---- this block's twiddles and fractional-sample steps
   {
     const double delta = R.delta, theta = R.theta;
@@ -238,23 +265,13 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
       const float4 d = A.cdesc[i];
       double ph = theta * (double)d.y - (delta * (double)d.x + (double)d.z);
       if (PW > 1) ph -= (double)pw * (double)d.w;
-      if (i == Sh::LAST + 3 && B.lsb) ph += 0.5;           // the lower sideband keeps a - w b
+      if (i == Sh::LAST + 3 && B0.lsb) ph += 0.5;           // the lower sideband keeps a - w b
       sm.tab[fi][i] = exact_rotator(ph);
     }
   }
   if (NBITS == 2 && PW == 1)
-    for (int i = tid; i < 256; i += NT) sm.quad[i] = A.quad[B.levels * 256 + i];
-#pragma unroll
-  for (int i0 = 0; i0 < NIT; i0 += AHEAD) {
-    if (i0 > 0) {
-#pragma unroll
-      for (int i = 0; i < AHEAD; i++)
-        if (t + (i0 + i) * NTF < GROUPS) load_rows(t + (i0 + i) * NTF, lo[i], hi[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < AHEAD; i++)
-      if (t + (i0 + i) * NTF < GROUPS) store_quads(t + (i0 + i) * NTF, lo[i], hi[i]);
-  }
+    for (int i = tid; i < 256; i += NT) sm.quad[i] = A.quad[B0.levels * 256 + i];
+  stage(B0);
   __syncthreads();
   if (NBITS == 2 && PW > 1) {
     if (tid < 256 * Sh::NSUM) {
@@ -278,9 +295,43 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
   float2* const buf = sm.buf[fi];
   const float2* const tab = sm.tab[fi];
 
+  // ---- what two bands share: the last pass's twiddles and the rotation of
+  // channel PW (t + e M/16) + pw, this thread's phase (FP64, in turns) times
+  // E[e]; for one band both are formed where they are used, for registers
+  const float2* const cl = tab + Sh::LAST;
+  constexpr int NW = RL == 16 ? 4 : 6;
+  float2 w[NW], F, FE[8];
+  auto last_powers = [&] {
+#pragma unroll
+    for (int i = 0; i < NW; i++) w[i] = cmulx(A.base[i * NTF + t], cl[RL == 16 ? i : 1 + i / 2]);
+  };
+  auto channel_phase = [&] {
+    const float s = dead ? 0.0f : (NBITS == 8 ? A.scale * (float)(1.0 / 3.3) : A.scale);
+    F = exact_rotator(R.phase + R.theta * (double)(PW * t + pw));
+    F = make_float2(F.x * s, F.y * s);
+  };
+  if (Sh::TWO) {
+    last_powers();
+    channel_phase();
+#pragma unroll
+    for (int e = 0; e < 8; e++) FE[e] = cmulx(F, cl[4 + e]);
+  }
+
+#pragma unroll 1
+  for (int band = 0; band < (Sh::TWO ? nband : 1); band++) {
+  const DevBand& B = band ? B1 : B0;
+  // what a pass derives from the thread's number and its twiddles is formed
+  // anew for each band: kept over the loop it would not fit the registers
+  int tl = t;
+  if (Sh::TWO) asm volatile("" : "+v"(tl));
+  __builtin_assume(tl >= 0 && tl < NTF);
+  auto fresh = [](float2 w) {
+    if (Sh::TWO) asm volatile("" : "+v"(w.x), "+v"(w.y));
+    return w;
+  };
   // ---- pass 1: decode, radix R1 (this thread's 16 of the R1 outputs)
   {
-    const int p = t / J1, j = t % J1;
+    const int p = tl / J1, j = tl % J1;
     const float2* c = tab + p * Sh::CP;
     Tw16 w;
     w.w8 = c[0]; w.w4 = c[1]; w.w2 = c[2]; w.w2h = c[3]; w.w1 = c[4]; w.w1a = c[5]; w.w1b = c[6]; w.w1c = c[7];
@@ -405,10 +456,13 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
     }
   }
 
+  sync();
+  const bool more = band + 1 < nband;
+  if (Sh::TWO && more && t < GROUPS) store_quads(B1, t, lo1, hi1);   // every quad of this band has been read
+
   // ---- middle pass: radix 16 from R1 to 16 R1 bins
   if (MID) {
-    sync();
-    const int j = t % J2, k = t / J2;
+    const int j = tl % J2, k = tl / J2;
     Tw16 w;
     const float2* c = tab + Sh::MIDOFF + 8 * k;
     w.w8 = c[0]; w.w4 = c[1]; w.w2 = c[2]; w.w2h = c[3]; w.w1 = c[4]; w.w1a = c[5]; w.w1b = c[6]; w.w1c = c[7];
@@ -425,27 +479,21 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
 #pragma unroll
     for (int q = 0; q < 16; q++) op[R1 * q] = v[bitrev4(q)];
   }
+  if (!Sh::TWO) {
+    last_powers();
+    channel_phase();
+  }
+  if (MID) sync();
 
   // ---- last pass (radix RL), the sideband's half; fractional-sample rotation
-  float2 w[RL == 16 ? 4 : 6];
-#pragma unroll
-  for (int i = 0; i < (RL == 16 ? 4 : 6); i++) w[i] = A.base[i * NTF + t];
-  // channel PW (t + e M/16) + pw: this thread's phase (FP64, in turns) times E[e]
-  float2 F;
-  {
-    const float s = dead ? 0.0f : (NBITS == 8 ? A.scale * (float)(1.0 / 3.3) : A.scale);
-    F = cmulx(exact_rotator(R.phase + R.theta * (double)(PW * t + pw)), make_float2(B.polre * s, B.polim * s));
-  }
-  sync();
   float2 x[8];                                             // bin t + e M/16
-  const float2* cl = tab + Sh::LAST;
   if (RL == 16) {
     Tw16 tw;
-    tw.w8 = cmulx(w[0], cl[0]); tw.w4 = cmulx(w[1], cl[1]); tw.w2 = cmulx(w[2], cl[2]); tw.w1 = cmulx(w[3], cl[3]);
+    tw.w8 = w[0]; tw.w4 = w[1]; tw.w2 = fresh(w[2]); tw.w1 = fresh(w[3]);
     tw16_multiples(tw);
     float2 v[16];
 #pragma unroll
-    for (int r = 0; r < 16; r++) v[r] = buf[r * (NL + LPAD) + t];
+    for (int r = 0; r < 16; r++) v[r] = buf[r * (NL + LPAD) + tl];
     dft16_tw<true>(v, tw);
 #pragma unroll
     for (int e = 0; e < 8; e++) x[e] = v[bitrev4(e)];
@@ -454,26 +502,33 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
     for (int u = 0; u < 2; u++) {
       float2 v[8];
 #pragma unroll
-      for (int r = 0; r < 8; r++) v[r] = buf[r * (NL + LPAD) + t + u * NTF];
-      dft8_tw<true>(v, cmulx(w[u], cl[1]), cmulx(w[2 + u], cl[2]), cmulx(w[4 + u], cl[3]));
+      for (int r = 0; r < 8; r++) v[r] = buf[r * (NL + LPAD) + tl + u * NTF];
+      dft8_tw<true>(v, w[u], w[2 + u], fresh(w[4 + u]));
 #pragma unroll
       for (int q = 0; q < 4; q++) x[u + 2 * q] = v[bitrev3(q)];
     }
   }
-  if (!mine) return;
-  const float2* E = tab + Sh::LAST + 4;
-  const long long c0 = cidx(PW * t + pw, A.gstride), cstep = (PW * NTF / 16) * A.gstride;
-  auto store = [&](auto out) {
+  if (Sh::TWO && more) sync();                             // the buffer has been read
+  if (mine) {
+    const long long outbase = B.specoff + (long long)cb * A.bstride;
+    const long long c0 = cidx(PW * tl + pw, A.gstride), cstep = (PW * NTF / 16) * A.gstride;
+    const bool turned = B.polre != 1.0f || B.polim != 0.0f;
+    auto store = [&](auto out) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const long long at = NTF % 16 == 0 ? c0 + e * cstep : cidx(t + e * NTF, A.gstride);
-      put_spec(out, at, PW * (t + e * NTF) + pw, cmulx(x[e], cmulx(F, E[e])));
-    }
-  };
-  if (A.prec == FXG_XMAC_FP32) store((float2*)A.spectra + outbase);
-  else if (A.prec == FXG_XMAC_FP16) store((__half2*)A.spectra + outbase);
-  else if (A.prec == FXG_XMAC_FP8) store(Fp8Out{(unsigned short*)A.spectra + outbase, A.cexp + (long long)gband * C});
-  else store((__hip_bfloat162*)A.spectra + outbase);
+      for (int e = 0; e < 8; e++) {
+        const long long at = NTF % 16 == 0 ? c0 + e * cstep : cidx(tl + e * NTF, A.gstride);
+        float2 y = cmulx(x[e], Sh::TWO ? FE[e] : cmulx(F, cl[4 + e]));
+        if (turned) y = cmulx(y, make_float2(B.polre, B.polim));
+        put_spec(out, at, PW * (tl + e * NTF) + pw, y);
+      }
+    };
+    if (A.prec == FXG_XMAC_FP32) store((float2*)A.spectra + outbase);
+    else if (A.prec == FXG_XMAC_FP16) store((__half2*)A.spectra + outbase);
+    else if (A.prec == FXG_XMAC_FP8)
+      store(Fp8Out{(unsigned short*)A.spectra + outbase, A.cexp + (long long)(band ? pair.y : pair.x) * C});
+    else store((__hip_bfloat162*)A.spectra + outbase);
+  }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -523,6 +578,11 @@ static void fill_tables(std::vector<float4>* cdesc, std::vector<float2>* base) {
     }
 }
 
+// Two bands to a workgroup (8192 points 25.9 -> 25.2 ms, 2048 points 2.80 ->
+// 2.40) where that leaves several times what the chip holds at once, two to
+// seven workgroups a CU; below it one each, for the latency of a small call
+constexpr long long kPairWorkgroups = 4096;
+
 #define FX_LENGTHS(X) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192) X(16384) \
   X(32768) X(65536)
 
@@ -540,14 +600,18 @@ void fstage_quad_levels(const float* lut, float4* out) {
     out[b] = make_float4(lut[b & 3], lut[(b >> 2) & 3], lut[(b >> 4) & 3], lut[(b >> 6) & 3]);
 }
 
-hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream) {
+hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, const BandLists& l, int nblocks,
+                             hipStream_t stream) {
   if (nbits != 2 && nbits != 8) return hipErrorInvalidValue;
   FStageArgs b = a;
   b.nchunk = nblocks;
   switch (L) {
 #define X(Lv)                                                                                                       \
     case Lv: {                                                                                                      \
-      const dim3 grid((unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8 * FsShape<Lv>::PW), nbands); \
+      const unsigned gx = (unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8 * FsShape<Lv>::PW); \
+      const bool two = FsShape<Lv>::TWO && (long long)gx * l.npairs >= kPairWorkgroups;                             \
+      b.pairs = two ? l.pairs : l.singles;                                                                          \
+      const dim3 grid(gx, two ? l.npairs : l.nsingles);                                                             \
       if (nbits == 2) hipLaunchKernelGGL((k_fstage_lin<Lv, 2>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);         \
       else hipLaunchKernelGGL((k_fstage_lin<Lv, 8>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);                    \
       break;                                                                                                        \

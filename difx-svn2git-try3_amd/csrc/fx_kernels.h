@@ -54,6 +54,12 @@ struct FStageArgs {
   const float2* base;         // last-pass twiddles at d = 0, per thread
   const float4* quad;         // levels of four 2-bit samples by their byte: VDIF, Mark5B
   int nchunk;                 // blocks of the launch
+  const int2* pairs;          // global bands of each grid row: two of one rotation, or one (y < 0)
+};
+// the same bands for launch_fstage_lin, in pairs of one rotation and one by one
+struct BandLists {
+  const int2 *pairs = nullptr, *singles = nullptr;
+  int npairs = 0, nsingles = 0;
 };
 
 struct XmacArgs {
@@ -149,7 +155,8 @@ hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const 
 hipError_t launch_fstage(int L, int nbits, int cplx, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
 // linear and post-F rotation of real samples; its tables for
 // one length, and the levels of four 2-bit samples by their byte (256 entries)
-hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
+hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, const BandLists& l, int nblocks,
+                             hipStream_t stream);
 bool fstage_lin_tables(int L, std::vector<float4>* cdesc, std::vector<float2>* base);
 void fstage_quad_levels(const float* lut, float4* out);
 hipError_t launch_unpack(const DevStation* st, const DevStationSub* ss, const int2* ftab, const float* lut8,
