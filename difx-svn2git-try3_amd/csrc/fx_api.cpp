@@ -112,7 +112,7 @@ struct fxg_job {
   DBuf d_fblank, d_pbw;           // INTERLACEDVDIF: per-frame band blanking, per-(block, band) weights
   std::vector<long long> pbw_off; // per datastream: offset of its weights in d_pbw (-1: none)
   // per-subint
-  DBuf d_ss, d_flags, d_ftab, d_blocks, d_weights, d_results, d_ct;
+  DBuf d_ss, d_flags, d_ftab, d_blocks, d_bw, d_weights, d_results, d_ct;
   DBuf d_rotgroups, d_rots;       // rotations of the bands, and of each block (k_prologue)
   DBuf d_pairs;                   // band lists of that F stage
   BandLists lists2, lists8;       // its 2-bit and 8-bit bands
@@ -546,7 +546,7 @@ int fxg_unpack_noalloc(fxg_ctx* c, const fxg_datastream* ds, const uint8_t* data
 static void job_free(fxg_job* j) {
   DBuf* bufs[] = {&j->d_st, &j->d_bands, &j->d_segs, &j->d_wterms, &j->d_fblank, &j->d_pbw, &j->d_inoff, &j->d_tw,
                   &j->d_lut8,
-                  &j->d_ss, &j->d_flags, &j->d_ftab, &j->d_blocks, &j->d_weights, &j->d_results,
+                  &j->d_ss, &j->d_flags, &j->d_ftab, &j->d_blocks, &j->d_bw, &j->d_weights, &j->d_results,
                   &j->d_spec, &j->d_V, &j->d_ct, &j->d_bandlist, &j->d_iota, &j->d_zero, &j->d_z, &j->d_rtab,
                   &j->d_pcal, &j->d_pcalaux, &j->d_pcaltone, &j->d_pcalpart, &j->d_vpart, &j->d_cexp,
                   &j->d_eoff, &j->d_kurt, &j->d_kurtout, &j->d_kurtnz, &j->d_rotgroups, &j->d_rots, &j->d_cdesc,
@@ -688,6 +688,7 @@ int fxg_job_create(fxg_ctx* c, const fxg_job_desc* desc, fxg_job** out) {
       (rc = j->d_inoff.ensure(sizeof(long long) * std::max<size_t>(1, inoff.size()))) ||
       (rc = j->d_tw.ensure(sizeof(float2) * tw.size())) ||
       (rc = j->d_blocks.ensure(sizeof(DevBlock) * (size_t)P.nds * desc->blockspersend)) ||
+      (rc = j->d_bw.ensure(sizeof(float) * (size_t)P.nds * desc->blockspersend)) ||
       (rc = j->d_weights.ensure(sizeof(float) * wt.size())) ||
       (rc = j->d_results.ensure(sizeof(float) * 2 * (size_t)std::max<long long>(1, P.info.result_length))) ||
       (rc = j->d_spec.ensure(specbytes)) ||
@@ -1102,7 +1103,7 @@ static int launch_front(fxg_job* j, const LaunchShape& sh, hipStream_t s) {
   if ((rc = j->ev_end())) return rc;
   if ((rc = j->ev_begin(FXG_STAGE_PROLOGUE))) return rc;
   HIPCHK(launch_prologue(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_flags.as<int>(),
-                         j->d_ftab.as<int2>(), j->desc.blockspersend, j->d_blocks.as<DevBlock>(), P.nds,
+                         j->d_ftab.as<int2>(), j->desc.blockspersend, j->d_blocks.as<DevBlock>(), j->d_bw.as<float>(), P.nds,
                          j->d_rotgroups.as<DevRotGroup>(), j->fstage_lin ? j->d_rots.as<DevRot>() : nullptr, s));
   if ((rc = j->ev_end())) return rc;
   return 0;
@@ -1275,7 +1276,7 @@ static int launch_back(fxg_job* j, float* dres, hipStream_t s) {
     if ((rc = j->ev_end())) return rc;
   }
   if ((rc = j->ev_begin(FXG_STAGE_WEIGHTS))) return rc;
-  HIPCHK(launch_weights(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_blocks.as<DevBlock>(), nblocks,
+  HIPCHK(launch_weights(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_bw.as<float>(), nblocks,
                         j->d_wterms.as<DevWTerm>(), (int)P.wterms.size(), j->d_weights.as<float>(), s));
   if ((rc = j->ev_end())) return rc;
   // the slot is zeroed before accumulation (core.cpp:319) by a kernel, so

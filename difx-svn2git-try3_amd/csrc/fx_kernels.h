@@ -149,8 +149,8 @@ struct CornerTurn {
 hipError_t launch_cornerturn(const DevStation* st, const DevStationSub* ss, unsigned char* ct, int nst,
                              const CornerTurn& c, hipStream_t stream);
 hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const int* flags,
-                           const int2* ftab, int nblocks, DevBlock* out, int nst, const DevRotGroup* groups,
-                           DevRot* rots, hipStream_t stream);
+                           const int2* ftab, int nblocks, DevBlock* out, float* bw, int nst,
+                           const DevRotGroup* groups, DevRot* rots, hipStream_t stream);
 // cplx: complex samples (L = nchan, every output of the transform kept)
 hipError_t launch_fstage(int L, int nbits, int cplx, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
 // linear and post-F rotation of real samples; its tables for

@@ -779,7 +779,7 @@ int64_t plan_device_bytes(const Plan& p, const fxg_job_desc* d) {
   long long spec = (long long)p.nbands_total * p.C * p.chunk_blocks * spectrum_bytes(d->xmac_precision);
   if (d->xmac_precision == FXG_XMAC_FP8) spec += (long long)p.nbands_total * p.C;   // the scale exponents
   long long v = p.vsize * 8;
-  long long blocks = ((long long)p.nds * (long long)sizeof(DevBlock) + (long long)p.rots.size() * (long long)sizeof(DevRot)) *
+  long long blocks = ((long long)p.nds * (long long)(sizeof(DevBlock) + sizeof(float)) + (long long)p.rots.size() * (long long)sizeof(DevRot)) *
                      d->blockspersend;
   long long res = p.info.result_length * 8;
   long long tables = (long long)p.segs.size() * sizeof(DevSeg) + p.bands.size() * sizeof(DevBand) + (1 << 20);

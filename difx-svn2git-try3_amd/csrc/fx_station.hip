@@ -332,8 +332,8 @@ __device__ __forceinline__ DevRot block_rotation(const DevStation& S, const DevR
 
 __global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSub* __restrict__ ss,
                            const int* __restrict__ flags, const int2* __restrict__ ftab, int nblocks,
-                           DevBlock* __restrict__ out, const DevRotGroup* __restrict__ groups,
-                           DevRot* __restrict__ rots) {
+                           DevBlock* __restrict__ out, float* __restrict__ bw,
+                           const DevRotGroup* __restrict__ groups, DevRot* __restrict__ rots) {
   const int s = blockIdx.y;
   const int index = blockIdx.x * blockDim.x + threadIdx.x;
   if (index >= nblocks) return;
@@ -341,6 +341,7 @@ __global__ void k_prologue(const DevStation* __restrict__ st, const DevStationSu
   const DevStationSub Q = ss[s];
   const DevBlock g = block_geometry(S, Q, flags, ftab, index);
   out[(long long)s * nblocks + index] = g;
+  bw[(long long)s * nblocks + index] = g.status != 0 ? -1.0f : g.weight;
   if (rots)
     for (int k = 0; k < S.nrot; k++) rots[(long long)(S.rot0 + k) * nblocks + index] = block_rotation(S, groups[S.rot0 + k], g);
 }
@@ -1490,10 +1491,10 @@ hipError_t launch_frames(const DevStation* st, const DevStationSub* ss, int2* ft
 }
 
 hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const int* flags,
-                           const int2* ftab, int nblocks, DevBlock* out, int nst, const DevRotGroup* groups,
-                           DevRot* rots, hipStream_t stream) {
+                           const int2* ftab, int nblocks, DevBlock* out, float* bw, int nst,
+                           const DevRotGroup* groups, DevRot* rots, hipStream_t stream) {
   dim3 grid((unsigned)((nblocks + 127) / 128), nst);
-  hipLaunchKernelGGL(k_prologue, grid, dim3(128), 0, stream, st, ss, flags, ftab, nblocks, out, groups, rots);
+  hipLaunchKernelGGL(k_prologue, grid, dim3(128), 0, stream, st, ss, flags, ftab, nblocks, out, bw, groups, rots);
   return hipGetLastError();
 }
 

@@ -112,47 +112,110 @@ __global__ __launch_bounds__(576) void k_xmac_f32(XmacArgs A) {
 // recorded band's weight on INTERLACEDVDIF datastreams, else the block's
 // data weight
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float band_weight(const DevStation* st, const DevStationSub* ss, const DevBlock* blocks,
-                                             int nblocks, int d, int b, int k) {
-  const DevBlock& g = blocks[(long long)d * nblocks + k];
-  if (g.status != 0) return 0.0f;
-  if (b < 0) return g.weight;
-  return ss[d].pbw[(long long)k * st[d].nchan + b];
+// acc + 1 + ... + 1 (n ones) in FP32, each addition rounded.  One addition of m
+// of them rounds the same where acc is whole, or at least m, and the sum stays
+// below 2^22: then at most one binade is crossed, and an integer added after its
+// rounding moves no tie, a spacing there being a quarter or less.
+__device__ __forceinline__ float add_ones(float acc, int n) {
+  while (n > 0) {
+    int m = 1;
+    if (acc + (float)n < 4194304.0f) m = acc == truncf(acc) ? n : min(n, max(1, (int)acc));
+    acc += (float)m;
+    n -= m;
+  }
+  return acc;
 }
 
+// One workgroup per entry.  The sums are FP32 in block order, a serial chain
+// (the reference's rounding), but nearly every term is 0 or 1: all wavefronts
+// sort 4096 terms into masks by 64, and the first adds the ones of all of them
+// at once, or, where there are other terms, goes through them in order; the
+// next terms load meanwhile.  The weights come from their own array: out of the
+// 80-byte block records the lines alone took a CU 100 us.  10 entries of 62500
+// blocks: 474 us one addition at a time -> 42.
 __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ st,
                                                  const DevStationSub* __restrict__ ss,
-                                                 const DevBlock* __restrict__ blocks, int nblocks,
+                                                 const float* __restrict__ bw, int nblocks,
                                                  const DevWTerm* __restrict__ terms, int nterms,
                                                  float* __restrict__ wout) {
-  // one workgroup per entry: the per-block terms are gathered in parallel
-  // into LDS and one lane adds them in block order
-  constexpr int CH = 4096;
-  __shared__ float4 term4[CH / 4];
-  float* term = (float*)term4;
+  constexpr int CH = 4096, PER = CH / 256;
+  __shared__ float term[CH];
+  __shared__ unsigned long long ones[CH / 64], odd[CH / 64];
   const int i = blockIdx.x;
   if (i >= nterms) return;
   const DevWTerm T = terms[i];
+  const int lane = threadIdx.x & 63;
+  float v[PER];
+  // the weights of one side: bw, negative where a block was not processed, and
+  // the band's own in its place
+  auto side = [&](int d, int b, int t0, float (&w)[PER]) {
+    const float* const src = bw + (long long)d * nblocks;
+#pragma unroll
+    for (int q = 0; q < PER; q++) w[q] = src[min(t0 + q * 256 + (int)threadIdx.x, nblocks - 1)];
+    if (b >= 0) {
+      const float* const own = ss[d].pbw + b;
+      const int nchan = st[d].nchan;
+#pragma unroll
+      for (int q = 0; q < PER; q++)
+        if (w[q] >= 0.0f) w[q] = own[(long long)min(t0 + q * 256 + (int)threadIdx.x, nblocks - 1) * nchan];
+    }
+#pragma unroll
+    for (int q = 0; q < PER; q++) w[q] = fmaxf(w[q], 0.0f);
+  };
+  auto load = [&](int t0) {
+    side(T.d1, T.b1, t0, v);
+    if (T.d2 >= 0) {
+      float w[PER];
+      side(T.d2, T.b2, t0, w);
+#pragma unroll
+      for (int q = 0; q < PER; q++) v[q] *= w[q];
+    }
+  };
   float acc = 0.0f;
+  if (nblocks > 0) load(0);
   for (int t0 = 0; t0 < nblocks; t0 += CH) {
-    const int n = min(CH, nblocks - t0);
-    for (int k = threadIdx.x; k < CH; k += blockDim.x) {
-      float v = 0.0f;
-      if (k < n) {
-        const float w1 = band_weight(st, ss, blocks, nblocks, T.d1, T.b1, t0 + k);
-        v = T.d2 >= 0 ? w1 * band_weight(st, ss, blocks, nblocks, T.d2, T.b2, t0 + k) : w1;
-      }
-      term[k] = v;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      const int k = q * 256 + threadIdx.x;
+      const float x = t0 + k < nblocks ? v[q] : 0.0f;
+      term[k] = x;
+      const unsigned long long o = __ballot(x == 1.0f), z = __ballot(x != 0.0f) & ~o;
+      if (lane == 0) { ones[k >> 6] = o; odd[k >> 6] = z; }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int k = 0; k < (n + 3) / 4; k++) {
-        const float4 q = term4[k];
-        acc += q.x;
-        acc += q.y;
-        acc += q.z;
-        acc += q.w;
+    if (t0 + CH < nblocks) load(t0 + CH);
+    if (threadIdx.x < 64) {
+      int n = __popcll(ones[lane]);
+      unsigned long long mixed = __ballot(odd[lane] != 0ull);
+      // the ones before group g are added together, then its terms in order
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int u = __shfl_up(n, d);
+        if (lane >= d) n += u;
       }
+      int done = 0;
+      while (mixed) {
+        const int g = __builtin_ctzll(mixed);
+        mixed &= mixed - 1ull;
+        unsigned long long left = ones[g], rest = odd[g];
+        acc = add_ones(acc, __shfl(n, g) - __popcll(left) - done);
+        done = __shfl(n, g);
+        if (__popcll(rest) > 16) {
+#pragma unroll 16
+          for (int j = 0; j < 64; j++) acc += term[64 * g + j];
+          continue;
+        }
+        while (rest) {
+          const int b = __builtin_ctzll(rest);
+          const unsigned long long below = (1ull << b) - 1ull;
+          acc = add_ones(acc, __popcll(left & below));
+          acc += term[64 * g + b];
+          left &= ~below;
+          rest &= rest - 1ull;
+        }
+        acc = add_ones(acc, __popcll(left));
+      }
+      acc = add_ones(acc, __shfl(n, 63) - done);
     }
     __syncthreads();
   }
@@ -265,10 +328,10 @@ hipError_t launch_zero(float* p, long long n, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t launch_weights(const DevStation* st, const DevStationSub* ss, const DevBlock* blocks, int nblocks,
+hipError_t launch_weights(const DevStation* st, const DevStationSub* ss, const float* bw, int nblocks,
                           const DevWTerm* terms, int nterms, float* w, hipStream_t stream) {
   if (nterms == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_weights, dim3(nterms), dim3(256), 0, stream, st, ss, blocks, nblocks, terms, nterms, w);
+  hipLaunchKernelGGL(k_weights, dim3(nterms), dim3(256), 0, stream, st, ss, bw, nblocks, terms, nterms, w);
   return hipGetLastError();
 }
 
