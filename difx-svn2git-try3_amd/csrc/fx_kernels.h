@@ -180,7 +180,7 @@ hipError_t launch_xmac_mfma_f32(const XmacArgs& a, const void* zero16, hipStream
 // V[i] (+)= sum over splits of P[s][i], i < n, in split order
 hipError_t launch_xmac_reduce(const float2* P, int nsplit, long long vsplit, float2* V, long long n, int accumulate,
                               hipStream_t stream);
-hipError_t launch_weights(const DevStation* st, const DevStationSub* ss, const DevBlock* blocks, int nblocks,
+hipError_t launch_weights(const DevStation* st, const DevStationSub* ss, const float* bw, int nblocks,
                           const DevWTerm* terms, int nterms, float* w, hipStream_t stream);
 // few / many: some band has at most kPcalFewBins bins / more
 hipError_t launch_pcal(const PcalArgs& a, int npcal, bool few, bool many, hipStream_t stream);
