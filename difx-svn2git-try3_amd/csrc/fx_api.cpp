@@ -1279,9 +1279,6 @@ static int launch_back(fxg_job* j, float* dres, hipStream_t s) {
   HIPCHK(launch_weights(j->d_st.as<DevStation>(), j->d_ss.as<DevStationSub>(), j->d_bw.as<float>(), nblocks,
                         j->d_wterms.as<DevWTerm>(), (int)P.wterms.size(), j->d_weights.as<float>(), s));
   if ((rc = j->ev_end())) return rc;
-  // the slot is zeroed before accumulation (core.cpp:319) by a kernel, so
-  // that the sequence can live in a graph
-  HIPCHK(launch_zero(dres, 2 * P.info.result_length, s));
   float vscale = 1.0f / (j->scale * j->scale);
   if ((rc = j->ev_begin(FXG_STAGE_SCATTER))) return rc;
   HIPCHK(launch_scatter(j->d_segs.as<DevSeg>(), (int)P.segs.size(), P.maxseglen, j->d_V.as<float2>(),

@@ -106,9 +106,9 @@ struct DevWTerm {
 };
 
 // ---- result scatter segments -----------------------------------------------
-enum SegKind { SEG_VIS = 0, SEG_FLOATS = 1 };
+enum SegKind { SEG_VIS = 0, SEG_FLOATS = 1, SEG_ZERO = 2 };   // SEG_ZERO: nchan floats no other segment writes
 struct DevSeg {
-  long long resoff;     // cf32 offset (SEG_VIS) or float offset (SEG_FLOATS)
+  long long resoff;     // cf32 offset (SEG_VIS) or float offset (SEG_FLOATS, SEG_ZERO)
   long long voff;       // element offset into V (SEG_VIS) or into the weight table
   int kind, nchan;
   int conj;             // take conj(V[b][a]) instead of V[a][b]

@@ -739,6 +739,28 @@ int build_plan(const fxg_job_desc* d, Plan* p, std::string* err) {
       REQUIRE(x.in_station.size() <= 64 && x.nchan % 16 == 0, FXG_EUNSUPPORTED,
               "fp8 cross-multiply needs at most 64 inputs and a multiple of 16 channels per frequency");
   P.info.result_length = at;
+  // the floats of the slot that no segment writes are cleared with them
+  // (core.cpp:319 zeroes the whole slot)
+  {
+    std::vector<std::pair<long long, long long>> cover;
+    cover.reserve(P.segs.size() + 1);
+    for (const DevSeg& g : P.segs) {
+      if (g.kind == SEG_VIS) cover.emplace_back(2 * g.resoff, 2 * (g.resoff + g.nchan));
+      else cover.emplace_back(g.resoff, g.resoff + 1);
+    }
+    std::sort(cover.begin(), cover.end());
+    cover.emplace_back(2 * at, 2 * at);
+    P.maxseglen = std::max(P.maxseglen, 1024);
+    long long done = 0;
+    for (const auto& c : cover) {
+      for (long long f = done; f < c.first; f += P.maxseglen) {
+        DevSeg z{};
+        z.kind = SEG_ZERO; z.resoff = f; z.nchan = (int)std::min<long long>(P.maxseglen, c.first - f);
+        P.segs.push_back(z);
+      }
+      done = std::max(done, c.second);
+    }
+  }
   P.info.arraystridelen = P.arraystride[0];
   P.info.xmacstridelen = P.xmacstride;
   P.info.rotatestridelen = P.rotatestride;

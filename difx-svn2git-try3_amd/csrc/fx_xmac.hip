@@ -224,7 +224,8 @@ __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // scatter: result[seg.resoff + c] = mean of V[seg.voff + c avg + i], i < avg
-// (conjugated if flagged), scaled by vscale; float segments copy one weight
+// (conjugated if flagged), scaled by vscale; float segments copy one weight;
+// zero segments clear what nothing else writes
 // ---------------------------------------------------------------------------
 constexpr int kScatterPer = 4;   // channels per thread (their loads in flight together)
 
@@ -237,6 +238,12 @@ __global__ __launch_bounds__(256) void k_scatter(const DevSeg* __restrict__ segs
   const int cb = blockIdx.x * (256 * kScatterPer) + threadIdx.x;
   if (g.kind == SEG_FLOATS) {
     if (cb == 0) res[g.resoff] = w[g.voff];
+    return;
+  }
+  if (g.kind == SEG_ZERO) {
+#pragma unroll
+    for (int q = 0; q < kScatterPer; q++)
+      if (cb + q * 256 < g.nchan) res[g.resoff + cb + q * 256] = 0.0f;
     return;
   }
   if (cb >= g.nchan) return;

@@ -1,10 +1,13 @@
 """The sums behind the spectra: weights over thousands of blocks (k_weights
-adds runs of ones at once).  The weights are the oracle's bit for bit (the
+adds runs of ones at once), results that land in a caller's device buffer with
+nothing left of what it held.  The weights are the oracle's bit for bit (the
 same FP32 terms in block order)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from fxcorr import JobSpec
+from fxcorr import JobSpec, check
 from fxsynth import make_subint
 from fxtestlib import GpuJob, oracle_results, plan_info, region_slices
 
@@ -34,4 +37,28 @@ def test_long_weight_sums(gpu, oracle, nblocks, payload, every):
     xend, a0, a1 = region_slices(oracle, job, plan_info(oracle, "orc_", job))
     for r in (slice(xend, a0), slice(a1, None)):
         assert np.array_equal(got[r].view(np.uint32), ref[r].view(np.uint32))
+    g.close()
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(crosspol=False), dict(zoom=[(1, 64, 32)]), dict(pcal_interval_mhz=1.0)],
+                         ids=["full", "parallel", "zoom", "pcal"])
+def test_results_replace_what_the_buffer_held(gpu, oracle, kw):
+    lib, ctx = gpu
+    spec = JobSpec(nstations=3, nsubbands=2, npol=2, bw_mhz=16.0, nchan=128, blockspersend=20, **kw)
+    job, keep = spec.build()
+    sd = data(spec)
+    ref = oracle_results(oracle, job, sd).view(np.float32)
+    g = GpuJob(lib, ctx, job)
+    held = np.full(ref.size, np.nan, dtype=np.float32)
+    p = C.c_void_p()
+    check(lib, lib.fxg_device_alloc(ctx, held.nbytes, C.byref(p)), "alloc")
+    check(lib, lib.fxg_memcpy_h2d(ctx, p, held.ctypes.data, held.nbytes), "h2d")
+    sub = sd.subint_desc()
+    st, keep2 = sd.station_inputs()
+    check(lib, lib.fxg_subint_process(g.h, C.byref(sub), st, 0, p, 1), "process")
+    check(lib, lib.fxg_memcpy_d2h(ctx, held.ctypes.data, p, held.nbytes), "d2h")
+    lib.fxg_device_free(ctx, p)
+    assert np.all(np.isfinite(held))
+    assert not np.any(held[ref == 0.0])
+    assert np.array_equal(held, g.process(sd).view(np.float32))
     g.close()
