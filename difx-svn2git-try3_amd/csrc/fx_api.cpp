@@ -1264,7 +1264,7 @@ static int launch_back(fxg_job* j, float* dres, hipStream_t s) {
       } else {
         HIPCHK(launch_xmac_f32(xa, prec, s));
       }
-      if (rows > 1) HIPCHK(launch_xmac_reduce(j->d_vpart.as<float2>(), rows, vsz, V, vsz, c0 > 0, s));
+      if (rows > 1) HIPCHK(launch_xmac_reduce(j->d_vpart.as<float2>(), rows, vsz, V, xa.nin, xa.nchan, c0 > 0, s));
       if ((rc = j->ev_end())) return rc;
     }
     j->tap_chunk0 = c0;

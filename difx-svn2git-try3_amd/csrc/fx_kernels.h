@@ -177,9 +177,9 @@ hipError_t launch_xmac_mfma_streaming(const XmacArgs& a, int prec, const void* z
 // input offsets and block stride
 bool xmac_mfma_f32_ok(const XmacArgs& a, const long long* in_off_host);
 hipError_t launch_xmac_mfma_f32(const XmacArgs& a, const void* zero16, hipStream_t stream);
-// V[i] (+)= sum over splits of P[s][i], i < n, in split order
-hipError_t launch_xmac_reduce(const float2* P, int nsplit, long long vsplit, float2* V, long long n, int accumulate,
-                              hipStream_t stream);
+// V (+)= sum over splits of P[s], in split order, V [nin][nin][nchan]
+hipError_t launch_xmac_reduce(const float2* P, int nsplit, long long vsplit, float2* V, int nin, int nchan,
+                              int accumulate, hipStream_t stream);
 hipError_t launch_weights(const DevStation* st, const DevStationSub* ss, const float* bw, int nblocks,
                           const DevWTerm* terms, int nterms, float* w, hipStream_t stream);
 // few / many: some band has at most kPcalFewBins bins / more

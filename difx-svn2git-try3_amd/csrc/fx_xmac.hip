@@ -295,26 +295,37 @@ hipError_t launch_xmac_f32(const XmacArgs& a, int prec, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// V[i] (+)= sum_s P[s*vsplit + i]: the block-split partial sums, added in
-// split order so that the result does not depend on scheduling
+// V (+)= sum_s P[s*vsplit + .], V [nin][nin][nchan]: the partial sums
+// of block ranges, of the input pairs a <= b that are read, added in
+// split order so that the result does not depend on scheduling, eight loads in
+// flight.  14 inputs, 256 channels, 32 rows 33 us -> 11.
 __global__ __launch_bounds__(256) void k_xmac_reduce(const float2* __restrict__ P, int nsplit, long long vsplit,
-                                                     float2* __restrict__ V, long long n, int accumulate) {
+                                                     float2* __restrict__ V, unsigned nin, unsigned nchan, long long n,
+                                                     int accumulate) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
+  const unsigned q = (unsigned)(i / nchan);
+  if (q / nin > q % nin) return;
   float2 acc = accumulate ? V[i] : make_float2(0.f, 0.f);
-  for (int s = 0; s < nsplit; s++) {
-    const float2 p = P[(long long)s * vsplit + i];
-    acc.x += p.x;
-    acc.y += p.y;
+  for (int s0 = 0; s0 < nsplit; s0 += 8) {
+    float2 p[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) p[s] = s0 + s < nsplit ? P[(long long)(s0 + s) * vsplit + i] : make_float2(0.f, 0.f);
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      acc.x += p[s].x;
+      acc.y += p[s].y;
+    }
   }
   V[i] = acc;
 }
 
-hipError_t launch_xmac_reduce(const float2* P, int nsplit, long long vsplit, float2* V, long long n, int accumulate,
-                              hipStream_t stream) {
+hipError_t launch_xmac_reduce(const float2* P, int nsplit, long long vsplit, float2* V, int nin, int nchan,
+                              int accumulate, hipStream_t stream) {
+  const long long n = (long long)nin * nin * nchan;
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_xmac_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, P, nsplit, vsplit, V, n,
-                     accumulate);
+  hipLaunchKernelGGL(k_xmac_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, P, nsplit, vsplit, V,
+                     (unsigned)nin, (unsigned)nchan, n, accumulate);
   return hipGetLastError();
 }
 
