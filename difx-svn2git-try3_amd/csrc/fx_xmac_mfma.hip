@@ -173,6 +173,54 @@ struct DlTiles {
   }
 };
 
+// LDS written by the workgroup can be read by all of it (loads and stores to
+// memory may stay in flight)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// V of a workgroup's 32x32 tiles, one channel to a wavefront in the
+// accumulators: 256 input pairs at a time change through LDS (two buffers in
+// turn) into lines of CG channels, so that a store instruction fills whole
+// lines instead of 8 bytes in each of 64.  Pairs a > b are not kept.
+template <int CG, class TL, class ACC, class IN>
+__device__ __forceinline__ void store_tiles32(float2* buf, const ACC (&re)[TL::N], const ACC (&im)[TL::N], IN input_of,
+                                              float2* V, int nin, int nchan, int c0, int accumulate) {
+  constexpr int PS = CG + 1;
+  const int tid = threadIdx.x, w = tid >> 6, half = (tid & 63) >> 5, row = tid & 31;
+  const int ch = tid % CG, p0 = tid / CG;
+#pragma unroll
+  for (int k = 0; k < TL::N; k++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      float2* const B = buf + (g & 1) * 256 * PS;
+      // pair p0 + 64 i: rows a + 2 i of column b
+      const int a = input_of(32 * TL::I(k) + 8 * g + (p0 >> 5)), b = input_of(32 * TL::J(k) + (p0 & 31));
+      const int last = b < nin ? b : -1;
+      float2* const ptr = V + ((long long)a * nin + b) * nchan + c0 + ch;
+      const long long step = 2LL * nin * nchan;
+      float2 o[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        o[i] = make_float2(0.0f, 0.0f);
+        if (accumulate && a + 2 * i <= last) o[i] = ptr[i * step];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        B[((4 * half + q) * 32 + row) * PS + w] = make_float2(re[k][4 * g + q], im[k][4 * g + q]);
+      lds_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (a + 2 * i <= last) {
+          float2 v = B[(p0 + 64 * i) * PS + ch];
+          if (accumulate) { v.x += o[i].x; v.y += o[i].y; }
+          ptr[i * step] = v;
+        }
+    }
+}
+
 template <int T, bool BF, bool CROSS>
 __global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_dl(XmacArgs A, const uint4* __restrict__ zero16) {
   static_assert(!CROSS || T == 4, "a cross workgroup holds two 64-input chunks");
@@ -283,23 +331,10 @@ __global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_dl(XmacArgs A,
     __builtin_amdgcn_s_waitcnt(WAITIMM);   // this wavefront's loads of stage sg + 1 have landed
     barrier();                             // everyone's have, and nobody still reads stage sg
   }
-  __builtin_amdgcn_s_waitcnt(0);           // the zero-filled stages past the end, before exit
-
-  const int c = c0 + w;
-  if (c >= A.nchan) return;
-#pragma unroll
-  for (int k = 0; k < NTILE; k++) {
-    const int b = input_of(32 * TL::J(k) + row);
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int a = input_of(32 * TL::I(k) + 8 * (r >> 2) + 4 * half + (r & 3));
-      if (a >= A.nin || b >= A.nin) continue;
-      float2* ptr = Vout + ((long long)a * A.nin + b) * A.nchan + c;
-      float2 v = make_float2(accR[k][r], accI[k][r]);
-      if (A.accumulate) { float2 o = *ptr; v.x += o.x; v.y += o.y; }
-      *ptr = v;
-    }
-  }
+  __builtin_amdgcn_s_waitcnt(0);           // the zero-filled stages past the end
+  barrier();                               // before the ring is reused
+  static_assert(NBUF * STAGE >= 2 * 2 * 256 * (CG + 1), "the ring holds the tiles on their way out");
+  store_tiles32<CG, TL>((float2*)lds, accR, accI, input_of, Vout, A.nin, A.nchan, c0, A.accumulate);
 }
 
 // ---------------------------------------------------------------------------
@@ -333,14 +368,18 @@ template <int N> __device__ __forceinline__ void wait_vm() {
 template <int T>
 __global__ __launch_bounds__(1024, T <= 2 ? 8 : 4) void k_xmac_f32_t16(XmacArgs A, const uint4* __restrict__ zero16) {
   constexpr int CG = 16;                 // channels (wavefronts) per workgroup
-  constexpr int TT = 8;                  // blocks per stage
-  constexpr int NBUF = T == 1 ? 4 : T == 3 ? 3 : 2;
+  constexpr int TT = T == 1 ? 8 : 4;     // blocks per stage
+  constexpr int RPI = 8 / TT;            // rows of a load instruction
+  constexpr int NBUF = T == 3 ? 5 : 4;
   constexpr int NTILE = T * (T + 1) / 2;
   constexpr int RBW = 2 * CG;            // dwords per (row, block)
-  constexpr int SDW = TT * RBW + 4;      // dwords per row per stage
-  constexpr int STAGE = 16 * T * SDW;
-  __shared__ __align__(16) unsigned lds[NBUF * STAGE];
-  static_assert(NBUF * STAGE >= CG * 16 * 17, "the ring holds the wavefronts' transposes");
+  constexpr int SDW = 8 * RBW + 4;       // dwords per load instruction: RPI rows of a stage, padded
+  constexpr int GPT = 16 / RPI;          // load instructions per 16 rows
+  constexpr int STAGE = GPT * T * SDW;
+  constexpr int LPW = (GPT * T + CG - 1) / CG;   // and per wavefront at most
+  constexpr int PS = CG + 1;             // float2 a pair on the way out
+  constexpr int OUT = 2 * 256 * PS * (NTILE > 1 ? 2 : 1);
+  __shared__ __align__(16) unsigned lds[NBUF * STAGE > OUT ? NBUF * STAGE : OUT];
 
   const char* spec = (const char*)A.spec;
   const int tid = threadIdx.x;
@@ -350,40 +389,41 @@ __global__ __launch_bounds__(1024, T <= 2 ? 8 : 4) void k_xmac_f32_t16(XmacArgs 
   const int grp = (nwg % 8 == 0) ? (bid % 8) * (nwg / 8) + bid / 8 : bid;   // XCD-aware groups
   const int c0 = grp * CG;
   const int row = l & 15, kk = l >> 4;
-  const int lt = l >> 3, lp = l & 7;                // load lane: block and 2-channel piece
+  // load lane: row of the instruction, block and 2-channel piece
+  const int lr = l / (8 * TT), lt = (l >> 3) % TT, lp = l & 7;
   const int sb0 = blockIdx.y * A.split_blocks;
   const int nb = min(A.nblocks - sb0, A.split_blocks);
   float2* const Vout = A.V + (long long)blockIdx.y * A.vsplit;
   const int in0 = 64 * blockIdx.z;                  // this chunk's first input
-  // the rows this wavefront loads: w, w + 16, ... (the valid ones come first)
+  // the RPI rows of each of this wavefront's loads, w, w + 16, ...; those with
+  // an input come first
   const int wu = __builtin_amdgcn_readfirstlane(w);
-  long long ioff[T];
+  long long ioff[LPW];
   int nv = 0;
 #pragma unroll
-  for (int u = 0; u < T; u++) {
-    const int a = in0 + 16 * u + wu;
-    ioff[u] = a < A.nin ? A.in_off[a] + c0 : 0;
-    if (a < A.nin) nv = u + 1;
+  for (int u = 0; u < LPW; u++) {
+    const int a = in0 + RPI * (CG * u + wu);
+    ioff[u] = a + lr < A.nin ? A.in_off[a + lr] + c0 : -1;
+    if (a < A.nin && CG * u + wu < GPT * T) nv = u + 1;
   }
   auto issue = [&](int stage, int buf) {
     const int t = stage * TT + lt;
 #pragma unroll
-    for (int u = 0; u < T; u++) {
+    for (int u = 0; u < LPW; u++) {
       if (u >= nv) break;
       const void* src = zero16;
-      if (t < nb) src = spec + 8 * (ioff[u] + (long long)(sb0 + t) * A.block_stride + 2 * lp);
+      if (ioff[u] >= 0 && t < nb) src = spec + 8 * (ioff[u] + (long long)(sb0 + t) * A.block_stride + 2 * lp);
       __builtin_amdgcn_global_load_lds(
-          src, (__attribute__((address_space(3))) void*)(lds + buf * STAGE + (16 * u + wu) * SDW), 16, 0, 0);
+          src, (__attribute__((address_space(3))) void*)(lds + buf * STAGE + (CG * u + wu) * SDW), 16, 0, 0);
     }
   };
   // all but the newest NBUF - 2 stages of this wavefront's loads have landed
   auto landed = [&] {
     if (nv == 1) wait_vm<(NBUF - 2) * 1>();
     else if (nv == 2) wait_vm<(NBUF - 2) * 2>();
-    else if (nv == 3) wait_vm<(NBUF - 2) * 3>();
-    else if (nv == 4) wait_vm<(NBUF - 2) * 4>();
     else wait_vm<0>();
   };
+  static_assert(LPW <= 2, "landed");
   auto barrier = [] {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -404,14 +444,14 @@ __global__ __launch_bounds__(1024, T <= 2 ? 8 : 4) void k_xmac_f32_t16(XmacArgs 
   int buf = 0;
   for (int sg = 0; sg < nstage; sg++) {
     issue(sg + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
-    const float* base = (const float*)(lds + buf * STAGE) + row * SDW + kk * RBW + 2 * w;
+    const float* base = (const float*)(lds + buf * STAGE) + row / RPI * SDW + (row % RPI * TT + kk) * RBW + 2 * w;
 #pragma unroll
     for (int ks = 0; ks < TT / 4; ks++) {
       float2 f[T];
       float n[T];
 #pragma unroll
       for (int I = 0; I < T; I++) {
-        f[I] = *(const float2*)(base + 16 * I * SDW + 4 * ks * RBW);
+        f[I] = *(const float2*)(base + GPT * I * SDW + 4 * ks * RBW);
         n[I] = -f[I].x;
       }
       int k = 0;
@@ -430,39 +470,40 @@ __global__ __launch_bounds__(1024, T <= 2 ? 8 : 4) void k_xmac_f32_t16(XmacArgs 
     buf = buf + 1 == NBUF ? 0 : buf + 1;
   }
   __builtin_amdgcn_s_waitcnt(0);         // the stages past the end have landed
-  barrier();                             // before the ring is reused for the transposes
+  barrier();                             // before the ring is reused
 
-  const int c = c0 + w;
-  float* const tr = (float*)lds + w * 16 * 17;
+  // tile by tile into lines of 16 channels, as store_tiles32
+  const int ch = tid & 15, p0 = tid >> 4;
   int k = 0;
 #pragma unroll
   for (int I = 0; I < T; I++)
 #pragma unroll
     for (int J = I; J < T; J++, k++) {
-      f32x4_t im = accI[k];
-      if (I == J) {
-        // Im V[a][b] = Q[a][b] - Q[b][a], within this wavefront
+      float2* const B = (float2*)lds + (k & 1) * 256 * PS;
+      // pair p0 + 64 i: rows a + 4 i of column b
+      const int a = in0 + 16 * I + (p0 >> 4), b = in0 + 16 * J + (p0 & 15);
+      const int last = b < A.nin ? b : -1;
+      float2* const ptr = Vout + ((long long)a * A.nin + b) * A.nchan + c0 + ch;
+      const long long step = 4LL * A.nin * A.nchan;
+      float2 o[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) tr[(4 * kk + r) * 17 + row] = im[r];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int r = 0; r < 4; r++) im[r] -= tr[row * 17 + 4 * kk + r];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int i = 0; i < 4; i++) {
+        o[i] = make_float2(0.0f, 0.0f);
+        if (A.accumulate && a + 4 * i <= last) o[i] = ptr[i * step];
       }
-      const int b = in0 + 16 * J + row;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int a = in0 + 16 * I + 4 * kk + r;
-        if (a >= A.nin || b >= A.nin || c >= A.nchan) continue;
-        float2* ptr = Vout + ((long long)a * A.nin + b) * A.nchan + c;
-        float2 v = make_float2(accR[k][r], im[r]);
-        if (A.accumulate) { float2 o = *ptr; v.x += o.x; v.y += o.y; }
-        *ptr = v;
-      }
+      for (int r = 0; r < 4; r++) B[((4 * kk + r) * 16 + row) * PS + w] = make_float2(accR[k][r], accI[k][r]);
+      lds_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (a + 4 * i <= last) {
+          const int p = p0 + 64 * i;
+          float2 v = B[p * PS + ch];
+          // Im V[a][b] = Q[a][b] - Q[b][a]
+          if (I == J) v.y -= B[((p & 15) * 16 + (p >> 4)) * PS + ch].y;
+          if (A.accumulate) { v.x += o[i].x; v.y += o[i].y; }
+          ptr[i * step] = v;
+        }
     }
 }
 
@@ -571,21 +612,8 @@ __global__ __launch_bounds__(512) void k_xmac_f32_cross(XmacArgs A, const uint4*
     barrier();                           // everyone's have, and nobody still reads this stage
   }
 
-  const int c = c0 + w;
-  if (c >= A.nchan) return;
-#pragma unroll
-  for (int k = 0; k < NTILE; k++) {
-    const int b = input_of(32 * TL::J(k) + row);
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int a = input_of(32 * TL::I(k) + 8 * (r >> 2) + 4 * half + (r & 3));
-      if (a >= A.nin || b >= A.nin) continue;
-      float2* ptr = Vout + ((long long)a * A.nin + b) * A.nchan + c;
-      float2 v = make_float2(accR[k][r], accI[k][r]);
-      if (A.accumulate) { float2 o = *ptr; v.x += o.x; v.y += o.y; }
-      *ptr = v;
-    }
-  }
+  static_assert(2 * STAGE >= 2 * 2 * 256 * (CG + 1), "the ring holds the tiles on their way out");
+  store_tiles32<CG, TL>((float2*)lds, accR, accI, input_of, Vout, A.nin, A.nchan, c0, A.accumulate);
 }
 
 // ---------------------------------------------------------------------------
