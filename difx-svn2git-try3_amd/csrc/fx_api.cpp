@@ -618,7 +618,7 @@ int fxg_job_create(fxg_ctx* c, const fxg_job_desc* desc, fxg_job** out) {
   if (hipStreamCreateWithFlags(&j->copy_stream, hipStreamNonBlocking) != hipSuccess)
     return fail(set_err(FXG_EHIP, "copy stream"));
 
-  j->fstage_lin = !P.st[0].cplx && P.st[0].order != 2;
+  j->fstage_lin = P.st[0].order != 2 && (!P.st[0].cplx || P.L <= kFStageLinCMax);
   const int prec = desc->xmac_precision;
   // spectrum scale for reduced precision: 2^-round(log2(sqrt(L)))
   // (fp8: per-channel exponents instead, below)
@@ -1148,7 +1148,9 @@ static void fill_fstage_args(fxg_job* j, FStageArgs* fa) {
 // the F stage of every nbits-bit band over nblocks blocks from fa.chunk0
 static hipError_t launch_job_fstage(const fxg_job* j, int nbits, FStageArgs& fa, int nblocks, hipStream_t s) {
   const Plan& P = j->plan;
-  if (j->fstage_lin) return launch_fstage_lin(P.L, nbits, fa, nbits == 8 ? j->lists8 : j->lists2, nblocks, s);
+  if (j->fstage_lin)
+    return (P.st[0].cplx ? launch_fstage_lin_c : launch_fstage_lin)(P.L, nbits, fa, nbits == 8 ? j->lists8 : j->lists2,
+                                                                    nblocks, s);
   fa.bandlist = j->d_bandlist.as<int>() + (nbits == 8 ? j->nb2 : 0);
   return launch_fstage(P.L, nbits, P.st[0].cplx, fa, nbits == 8 ? j->nb8 : j->nb2, nblocks, s);
 }
@@ -1162,7 +1164,7 @@ static hipError_t launch_block_fstage(const fxg_job* j, int ds, FStageArgs& fa, 
     // the list of every band by itself, after the pairs and the lists by sample size
     l.singles = j->lists8.singles + j->lists8.nsingles + S.band0;
     l.nsingles = S.nchan;
-    return launch_fstage_lin(P.L, S.nbits, fa, l, 1, s);
+    return (S.cplx ? launch_fstage_lin_c : launch_fstage_lin)(P.L, S.nbits, fa, l, 1, s);
   }
   fa.bandlist = j->d_iota.as<int>() + S.band0;
   return launch_fstage(P.L, S.nbits, S.cplx, fa, S.nchan, 1, s);

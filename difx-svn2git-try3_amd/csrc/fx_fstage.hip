@@ -532,13 +532,313 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
 }
 
 // ---------------------------------------------------------------------------
+// k_fstage_lin_c<L, NBITS>: complex samples (Mode with usecomplex,
+// mode.cpp:1184-1241), linear rotation.  L complex samples a block, each a
+// unit of 2 NBITS bits with the real part low, through the passes of
+// k_fstage_lin with the same tables; every output is kept, channel c of the
+// band being bin m (USB: m = c; DSB: the halves swapped, m = c + L/2 mod L;
+// LSB: conjugated in reverse order, m = L - c with DC kept; LSB DSB: m = L/2 -
+// c mod L, conjugated; a conjugated bin's phase has its sign in DevRot).
+// The first pass reads units half a block apart in pairs: one LDS byte (2-bit)
+// and one 16-byte lookup, or one word (8-bit), decode two complex samples.
+// Bound by FP32 VALU issue like k_fstage_lin; the pairs lie in the exchange
+// buffer, for two workgroups a CU up to 8192 points, which a third barrier
+// pays.  1024 points, 2-bit, 8 stations of 8 bands, 4001 blocks (0.26
+// Gsamples): 1.10 -> 0.70 ms against k_fstage_c's rotator tables and radix-4
+// pass.
+// ---------------------------------------------------------------------------
+template <int L, int NBITS>
+__global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin_c(FStageArgs A) {
+  using Sh = FsShape<L>;
+  static_assert(Sh::PW == 1, "a workgroup holds whole blocks");
+  constexpr int P = Sh::P, R1 = Sh::R1, J1 = Sh::J1, J2 = Sh::J2, RL = Sh::RL, NTF = Sh::NTF, NB = Sh::NB, NT = Sh::NT;
+  constexpr bool MID = Sh::MID;
+  constexpr int UB = 2 * NBITS, UPW = 32 / UB;            // bits of a unit, units of a word
+  constexpr int GROUPS = L / 2 / UPW;                     // words of half a block
+  constexpr int NIT = (GROUPS + NTF - 1) / NTF;
+  constexpr int NL = L / RL, LPAD = 32 / RL;
+  constexpr int NE = Sh::NE + 8;                          // E[e] = e^{2 pi i theta e L/16} for e >= 8 at the end
+  struct Smem {
+    float2 tab[NB][NE];
+    float4 quad[NBITS == 2 ? 256 : 1];
+    float2 buf[NB][L + 32 + (NTF < 32 ? 1 : 0)];
+  };
+  __shared__ __align__(16) Smem sm;
+
+  const int tid = threadIdx.x;
+  const int fi = NB == 1 ? 0 : tid / NTF, t = NB == 1 ? tid : tid % NTF;
+  unsigned* const raw = (unsigned*)sm.buf[fi];
+  unsigned* const ok = raw + 2 * GROUPS;
+  static_assert(NBITS == 8 ? 2 * GROUPS <= 2 * L : 4 * GROUPS <= 2 * L, "pairs and validity fit the buffer");
+  // consecutive blocks go to one XCD, as in k_fstage_lin
+  const int grp = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  if (grp * NB >= A.nchunk) return;
+  const int cbx = grp * NB + fi;
+  const bool mine = NB == 1 || cbx < A.nchunk;
+  const int cb = mine ? cbx : A.nchunk - 1;
+  const int gband = A.pairs[blockIdx.y].x;
+  const DevBand& B = A.bands[gband];
+  const DevStationSub& Q = A.ss[B.station];
+  const DevRot& R = A.rots[(long long)B.rot * A.nblocks_subint + A.chunk0 + cb];
+  const bool dead = R.status != 0;
+  if (NB == 1 && dead) {
+    zero_spec(A.spectra, A.prec, B.specoff + (long long)cb * A.bstride, L, A.gstride, tid, NT);
+    return;
+  }
+
+  // ---- the block's samples: two rows half a block apart, to pairs of units
+  const bool fast = R.allvalid != 0 || dead;
+  const long long bit0 = (long long)(dead ? 0 : R.t0) * UB;
+  const long long nwords = Q.ctstride >> 2;
+  const unsigned* const src = (const unsigned*)(A.ct + Q.ctbase + (long long)B.band * Q.ctstride);
+  unsigned lo[NIT][2], hi[NIT][2];
+#pragma unroll
+  for (int i = 0; i < NIT; i++)
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+      const long long w = (bit0 >> 5) + t + i * NTF + m * GROUPS;
+      lo[i][m] = w < nwords ? src[w] : 0u;
+      hi[i][m] = w + 1 < nwords ? src[w + 1] : 0u;
+    }
+  {
+    const double delta = R.delta, theta = R.theta;
+    for (int i = NTF - 1 - t; i < NE; i += NTF) {
+      const float4 d = A.cdesc[i];
+      sm.tab[fi][i] = exact_rotator(theta * (double)d.y - (delta * (double)d.x + (double)d.z));
+    }
+  }
+  if (NBITS == 2)
+    for (int i = tid; i < 256; i += NT) sm.quad[i] = A.quad[B.levels * 256 + i];
+#pragma unroll
+  for (int i = 0; i < NIT; i++) {
+    const int g = t + i * NTF;
+    unsigned a[2], v[2] = {0u, 0u};
+#pragma unroll
+    for (int m = 0; m < 2; m++) a[m] = __builtin_amdgcn_alignbit(hi[i][m], lo[i][m], (int)(bit0 & 31));
+    if (!fast) {
+      const DevStation& S = A.st[B.station];
+#pragma unroll
+      for (int m = 0; m < 2; m++)
+        v[m] = valid_samples<UPW>(S, Q, A.ftab, R.t0 + (long long)(m * GROUPS + g) * UPW, R.validend, B.band);
+      if (NBITS == 2) {
+        // a bit for each float of the pair: real and imaginary parts of both
+        auto spread = [](unsigned x) { return ((x & 15u) * 0x00204081u) & 0x01010101u; };
+        unsigned m0 = spread(v[0]) * 3u | spread(v[1]) * 12u, m1 = spread(v[0] >> 4) * 3u | spread(v[1] >> 4) * 12u;
+        if (S.granularity > 1) {
+          // one band of 2-bit complex samples: the unpacker's erasure by float
+          // index zeroes sample L/2 (even start) or the imaginary part of
+          // sample L/2 - 1 (odd start)
+          if ((R.t0 & 1) == 0) { if (g == 0) m0 &= ~12u; }
+          else if (g == GROUPS - 1) m1 &= ~(2u << 24);
+        }
+        ok[2 * g] = m0;
+        ok[2 * g + 1] = m1;
+      }
+    }
+    if (NBITS == 8) {
+#pragma unroll
+      for (int m = 0; m < 2; m++) {
+        a[m] ^= 0x80808080u;                               // signed levels, 0 = none
+        if (!fast) a[m] &= ((v[m] & 1u) | (v[m] & 2u) << 15) * 0xFFFFu;
+      }
+      *(uint2*)&raw[2 * g] = make_uint2(__builtin_amdgcn_perm(a[1], a[0], 0x05040100u),
+                                        __builtin_amdgcn_perm(a[1], a[0], 0x07060302u));
+    } else {
+      auto spread = [](unsigned x) {
+        x = (x | (x << 8)) & 0x00FF00FFu;
+        return (x | (x << 4)) & 0x0F0F0F0Fu;
+      };
+      *(uint2*)&raw[2 * g] = make_uint2(spread(a[0] & 0xFFFFu) | spread(a[1] & 0xFFFFu) << 4,
+                                        spread(a[0] >> 16) | spread(a[1] >> 16) << 4);
+    }
+  }
+  __syncthreads();
+
+  auto sync = [] {
+    if (NTF > 64) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  };
+  float2* const buf = sm.buf[fi];
+  const float2* const tab = sm.tab[fi];
+
+  // ---- pass 1: decode, radix R1 (this thread's 16 of the R1 outputs)
+  {
+    const int p = t / J1, j = t % J1;
+    const float2* c = tab + p * Sh::CP;
+    Tw16 w;
+    w.w8 = c[0]; w.w4 = c[1]; w.w2 = c[2]; w.w2h = c[3]; w.w1 = c[4]; w.w1a = c[5]; w.w1b = c[6]; w.w1c = c[7];
+    // units j + r J1 and, half a block on, j + (r + R1/2) J1: eight of them
+    // from r0 (four from r0 and four from r0 + 16 where P = 4), all their LDS
+    // reads in flight together
+    auto pairs_at = [&](int r0, float4* x) {
+      unsigned q[8];
+      auto at = [&](int i) { return j + (r0 + (P == 4 ? (i & 3) + 4 * (i & 4) : i)) * J1; };
+      if (NBITS == 8) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) q[i] = raw[at(i)];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          x[i] = make_float4((float)(signed char)(q[i] & 0xFFu), (float)(signed char)((q[i] >> 8) & 0xFFu),
+                             (float)(signed char)((q[i] >> 16) & 0xFFu), (float)(signed char)(q[i] >> 24));
+        return;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) q[i] = ((const unsigned char*)raw)[at(i)];
+#pragma unroll
+      for (int i = 0; i < 8; i++) x[i] = sm.quad[q[i]];
+      if (!fast) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const unsigned m = ((const unsigned char*)ok)[at(i)];
+          x[i].x = m & 1u ? x[i].x : 0.0f;
+          x[i].y = m & 2u ? x[i].y : 0.0f;
+          x[i].z = m & 4u ? x[i].z : 0.0f;
+          x[i].w = m & 8u ? x[i].w : 0.0f;
+        }
+      }
+    };
+    float2 v[16];
+    if (P == 1) {
+      float4 x[8];
+      pairs_at(0, x);
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        v[r] = make_float2(x[r].x, x[r].y);
+        v[r + 8] = make_float2(x[r].z, x[r].w);
+      }
+    } else if (P == 2) {
+      const float2 g2 = c[8];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        float4 x[8];
+        pairs_at(8 * h, x);
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+          v[8 * h + r] = bfly_plus(make_float2(x[r].x, x[r].y), make_float2(x[r].z, x[r].w), g2);
+      }
+    } else {
+      // x0 + g1 x1 + g2 x2 + g3 x3 of samples a quarter of the block apart
+      const float2 g1 = c[8], g2 = c[9], g3 = c[10];
+#pragma unroll
+      for (int h = 0; h < 4; h++) {
+        float4 x[8];
+        pairs_at(4 * h, x);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          v[4 * h + r] = bfly_plus(bfly_plus(bfly_plus(make_float2(x[r].x, x[r].y), make_float2(x[r + 4].x, x[r + 4].y), g1),
+                                             make_float2(x[r].z, x[r].w), g2),
+                                   make_float2(x[r + 4].z, x[r + 4].w), g3);
+        // summed before the next lookups, for registers
+#pragma unroll
+        for (int r = 0; r < 4; r++) asm volatile("" : "+v"(v[4 * h + r].x), "+v"(v[4 * h + r].y) :: "memory");
+      }
+    }
+    dft16_tw<false>(v, w);
+    sync();                                                // every pair read before the buffer is written
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int k = P * q + p;
+      const int slot = MID ? k * J1 + (j ^ (J2 * (k % (32 / J2)))) : j * (NL + LPAD) + k;
+      buf[slot] = v[bitrev4(q)];
+    }
+  }
+  sync();
+
+  // ---- middle pass: radix 16 from R1 to 16 R1 bins
+  if (MID) {
+    const int j = t % J2, k = t / J2;
+    Tw16 w;
+    const float2* c = tab + Sh::MIDOFF + 8 * k;
+    w.w8 = c[0]; w.w4 = c[1]; w.w2 = c[2]; w.w2h = c[3]; w.w1 = c[4]; w.w1a = c[5]; w.w1b = c[6]; w.w1c = c[7];
+    constexpr int NX = 32 / J2;
+    int off[NX];
+#pragma unroll
+    for (int i = 0; i < NX; i++) off[i] = k * J1 + j + J2 * (i ^ (k % NX));
+    float2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = buf[off[r % NX] + J2 * (r - r % NX)];
+    dft16_tw<false>(v, w);
+    sync();
+    float2* op = buf + j * (NL + LPAD) + k;
+#pragma unroll
+    for (int q = 0; q < 16; q++) op[R1 * q] = v[bitrev4(q)];
+    sync();
+  }
+
+  // ---- last pass (radix RL), bins t + e L/16
+  const float2* const cl = tab + Sh::LAST;
+  float2 x[16];
+  if (RL == 16) {
+    Tw16 tw;
+    tw.w8 = cmulx(A.base[t], cl[0]); tw.w4 = cmulx(A.base[NTF + t], cl[1]);
+    tw.w2 = cmulx(A.base[2 * NTF + t], cl[2]); tw.w1 = cmulx(A.base[3 * NTF + t], cl[3]);
+    tw16_multiples(tw);
+    float2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = buf[r * (NL + LPAD) + t];
+    dft16_tw<false>(v, tw);
+#pragma unroll
+    for (int e = 0; e < 16; e++) x[e] = v[bitrev4(e)];
+  } else {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      float2 v[8];
+#pragma unroll
+      for (int r = 0; r < 8; r++) v[r] = buf[r * (NL + LPAD) + t + u * NTF];
+      dft8_tw<false>(v, cmulx(A.base[u * NTF + t], cl[1]), cmulx(A.base[(2 + u) * NTF + t], cl[2]),
+                     cmulx(A.base[(4 + u) * NTF + t], cl[3]));
+#pragma unroll
+      for (int q = 0; q < 8; q++) x[u + 2 * q] = v[bitrev3(q)];
+    }
+  }
+  if (!mine) return;
+
+  // ---- to the channels: bin t + e L/16 is channel c0 + f L/16
+  const bool lsb = B.lsb;
+  const int c0 = !lsb ? t : t == 0 ? 0 : NTF - t;
+  const float s = dead ? 0.0f : (NBITS == 8 ? A.scale * (float)(1.0 / 3.3) : A.scale);
+  float2 dc = make_float2(0.0f, 0.0f);
+  float2 F = exact_rotator(R.phase + R.theta * (double)c0);
+  F = make_float2(F.x * s, F.y * s);
+  if (B.polre != 1.0f || B.polim != 0.0f) F = cmulx(F, make_float2(B.polre, B.polim));
+  if (lsb && !B.dsb && t == 0) {
+    // DC is not conjugated: its phase is theta0 - ph, where F's is theta0 + ph,
+    // theta0 = -theta L
+    float2 G = exact_rotator(-2.0 * R.theta * (double)L - R.phase);
+    G = make_float2(G.x * s, G.y * s);
+    if (B.polre != 1.0f || B.polim != 0.0f) G = cmulx(G, make_float2(B.polre, B.polim));
+    dc = cmulx(x[0], G);
+  }
+  const int f0 = (lsb ? (t == 0 ? 16 : 15) : 0) + (B.dsb ? 8 : 0), fs = lsb ? -1 : 1;
+  const long long outbase = B.specoff + (long long)cb * A.bstride;
+  auto store = [&](auto out) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int f = (f0 + fs * e) & 15, c = c0 + f * NTF;
+      float2 y = cmulx(lsb ? make_float2(x[e].x, -x[e].y) : x[e], cmulx(F, tab[f < 8 ? Sh::LAST + 4 + f : Sh::NE - 8 + f]));
+      if (e == 0 && lsb && !B.dsb && t == 0) y = dc;
+      put_spec(out, cidx(c, A.gstride), c, y);
+    }
+  };
+  if (A.prec == FXG_XMAC_FP32) store((float2*)A.spectra + outbase);
+  else if (A.prec == FXG_XMAC_FP16) store((__half2*)A.spectra + outbase);
+  else if (A.prec == FXG_XMAC_FP8) store(Fp8Out{(unsigned short*)A.spectra + outbase, A.cexp + (long long)gband * L});
+  else store((__hip_bfloat162*)A.spectra + outbase);
+}
+
+// ---------------------------------------------------------------------------
 // host side: the tables of one length
 // ---------------------------------------------------------------------------
 template <int L>
 static void fill_tables(std::vector<float4>* cdesc, std::vector<float2>* base) {
   using Sh = FsShape<L>;
   constexpr int M = Sh::M, PW = Sh::PW, P = Sh::P;
-  cdesc->assign(Sh::NE, make_float4(0.f, 0.f, 0.f, 0.f));
+  cdesc->assign(Sh::NE + 8, make_float4(0.f, 0.f, 0.f, 0.f));
   // entry = e^{2 pi i (theta y - delta x - z - pw w)}
   auto set = [&](int i, double x, double z, double w, double y = 0.0) {
     (*cdesc)[i] = make_float4((float)x, (float)y, (float)(z - std::floor(z)), (float)w);
@@ -565,6 +865,7 @@ static void fill_tables(std::vector<float4>* cdesc, std::vector<float2>* base) {
   const int ml[4] = {8, 4, 2, 1};
   for (int i = 0; i < 4; i++) set(Sh::LAST + i, ml[i], 0.0, (double)ml[i] / L);
   for (int e = 0; e < 8; e++) set(Sh::LAST + 4 + e, 0.0, 0.0, 0.0, (double)(L / 16) * e);
+  for (int e = 8; e < 16; e++) set(Sh::NE - 8 + e, 0.0, 0.0, 0.0, (double)(L / 16) * e);   // complex samples
   if (Sh::MID)
     for (int k = 0; k < Sh::R1; k++) tw16(Sh::MIDOFF + 8 * k, 16 * Sh::R1, k);
   // last pass at d = 0: powers 8, 4, 2, 1 (radix 16) or 4, 2, 1 of its two
@@ -617,6 +918,27 @@ hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, const BandLi
       break;                                                                                                        \
     }
     FX_LENGTHS(X)
+#undef X
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_fstage_lin_c(int L, int nbits, const FStageArgs& a, const BandLists& l, int nblocks,
+                               hipStream_t stream) {
+  if (nbits != 2 && nbits != 8) return hipErrorInvalidValue;
+  FStageArgs b = a;
+  b.nchunk = nblocks;
+  b.pairs = l.singles;
+  switch (L) {
+#define X(Lv)                                                                                                       \
+    case Lv: {                                                                                                      \
+      const dim3 grid((unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8), l.nsingles);     \
+      if (nbits == 2) hipLaunchKernelGGL((k_fstage_lin_c<Lv, 2>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);       \
+      else hipLaunchKernelGGL((k_fstage_lin_c<Lv, 8>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);                  \
+      break;                                                                                                        \
+    }
+    X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192)
 #undef X
     default: return hipErrorInvalidValue;
   }

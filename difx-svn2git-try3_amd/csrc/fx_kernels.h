@@ -157,6 +157,10 @@ hipError_t launch_fstage(int L, int nbits, int cplx, const FStageArgs& a, int nb
 // one length, and the levels of four 2-bit samples by their byte (256 entries)
 hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, const BandLists& l, int nblocks,
                              hipStream_t stream);
+// complex samples, up to kFStageLinCMax of them a block
+constexpr int kFStageLinCMax = 8192;
+hipError_t launch_fstage_lin_c(int L, int nbits, const FStageArgs& a, const BandLists& l, int nblocks,
+                               hipStream_t stream);
 bool fstage_lin_tables(int L, std::vector<float4>* cdesc, std::vector<float2>* base);
 void fstage_quad_levels(const float* lut, float4* out);
 hipError_t launch_unpack(const DevStation* st, const DevStationSub* ss, const int2* ftab, const float* lut8,

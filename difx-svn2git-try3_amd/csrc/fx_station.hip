@@ -5,7 +5,7 @@
 //               mk5mode.cpp:104-177)
 //   k_fstage<L> LUT unpack -> quadratic fringe rotation -> L-point FP32
 //               Stockham FFT -> sideband select -> fractional-sample rotation
-//               -> spectra (mode.cpp:909-1310); k_fstage_c complex samples;
+//               -> spectra (mode.cpp:909-1310); k_fstage_c complex samples with order 2;
 //               k_bigfft_a/b transforms above 16384 points.  Real samples
 //               with linear or post-F rotation: fx_fstage.hip
 //   k_unpack    standalone Mk5Mode::unpack equivalent
@@ -325,7 +325,9 @@ __device__ __forceinline__ DevRot block_rotation(const DevStation& S, const DevR
   const float val = (float)((double)G.fse - B.clock + sign * B.clockdelta / 2);
   r.theta = (double)val * S.bw / S.C;
   const double theta0 = B.dsb ? -0.5 * (double)val * S.bw : B.lsb ? -(double)val * S.bw : 0.0;
-  const double q = theta0 - (ph - rint(ph));
+  // (a conjugated transform, the lower sideband of complex samples, turns the
+  // rotator's phase round)
+  const double q = theta0 - (S.cplx && B.lsb ? -1.0 : 1.0) * (ph - rint(ph));
   r.phase = q - rint(q);
   return r;
 }
@@ -929,7 +931,8 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage(FStageArgs A) {
 // L-point transform with every output kept, channel c of the band taken from
 // bin m (USB: m = c; DSB: the halves swapped, m = c + L/2 mod L; LSB:
 // conjugated in reverse order, m = L - c with DC kept unconjugated; LSB DSB:
-// m = L/2 - c mod L, conjugated), then the fractional-sample rotation.
+// m = L/2 - c mod L, conjugated), then the fractional-sample rotation.  For
+// quadratic rotation, and linear at 16384 channels (the rest: k_fstage_lin_c).
 // ---------------------------------------------------------------------------
 template <int L, int NBITS>
 __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
