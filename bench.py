@@ -297,7 +297,7 @@ def roofline(spec, info, stage, launch, precision):
     samples = spec.nstations * spec.nrecbands * nblk * L
     if dom == "fstage":
         avg_s = stage["fstage"]["ms"] / stage["fstage"]["launches"] / 1e3
-        kname = f"fxg::k_fstage<{L}, 2>"
+        kname = f"fxg::k_fstage_lin<{L}, 2>"
         # 2-bit input read once + spectra written once
         nbytes = samples * 0.25 + spec.nstations * spec.nrecbands * nblk * C_ * specbytes
         # FFT 5 log2 L, fringe rotation 6, fractional-sample rotation 3 flops per sample
@@ -323,8 +323,11 @@ def roofline(spec, info, stage, launch, precision):
     nbytes = nin * C_ * nblk * specbytes * spec.nsubbands / nfreq
     peak = PEAK_TFLOPS[precision]
     bf = "true" if precision == "bf16" else "false"
-    kname = (f"fxg::k_xmac_mfma_dl<2, {bf}, false>" if launch["schedule"]["xmac_streaming"]
-             else f"fxg::k_xmac_mfma<2, {bf}, 16>")
+    streaming = launch["schedule"]["xmac_streaming"]
+    if precision == "fp32":
+        kname = "fxg::k_xmac_f32_t16<4>" if streaming else "fxg::k_xmac_f32<HIP_vector_type<float, 2u>>"
+    else:
+        kname = f"fxg::k_xmac_mfma_dl<2, {bf}, false>" if streaming else f"fxg::k_xmac_mfma<2, {bf}, 16>"
     tf = flops / avg_s / 1e12
     hbm_frac = nbytes / avg_s / 1e9 / HBM_PEAK_GBS
     roof = {"kernel": kname, "avg_launch_ms": avg_s * 1e3, "traffic": profiled_traffic(kname),

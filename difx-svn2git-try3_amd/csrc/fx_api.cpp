@@ -1186,7 +1186,7 @@ static std::vector<unsigned char> subint_key(const fxg_job* j, const fxg_subint_
   return k;
 }
 
-// F and X stages chunk by chunk, weights, the cleared result, scatter and
+// F and X stages chunk by chunk, weights, scatter (the result wholly) and
 // phase cal, launched on stream s into dres (a device result buffer).
 static int launch_back(fxg_job* j, float* dres, hipStream_t s) {
   Plan& P = j->plan;

@@ -1,5 +1,6 @@
-// fx_fstage.hip — the F stage of real-sampled data with linear (or post-F)
-// fringe rotation (mode.cpp:909-1310): level decoding, fringe rotation, FFT, sideband select, fractional-sample rotation.
+// fx_fstage.hip — the F stage with linear (real samples: or post-F) fringe
+// rotation (mode.cpp:909-1310): level decoding, fringe rotation, FFT, sideband
+// select, fractional-sample rotation.
 #include <hip/hip_runtime.h>
 #include "fx_kernels.h"
 #include "fx_device.h"

@@ -5,9 +5,10 @@
 //               mk5mode.cpp:104-177)
 //   k_fstage<L> LUT unpack -> quadratic fringe rotation -> L-point FP32
 //               Stockham FFT -> sideband select -> fractional-sample rotation
-//               -> spectra (mode.cpp:909-1310); k_fstage_c complex samples with order 2;
-//               k_bigfft_a/b transforms above 16384 points.  Real samples
-//               with linear or post-F rotation: fx_fstage.hip
+//               -> spectra (mode.cpp:909-1310); k_fstage_c complex samples (and
+//               linear at 16384 channels); k_bigfft_a/b transforms above
+//               16384 points.  Real samples with
+//               linear or post-F rotation, complex ones with linear: fx_fstage.hip
 //   k_unpack    standalone Mk5Mode::unpack equivalent
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -399,11 +400,8 @@ template <> struct DFT<8> {
     v[3] = add2(e3, o3); v[7] = sub2(e3, o3);
   }
 };
-// 16-point DFT from the first butterflies' outputs: sm[r] = v[r] + v[r + 8],
-// df[r] = v[r] - v[r + 8] (r < 8), so that a caller can fold the products
-// that form v into them
+// sm[r] = v[r] + v[r + 8], df[r] = v[r] - v[r + 8] (r < 8)
 __device__ __forceinline__ void dft16_from_halves(const float2* sm, const float2* df, float2* v);
-
 template <> struct DFT<16> {
   __device__ static void run(float2* v) {
     float2 sm[8], df[8];
@@ -506,8 +504,8 @@ __device__ __forceinline__ int pidx(int a) { return a + (a >> 4); }
 
 // ---------------------------------------------------------------------------
 // Rotator tables of one (band, block) at FFT length L, by the threads tid of
-// NT: FP64 phases, FP32 residual sin/cos (mode.cpp:909-1097).  rot: the pre-F
-// sub/step (and quadratic) rotators; frac: the fractional-sample sub/step.
+// NT: FP64 phases, FP32 residual sin/cos (mode.cpp:909-1097): the pre-F sub,
+// step (and quadratic) rotators and the fractional-sample sub and step.
 // ---------------------------------------------------------------------------
 // e^{i 2 pi t} for t in turns (|t| < 256) by the hardware sine and cosine
 __device__ __forceinline__ float2 turn_rotator(float t) {
@@ -524,7 +522,7 @@ __device__ __forceinline__ float2 angle_rotator(float x) {
 // C: the recorded channels, L/2 (real) or L (complex) -- a compile-time
 // power of two at every call, so the divisions by it are exact products
 __device__ __forceinline__ void rotator_tables(const DevBand& B, const DevStation& S, const DevBlock& G, int L,
-                                               int C, int tid, int NT, bool rot, bool frac, float2* rsub,
+                                               int C, int tid, int NT, float2* rsub,
                                                float2* rstep, float2* fsub, float2* fstep, float2* rquad) {
 #pragma clang fp contract(off)
   const int s = S.s;
@@ -540,22 +538,10 @@ __device__ __forceinline__ void rotator_tables(const DevBand& B, const DevStatio
   // The entries of the four tables are dealt out over the threads as one
   // index range (sub, step, frac sub, frac step), so that no wave computes
   // more than its share of the sin/cos.
-  const int nsub = (rot && S.order != 0) ? s : 0;
-  const int nstep = (rot && S.order != 0) ? S.nfrsteps : 0;
-  const int nfsub = frac ? s : 0;
-  const int nfstep = frac ? S.nfracsteps : 0;
+  const int nsub = s, nstep = S.nfrsteps, nfsub = s, nfstep = S.nfracsteps;
   const int e1 = nsub, e2 = e1 + nstep, e3 = e2 + nfsub, e4 = e3 + nfstep;
   const double sign = B.useB ? -1.0 : 1.0;
   const float val = (float)((double)G.fse - B.clock + sign * B.clockdelta / 2);
-  // order 0: the fringe phase of the block at its centre delay, added to
-  // the sub arguments (mode.cpp:1064-1073, 1111-1119)
-  float postf = 0.0f;
-  if (S.order == 0 && nfsub > 0) {
-    double phaserotation = (G.c - G.integerdelay) * lofreq;
-    if (S.fractionalLo) phaserotation += G.integerdelay * (lofreq - (int)lofreq);
-    phaserotation -= G.wall * looffset;
-    postf = (float)(-kTwoPi * (phaserotation - (int)phaserotation));
-  }
   // pre-F rotator points: order 1 x = a k/L + b (mode.cpp:804-812), order 2
   // x = (k/L)(b + a s/L) + c with quad points (k/L) 2a s/L and steps
   // (js/L) b + (js/L)^2 a (mode.cpp:821-837)
@@ -586,8 +572,7 @@ __device__ __forceinline__ void rotator_tables(const DevBand& B, const DevStatio
     } else if (e < e3) {
       const int k = e - e2;
       float cf = (float)((kTwoPi * k * S.bw) / C);
-      float arg = cf * val;
-      if (S.order == 0) arg = arg + postf;
+      const float arg = cf * val;
       // the band's polarisation phase correction rides on every channel's
       // fractional-sample rotator (a constant factor)
       fsub[k] = cmulf(angle_rotator(arg), make_float2(B.polre, B.polim));
@@ -746,7 +731,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage(FStageArgs A) {
   float2* rquad = fstep + S.nfracsteps;         // order 2 only
 
   // ---- rotator tables: FP64 phase, FP32 residual (mode.cpp:909-978, 1054-1097)
-  rotator_tables(B, S, G, L, L / 2, tid, NT, true, true, rsub, rstep, fsub, fstep, rquad);
+  rotator_tables(B, S, G, L, L / 2, tid, NT, rsub, rstep, fsub, fstep, rquad);
   ts.store(twlo, twhi, tw256, lut8s, tid);
   if (fast) {
 #pragma unroll
@@ -1003,7 +988,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
   float2* fsub = rstep + S.nfrsteps;
   float2* fstep = fsub + S.s;
   float2* rquad = fstep + S.nfracsteps;
-  rotator_tables(B, S, G, L, L, tid, NT, true, true, rsub, rstep, fsub, fstep, rquad);
+  rotator_tables(B, S, G, L, L, tid, NT, rsub, rstep, fsub, fstep, rquad);
   ts.store(twlo, twhi, tw256, lut8s, tid);
   if (fast) {
 #pragma unroll
@@ -1192,7 +1177,7 @@ __global__ __launch_bounds__(256) void k_rotab(FStageArgs A) {
   const DevBlock G = A.blocks[(long long)B.station * A.nblocks_subint + blk];
   if (G.status != 0) return;
   float2* rt = A.rtab + ((long long)gband * A.zcap + cbl) * A.rtabn;
-  rotator_tables(B, S, G, L, L / 2, threadIdx.x, 256, true, true, rt, rt + S.s, rt + 2 * S.s + S.nfrsteps,
+  rotator_tables(B, S, G, L, L / 2, threadIdx.x, 256, rt, rt + S.s, rt + 2 * S.s + S.nfrsteps,
                  rt + 3 * S.s + S.nfrsteps, rt + S.s + S.nfrsteps);
 }
 
