@@ -73,6 +73,7 @@ __global__ __launch_bounds__(256) void k_pcal_few(PcalArgs A) {
     int n = b - som;
     if (n < 0) n += N;
     n += sl * N;
+    float br = 0.0f, bi = 0.0f;                  // a block by itself first: shorter chains of roundings
     auto add = [&](int at, float2 x) {
       if (pc.rot) {
         int m = sor + at;
@@ -81,8 +82,8 @@ __global__ __launch_bounds__(256) void k_pcal_few(PcalArgs A) {
         if (pc.csamp) x = cmulf(x, r);                       // vectorMul_cf32 by the mixer
         else x = make_float2(x.x * r.x, x.x * r.y);
       }
-      ar += x.x;
-      ai += x.y;
+      br += x.x;
+      bi += x.y;
     };
     if (G.allvalid != 0) {
       while (n < L) {
@@ -122,6 +123,8 @@ __global__ __launch_bounds__(256) void k_pcal_few(PcalArgs A) {
         add(n, x);
       }
     }
+    ar += br;
+    ai += bi;
   }
   acc[tid] = make_float2(ar, ai);
   __syncthreads();
