@@ -347,15 +347,16 @@ __global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_dl(XmacArgs A,
 // Ai Br^T, formed once at the end, so three.  32x32 tiles cost 2 x 64 cycles
 // a block and channel for up to 32 inputs and 6 x 64 for up to 64; these
 // 24 (16 inputs), 80 (32), 168 (48), 288 (64).
-// Rows past the last input are neither loaded nor read back (a row of A or B
-// only reaches its own row or column of the tile); blocks past the last read
-// a 16-byte zero buffer.  LDS is a ring of stages of 8 blocks x 16 channels x
-// 16 T rows, filled by global_load_lds, as deep as leaves two workgroups on a
-// CU for one and two tiles: there the load stream is the bound, above it the
-// matrix cores.
-// 4 stations, 256 channels, 62500 blocks 1109 -> 320 us; 10 stations, 1024
-// channels, 4096 blocks 327 -> 249 us a frequency; 32 stations, 4096
-// channels, 500 blocks 494 -> 485 us.
+// Rows past the last input are not read back (a row of A or B only reaches its
+// own row or column of the tile); they and blocks past the last read a 16-byte
+// zero buffer.  LDS is a ring of stages of 4 or 8 blocks x 16 channels x 16 T
+// rows, filled by global_load_lds, as deep as leaves two workgroups on a CU for
+// one and two tiles: there the load stream is the bound, above it the matrix
+// cores.  At 64 inputs two stages of 8 blocks: four of 4 take 382 against 414
+// us at 500 blocks, but 1661 against 1570 at 2000 (4096 channels, constant
+// data).
+// 10 stations, 1024 channels, 4096 blocks 327 -> 249 us a frequency; 32
+// stations, 4096 channels, 500 blocks 494 -> 440 us, 2000 blocks 1.74 -> 1.67 ms.
 // ---------------------------------------------------------------------------
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -368,9 +369,9 @@ template <int N> __device__ __forceinline__ void wait_vm() {
 template <int T>
 __global__ __launch_bounds__(1024, T <= 2 ? 8 : 4) void k_xmac_f32_t16(XmacArgs A, const uint4* __restrict__ zero16) {
   constexpr int CG = 16;                 // channels (wavefronts) per workgroup
-  constexpr int TT = T == 1 ? 8 : 4;     // blocks per stage
+  constexpr int TT = T == 1 || T == 4 ? 8 : 4;   // blocks per stage
   constexpr int RPI = 8 / TT;            // rows of a load instruction
-  constexpr int NBUF = T == 3 ? 5 : 4;
+  constexpr int NBUF = T == 4 ? 2 : T == 3 ? 5 : 4;
   constexpr int NTILE = T * (T + 1) / 2;
   constexpr int RBW = 2 * CG;            // dwords per (row, block)
   constexpr int SDW = 8 * RBW + 4;       // dwords per load instruction: RPI rows of a stage, padded
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(1024, T <= 2 ? 8 : 4) void k_xmac_f32_t16(XmacArgs 
     else if (nv == 2) wait_vm<(NBUF - 2) * 2>();
     else wait_vm<0>();
   };
-  static_assert(LPW <= 2, "landed");
+  static_assert(LPW <= 2 || NBUF == 2, "landed");
   auto barrier = [] {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
