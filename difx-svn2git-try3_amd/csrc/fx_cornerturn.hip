@@ -167,13 +167,21 @@ __global__ __launch_bounds__(256) void k_cornerturn_u(const DevStation* __restri
   if (g0 >= groups) return;                             // the whole workgroup
   const long long fw = g0 * NC / wpf;                   // frame and word of the workgroup's first word
   const int rw = (int)(g0 * NC - fw * wpf);
+  // and of this thread's first group, and its step of 256 groups, by division:
+  // one frame at a time a workgroup's last group of a payload of 8 bytes is 2048
+  // steps off (the stage for 8 blocks of 512 samples, two 8-bit bands: 288 -> 9 us)
+  const unsigned r0 = (unsigned)rw + threadIdx.x * NC, step = 256 * NC / (unsigned)wpf;
+  long long fg = fw + r0 / (unsigned)wpf;
+  int rg = (int)(r0 % (unsigned)wpf);
   union { uint32_t w[NC]; VW v[NV]; } x[K];
 #pragma unroll
   for (int k = 0; k < K; k++) {
     const int o = (threadIdx.x + k * 256) * NC;
-    long long f = fw;
-    int r = rw + o;
-    while (r >= wpf) { r -= wpf; f++; }
+    long long f = fg;
+    int r = rg;
+    fg += step;
+    rg += 256 * NC - (int)step * wpf;
+    if (rg >= wpf) { rg -= wpf; fg++; }
     const long long left = total - g0 * NC - o;         // words from this group's first to the stream's end
 #pragma unroll
     for (int i = 0; i < NV; i++) {
