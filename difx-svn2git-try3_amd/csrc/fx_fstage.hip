@@ -5,6 +5,7 @@
 #include "fx_kernels.h"
 #include "fx_device.h"
 #include "fx_fft.h"
+#include "fx_place.h"
 #include "fx_spectra.h"
 #include <cmath>
 #include <vector>
@@ -166,17 +167,15 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin(FStageArgs A) 
   const int fi = NB == 1 ? 0 : tid / NTF, t = NB == 1 ? tid : tid % NTF;
   unsigned* const raw = RAWOWN ? sm.raw_own + fi * QW : (unsigned*)sm.buf[fi];
   unsigned* const ok = RAWOWN ? sm.ok_own + fi * QW : (unsigned*)sm.buf[fi] + QW;
-  // block groups within the chunk: workgroups are dealt to the 8 XCDs
-  // round-robin, so consecutive blocks go to one XCD (its L2 merges the
-  // halves of the lines that neighbouring blocks write in the grouped layout)
-  const int grp = (blockIdx.x % 8) * (gridDim.x / (8 * PW)) + blockIdx.x / (8 * PW);
-  const int pw = PW == 1 ? 0 : (blockIdx.x / 8) % PW;
-  if (grp * NB >= A.nchunk) return;
-  const int cbx = grp * NB + fi;
+  // this workgroup's bands and group of blocks within the chunk
+  const FsPlace place = fstage_place(blockIdx.x, blockIdx.y, gridDim.x, (unsigned)(A.nchunk + NB - 1) / NB, PW);
+  if (place.row >= (unsigned)A.nrows || place.grp * NB >= (unsigned)A.nchunk) return;
+  const int pw = PW == 1 ? 0 : place.pw;
+  const int cbx = place.grp * NB + fi;
   const bool mine = NB == 1 || cbx < A.nchunk;
   const int cb = mine ? cbx : A.nchunk - 1;
   // one band, or two that share a rotation (the polarisations of a frequency)
-  const int2 pair = A.pairs[blockIdx.y];
+  const int2 pair = A.pairs[place.row];
   const int nband = Sh::TWO && pair.y >= 0 ? 2 : 1;
   const DevBand& B0 = A.bands[pair.x];
   const DevBand& B1 = A.bands[nband == 2 ? pair.y : pair.x];
@@ -571,13 +570,12 @@ __global__ __launch_bounds__(FsShape<L>::NT, 4) void k_fstage_lin_c(FStageArgs A
   unsigned* const raw = (unsigned*)sm.buf[fi];
   unsigned* const ok = raw + 2 * GROUPS;
   static_assert(NBITS == 8 ? 2 * GROUPS <= 2 * L : 4 * GROUPS <= 2 * L, "pairs and validity fit the buffer");
-  // consecutive blocks go to one XCD, as in k_fstage_lin
-  const int grp = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-  if (grp * NB >= A.nchunk) return;
-  const int cbx = grp * NB + fi;
+  const FsPlace place = fstage_place(blockIdx.x, blockIdx.y, gridDim.x, (unsigned)(A.nchunk + NB - 1) / NB, 1);
+  if (place.row >= (unsigned)A.nrows || place.grp * NB >= (unsigned)A.nchunk) return;
+  const int cbx = place.grp * NB + fi;
   const bool mine = NB == 1 || cbx < A.nchunk;
   const int cb = mine ? cbx : A.nchunk - 1;
-  const int gband = A.pairs[blockIdx.y].x;
+  const int gband = A.pairs[place.row].x;
   const DevBand& B = A.bands[gband];
   const DevStationSub& Q = A.ss[B.station];
   const DevRot& R = A.rots[(long long)B.rot * A.nblocks_subint + A.chunk0 + cb];
@@ -910,10 +908,12 @@ hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, const BandLi
   switch (L) {
 #define X(Lv)                                                                                                       \
     case Lv: {                                                                                                      \
-      const unsigned gx = (unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8 * FsShape<Lv>::PW); \
-      const bool two = FsShape<Lv>::TWO && (long long)gx * l.npairs >= kPairWorkgroups;                             \
+      const int groups = (nblocks + FsShape<Lv>::NB - 1) / FsShape<Lv>::NB;                                         \
+      const bool two = FsShape<Lv>::TWO && (groups + 7LL) / 8 * 8 * l.npairs >= kPairWorkgroups;                    \
       b.pairs = two ? l.pairs : l.singles;                                                                          \
-      const dim3 grid(gx, two ? l.npairs : l.nsingles);                                                             \
+      b.nrows = two ? l.npairs : l.nsingles;                                                                        \
+      const FsGrid g = fstage_grid(groups, b.nrows, FsShape<Lv>::PW);                                               \
+      const dim3 grid(g.x, g.y);                                                                                    \
       if (nbits == 2) hipLaunchKernelGGL((k_fstage_lin<Lv, 2>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);         \
       else hipLaunchKernelGGL((k_fstage_lin<Lv, 8>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);                    \
       break;                                                                                                        \
@@ -931,10 +931,12 @@ hipError_t launch_fstage_lin_c(int L, int nbits, const FStageArgs& a, const Band
   FStageArgs b = a;
   b.nchunk = nblocks;
   b.pairs = l.singles;
+  b.nrows = l.nsingles;
   switch (L) {
 #define X(Lv)                                                                                                       \
     case Lv: {                                                                                                      \
-      const dim3 grid((unsigned)((nblocks + 8 * FsShape<Lv>::NB - 1) / (8 * FsShape<Lv>::NB) * 8), l.nsingles);     \
+      const FsGrid g = fstage_grid((nblocks + FsShape<Lv>::NB - 1) / FsShape<Lv>::NB, l.nsingles, 1);               \
+      const dim3 grid(g.x, g.y);                                                                                    \
       if (nbits == 2) hipLaunchKernelGGL((k_fstage_lin_c<Lv, 2>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);       \
       else hipLaunchKernelGGL((k_fstage_lin_c<Lv, 8>), grid, dim3(FsShape<Lv>::NT), 0, stream, b);                  \
       break;                                                                                                        \

@@ -54,7 +54,8 @@ struct FStageArgs {
   const float2* base;         // last-pass twiddles at d = 0, per thread
   const float4* quad;         // levels of four 2-bit samples by their byte: VDIF, Mark5B
   int nchunk;                 // blocks of the launch
-  const int2* pairs;          // global bands of each grid row: two of one rotation, or one (y < 0)
+  const int2* pairs;          // global bands of each row of workgroups: two of one rotation, or one (y < 0)
+  int nrows;
 };
 // the same bands for launch_fstage_lin, in pairs of one rotation and one by one
 struct BandLists {
