@@ -1,5 +1,5 @@
-// fx_place.h — which blocks a workgroup of the F stage takes, shared by the
-// kernels and host-side tests.
+// fx_place.h — which blocks a workgroup of the F stage takes and which rows of V
+// one of the cross-multiply stores, shared by the kernels and host-side tests.
 #pragma once
 #include "fx_bits.h"
 
@@ -28,5 +28,10 @@ FXG_HD FsPlace fstage_place(unsigned x, unsigned y, unsigned gx, unsigned groups
   const unsigned k = x / (8 * PW), pw = x / 8 % PW;
   return groups < 8 ? FsPlace{8 * k + x % 8, y, pw} : FsPlace{y, (groups < 64 ? x + y : x) % 8 * (gx / (8 * PW)) + k, pw};
 }
+
+// The turns of 8 rows in which a 32-row tile of V is stored, with `left` inputs
+// from its first row on: 2 inputs, 32768 channels, one block 38 us a launch with
+// all four turns, 29 with one.
+FXG_HD int tile_turns(int left) { return left <= 0 ? 0 : left < 32 ? (left + 7) / 8 : 4; }
 
 }  // namespace fxg

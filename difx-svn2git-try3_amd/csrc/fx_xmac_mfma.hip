@@ -16,6 +16,7 @@
 // one 16-byte LDS read.
 #include <hip/hip_runtime.h>
 #include "fx_kernels.h"
+#include "fx_place.h"
 
 namespace fxg {
 
@@ -192,9 +193,11 @@ __device__ __forceinline__ void store_tiles32(float2* buf, const ACC (&re)[TL::N
   const int tid = threadIdx.x, w = tid >> 6, half = (tid & 63) >> 5, row = tid & 31;
   const int ch = tid % CG, p0 = tid / CG;
 #pragma unroll
-  for (int k = 0; k < TL::N; k++)
+  for (int k = 0; k < TL::N; k++) {
+    const int turns = tile_turns(nin - input_of(32 * TL::I(k)));
 #pragma unroll
     for (int g = 0; g < 4; g++) {
+      if (g >= turns) break;                                // the whole workgroup
       float2* const B = buf + (g & 1) * 256 * PS;
       // pair p0 + 64 i: rows a + 2 i of column b
       const int a = input_of(32 * TL::I(k) + 8 * g + (p0 >> 5)), b = input_of(32 * TL::J(k) + (p0 & 31));
@@ -219,6 +222,9 @@ __device__ __forceinline__ void store_tiles32(float2* buf, const ACC (&re)[TL::N
           ptr[i * step] = v;
         }
     }
+    // after an odd number of turns the next tile writes the buffer just read
+    if (k + 1 < TL::N && (turns & 1)) lds_barrier();
+  }
 }
 
 template <int T, bool BF, bool CROSS>

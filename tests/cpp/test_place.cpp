@@ -1,6 +1,7 @@
 // fstage_place (fx_place.h): every workgroup's share of every group of blocks
 // is taken once, those of one group lie on one XCD and so do the neighbouring
 // groups of an eighth of a row, and a launch of few groups uses every XCD alike.
+// tile_turns: every row of V with an input is stored, and no turn has none.
 #include <algorithm>
 #include <cstdio>
 #include <vector>
@@ -43,6 +44,9 @@ int main() {
           if (!bad) printf("%u groups, %u rows, %u a group: %d\n", groups, rows, PW, e);
           bad++;
         }
+  for (int nin = 1; nin <= 130; nin++)
+    for (int row0 = 0; row0 < 128; row0 += 32)
+      for (int g = 0; g < 4; g++) bad += (row0 + 8 * g < nin) != (g < fxg::tile_turns(nin - row0));
   printf("%s: %d\n", bad ? "FAIL" : "PASS", bad);
   return bad ? 1 : 0;
 }
