@@ -127,57 +127,54 @@ __device__ __forceinline__ float add_ones(float acc, int n) {
 }
 
 // One workgroup per entry.  The sums are FP32 in block order, a serial chain
-// (the reference's rounding), but nearly every term is 0 or 1: all wavefronts
-// sort 4096 terms into masks by 64, and the first adds the ones of all of them
-// at once, or, where there are other terms, goes through them in order; the
-// next terms load meanwhile.  The weights come from their own array: out of the
-// 80-byte block records the lines alone took a CU 100 us.  10 entries of 62500
-// blocks: 474 us one addition at a time -> 42.
+// (the reference's rounding), but in most streams nearly every term is 0 or 1:
+// all wavefronts sort 4096 terms into masks by 64, and the first adds the ones
+// of all of them at once; a group of 64 with any other term it adds in order,
+// its terms read beforehand (odd term by odd term took twice as long as one
+// addition at a time where most are odd).  The next terms load meanwhile.  The
+// weights come from their own array: out of the 80-byte block records the lines
+// alone took a CU 100 us.  20000 blocks, against one addition at a time: all ones
+// 144 -> 14 us, a fifth of short frames lost 140 -> 74, bands blanked in every
+// third (INTERLACEDVDIF) 150 -> 79.
 __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ st,
                                                  const DevStationSub* __restrict__ ss,
                                                  const float* __restrict__ bw, int nblocks,
                                                  const DevWTerm* __restrict__ terms, int nterms,
                                                  float* __restrict__ wout) {
   constexpr int CH = 4096, PER = CH / 256;
-  __shared__ float term[CH];
+  __shared__ __align__(16) float term[CH];
   __shared__ unsigned long long ones[CH / 64], odd[CH / 64];
   const int i = blockIdx.x;
   if (i >= nterms) return;
   const DevWTerm T = terms[i];
   const int lane = threadIdx.x & 63;
-  float v[PER];
-  // the weights of one side: bw, negative where a block was not processed, and
-  // the band's own in its place
-  auto side = [&](int d, int b, int t0, float (&w)[PER]) {
+  // each side's weights: bw, negative where a block was not processed, and the
+  // band's own in its place
+  float w1[PER], w2[PER], o1[PER], o2[PER];
+  auto fetch = [&](int d, int b, int t0, float (&w)[PER], float (&o)[PER]) {
     const float* const src = bw + (long long)d * nblocks;
 #pragma unroll
     for (int q = 0; q < PER; q++) w[q] = src[min(t0 + q * 256 + (int)threadIdx.x, nblocks - 1)];
-    if (b >= 0) {
-      const float* const own = ss[d].pbw + b;
-      const int nchan = st[d].nchan;
+    if (b < 0) return;
+    const float* const own = ss[d].pbw + b;
+    const int nchan = st[d].nchan;
 #pragma unroll
-      for (int q = 0; q < PER; q++)
-        if (w[q] >= 0.0f) w[q] = own[(long long)min(t0 + q * 256 + (int)threadIdx.x, nblocks - 1) * nchan];
-    }
-#pragma unroll
-    for (int q = 0; q < PER; q++) w[q] = fmaxf(w[q], 0.0f);
+    for (int q = 0; q < PER; q++) o[q] = own[(long long)min(t0 + q * 256 + (int)threadIdx.x, nblocks - 1) * nchan];
   };
   auto load = [&](int t0) {
-    side(T.d1, T.b1, t0, v);
-    if (T.d2 >= 0) {
-      float w[PER];
-      side(T.d2, T.b2, t0, w);
-#pragma unroll
-      for (int q = 0; q < PER; q++) v[q] *= w[q];
-    }
+    fetch(T.d1, T.b1, t0, w1, o1);
+    if (T.d2 >= 0) fetch(T.d2, T.b2, t0, w2, o2);
   };
+  auto weight = [](int b, float w, float o) { return w < 0.0f ? 0.0f : b >= 0 ? o : w; };
   float acc = 0.0f;
   if (nblocks > 0) load(0);
   for (int t0 = 0; t0 < nblocks; t0 += CH) {
 #pragma unroll
     for (int q = 0; q < PER; q++) {
       const int k = q * 256 + threadIdx.x;
-      const float x = t0 + k < nblocks ? v[q] : 0.0f;
+      float x = weight(T.b1, w1[q], o1[q]);
+      if (T.d2 >= 0) x *= weight(T.b2, w2[q], o2[q]);
+      if (t0 + k >= nblocks) x = 0.0f;
       term[k] = x;
       const unsigned long long o = __ballot(x == 1.0f), z = __ballot(x != 0.0f) & ~o;
       if (lane == 0) { ones[k >> 6] = o; odd[k >> 6] = z; }
@@ -185,7 +182,8 @@ __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ 
     __syncthreads();
     if (t0 + CH < nblocks) load(t0 + CH);
     if (threadIdx.x < 64) {
-      int n = __popcll(ones[lane]);
+      const int own = __popcll(ones[lane]);
+      int n = own;
       unsigned long long mixed = __ballot(odd[lane] != 0ull);
       // the ones before group g are added together, then its terms in order
 #pragma unroll
@@ -197,25 +195,21 @@ __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ 
       while (mixed) {
         const int g = __builtin_ctzll(mixed);
         mixed &= mixed - 1ull;
-        unsigned long long left = ones[g], rest = odd[g];
-        acc = add_ones(acc, __shfl(n, g) - __popcll(left) - done);
-        done = __shfl(n, g);
-        if (__popcll(rest) > 16) {
-#pragma unroll 16
-          for (int j = 0; j < 64; j++) acc += term[64 * g + j];
-          continue;
+        float4 t[16];
+#pragma unroll
+        for (int j = 0; j < 16; j++) t[j] = ((const float4*)term)[16 * g + j];
+        const int upto = __builtin_amdgcn_readlane(n, g);
+        acc = add_ones(acc, upto - __builtin_amdgcn_readlane(own, g) - done);
+        done = upto;
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+          acc += t[j].x;
+          acc += t[j].y;
+          acc += t[j].z;
+          acc += t[j].w;
         }
-        while (rest) {
-          const int b = __builtin_ctzll(rest);
-          const unsigned long long below = (1ull << b) - 1ull;
-          acc = add_ones(acc, __popcll(left & below));
-          acc += term[64 * g + b];
-          left &= ~below;
-          rest &= rest - 1ull;
-        }
-        acc = add_ones(acc, __popcll(left));
       }
-      acc = add_ones(acc, __shfl(n, 63) - done);
+      acc = add_ones(acc, __builtin_amdgcn_readlane(n, 63) - done);
     }
     __syncthreads();
   }
