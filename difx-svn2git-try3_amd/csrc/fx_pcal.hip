@@ -28,13 +28,15 @@ namespace fxg {
 // k_pcal_few: the same sums for bands of at most kPcalFewBins bins, the usual
 // comb (1 MHz spacing has 2 x bandwidth/MHz bins).  A thread per bin leaves
 // most of a workgroup idle there and walks the block in a serial chain of
-// loads, so here a wavefront (more than 64 bins: the workgroup) takes one
-// block, its threads split into slices over the bins, each thread's bin kept
-// in a register over all blocks of the group and its samples' loads in flight
-// eight at a time; the slices are added in order at the end.  Bound by the
-// loads' latency at 4 wavefronts a workgroup, 8 KB of LDS.
+// loads, so here a wavefront takes one block (the workgroup does, with more
+// than 64 bins or fewer blocks in the group than wavefronts), its threads split
+// into slices over the bins, each thread's bin kept in a register over all
+// blocks of the group and its samples' loads in flight eight at a time; the
+// slices are added in order at the end (2 KB of LDS).
 // 6 stations x 8 bands of 32 bins, 8001 blocks of 1024 samples (0.39
-// Gsamples): 12.0 -> 0.50 ms.
+// Gsamples): 12.0 -> 0.50 ms.  25 blocks of 8192 8-bit samples of 5 bands of 64
+// bins, a third of the frames lost: a thread per bin 80 us, a wavefront a block
+// 98, the workgroup 36.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_pcal_few(PcalArgs A) {
   __shared__ float2 acc[256];
@@ -43,7 +45,7 @@ __global__ __launch_bounds__(256) void k_pcal_few(PcalArgs A) {
   if (N > kPcalFewBins) return;
   const int g = blockIdx.y;
   const DevBand B = A.bands[pc.gband];
-  const DevStation& S = A.st[B.station];
+  const DevStation S = A.st[B.station];
   const DevStationSub Q = A.ss[B.station];
   const int L = S.L, nbits = S.nbits;
   const int per = (A.nblocks + A.ngroups - 1) / A.ngroups;
@@ -55,13 +57,13 @@ __global__ __launch_bounds__(256) void k_pcal_few(PcalArgs A) {
   const unsigned cmask = (1u << UB) - 1u;
   const float* lutc = nbits == 8 ? A.lut8 : A.st[B.station].lut;
   // threads of one block, its slices, and this thread's bin and slice
-  const int team = N <= 64 ? 64 : 256, nteam = 256 / team;
+  const int team = N <= 64 && per > 3 ? 64 : 256, nteam = 256 / team;
   const int mine = __builtin_amdgcn_readfirstlane(tid / team), lane = tid % team;
   const int slices = team / N, sl = lane / N, b = lane - sl * N;
   const int step = N * slices;
   float ar = 0.0f, ai = 0.0f;
   for (int blk = blk0 + mine; blk < blk1; blk += nteam) {
-    const DevBlock& G = A.blocks[(long long)B.station * A.nblocks + blk];
+    const DevBlock G = A.blocks[(long long)B.station * A.nblocks + blk];
     if (G.status != 0) continue;                 // Mode::process returned before the extraction
     const long long t0 = G.nearestsample;
     const long long so = (long long)Q.datasamples + t0;
