@@ -126,16 +126,82 @@ __device__ __forceinline__ float add_ones(float acc, int n) {
   return acc;
 }
 
-// One workgroup per entry.  The sums are FP32 in block order, a serial chain
-// (the reference's rounding), but in most streams nearly every term is 0 or 1:
-// all wavefronts sort 4096 terms into masks by 64, and the first adds the ones
-// of all of them at once; a group of 64 with any other term it adds in order,
-// its terms read beforehand (odd term by odd term took twice as long as one
-// addition at a time where most are odd).  The next terms load meanwhile.  The
-// weights come from their own array: out of the 80-byte block records the lines
-// alone took a CU 100 us.  20000 blocks, against one addition at a time: all ones
-// 144 -> 14 us, a fifth of short frames lost 140 -> 74, bands blanked in every
-// third (INTERLACEDVDIF) 150 -> 79.
+// An entry's terms of N blocks a thread, STEP apart: both sides' weights are loaded
+// together (bw, negative where a block was not processed, and the band's own in
+// its place) and multiplied when they are used.  The weights come from their own
+// array: out of the 80-byte block records the lines alone took a CU 100 us.
+template <int N, int STEP>
+struct WeightTerms {
+  static constexpr bool few = STEP == 64;          // loads wholly past the last block are left out
+  const DevWTerm T;
+  const float *bw1, *bw2, *own1, *own2;
+  int nchan1, nchan2;
+  const int nblocks, at;
+  float w1[N], w2[N], o1[N], o2[N];
+  __device__ __forceinline__ WeightTerms(const DevStation* st, const DevStationSub* ss, const float* bw, int nblocks,
+                                         const DevWTerm& T, int at)
+      : T(T), nblocks(nblocks), at(at) {
+    bw1 = bw + (long long)T.d1 * nblocks;
+    if (T.b1 >= 0) { own1 = ss[T.d1].pbw + T.b1; nchan1 = st[T.d1].nchan; }
+    if (T.d2 < 0) return;
+    bw2 = bw + (long long)T.d2 * nblocks;
+    if (T.b2 >= 0) { own2 = ss[T.d2].pbw + T.b2; nchan2 = st[T.d2].nchan; }
+  }
+  __device__ __forceinline__ void side(int t0, const float* src, bool band, const float* own, int nchan, float (&w)[N],
+                                       float (&o)[N]) {
+#pragma unroll
+    for (int q = 0; q < N; q++)
+      if (!few || t0 + q * STEP < nblocks) w[q] = src[min(t0 + q * STEP + at, nblocks - 1)];
+    if (!band) return;
+#pragma unroll
+    for (int q = 0; q < N; q++)
+      if (!few || t0 + q * STEP < nblocks) o[q] = own[(long long)min(t0 + q * STEP + at, nblocks - 1) * nchan];
+  }
+  __device__ __forceinline__ void load(int t0) {
+    side(t0, bw1, T.b1 >= 0, own1, nchan1, w1, o1);
+    if (T.d2 >= 0) side(t0, bw2, T.b2 >= 0, own2, nchan2, w2, o2);
+  }
+  __device__ __forceinline__ float term(int t0, int q) const {
+    if (t0 + q * STEP + at >= nblocks) return 0.0f;
+    const float x = w1[q] < 0.0f ? 0.0f : T.b1 >= 0 ? o1[q] : w1[q];
+    if (T.d2 < 0) return x;
+    return x * (w2[q] < 0.0f ? 0.0f : T.b2 >= 0 ? o2[q] : w2[q]);
+  }
+};
+
+// acc + 64 terms in order, read together beforehand
+struct Terms64 {
+  float4 t[16];
+  __device__ __forceinline__ explicit Terms64(const float* p) {
+#pragma unroll
+    for (int j = 0; j < 16; j++) t[j] = ((const float4*)p)[j];
+  }
+  __device__ __forceinline__ float add(float acc) const {
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+      acc += t[j].x;
+      acc += t[j].y;
+      acc += t[j].z;
+      acc += t[j].w;
+    }
+    return acc;
+  }
+};
+
+// The sums are FP32 in block order, a serial chain (the reference's rounding), but
+// in most streams nearly every term is 0 or 1: terms are sorted into masks by 64,
+// the ones of many groups are added at once, and a group with any other term is
+// added in order (odd term by odd term took twice as long as one addition at a
+// time where most are odd).  The next terms load meanwhile.
+//   k_weights: a workgroup an entry, 4096 terms at a time, for long sums of few
+// entries; bound by the one wavefront that adds.  20000 blocks, against one
+// addition at a time: all ones 144 -> 15 us, a fifth of short frames lost 140 ->
+// 75, bands blanked in every third (INTERLACEDVDIF) 150 -> 80.
+//   k_weights_w: a wavefront an entry, 512 terms at a time, for up to 1024 blocks,
+// where the other's barriers and empty wavefronts cost more (9 stations of 16
+// bands, INTERLACEDVDIF, 300 blocks 18 us, this 9), and for more than 1024
+// entries, where four times as many fit the chip (2000 blocks 36 and 23; 9
+// stations of 4 bands 15 and 18).
 __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ st,
                                                  const DevStationSub* __restrict__ ss,
                                                  const float* __restrict__ bw, int nblocks,
@@ -146,41 +212,21 @@ __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ 
   __shared__ unsigned long long ones[CH / 64], odd[CH / 64];
   const int i = blockIdx.x;
   if (i >= nterms) return;
-  const DevWTerm T = terms[i];
   const int lane = threadIdx.x & 63;
-  // each side's weights: bw, negative where a block was not processed, and the
-  // band's own in its place
-  float w1[PER], w2[PER], o1[PER], o2[PER];
-  auto fetch = [&](int d, int b, int t0, float (&w)[PER], float (&o)[PER]) {
-    const float* const src = bw + (long long)d * nblocks;
-#pragma unroll
-    for (int q = 0; q < PER; q++) w[q] = src[min(t0 + q * 256 + (int)threadIdx.x, nblocks - 1)];
-    if (b < 0) return;
-    const float* const own = ss[d].pbw + b;
-    const int nchan = st[d].nchan;
-#pragma unroll
-    for (int q = 0; q < PER; q++) o[q] = own[(long long)min(t0 + q * 256 + (int)threadIdx.x, nblocks - 1) * nchan];
-  };
-  auto load = [&](int t0) {
-    fetch(T.d1, T.b1, t0, w1, o1);
-    if (T.d2 >= 0) fetch(T.d2, T.b2, t0, w2, o2);
-  };
-  auto weight = [](int b, float w, float o) { return w < 0.0f ? 0.0f : b >= 0 ? o : w; };
+  WeightTerms<PER, 256> W(st, ss, bw, nblocks, terms[i], threadIdx.x);
   float acc = 0.0f;
-  if (nblocks > 0) load(0);
+  W.load(0);
   for (int t0 = 0; t0 < nblocks; t0 += CH) {
 #pragma unroll
     for (int q = 0; q < PER; q++) {
       const int k = q * 256 + threadIdx.x;
-      float x = weight(T.b1, w1[q], o1[q]);
-      if (T.d2 >= 0) x *= weight(T.b2, w2[q], o2[q]);
-      if (t0 + k >= nblocks) x = 0.0f;
+      const float x = W.term(t0, q);
       term[k] = x;
       const unsigned long long o = __ballot(x == 1.0f), z = __ballot(x != 0.0f) & ~o;
       if (lane == 0) { ones[k >> 6] = o; odd[k >> 6] = z; }
     }
     __syncthreads();
-    if (t0 + CH < nblocks) load(t0 + CH);
+    if (t0 + CH < nblocks) W.load(t0 + CH);
     if (threadIdx.x < 64) {
       const int own = __popcll(ones[lane]);
       int n = own;
@@ -195,25 +241,67 @@ __global__ __launch_bounds__(256) void k_weights(const DevStation* __restrict__ 
       while (mixed) {
         const int g = __builtin_ctzll(mixed);
         mixed &= mixed - 1ull;
-        float4 t[16];
-#pragma unroll
-        for (int j = 0; j < 16; j++) t[j] = ((const float4*)term)[16 * g + j];
+        const Terms64 t(term + 64 * g);
         const int upto = __builtin_amdgcn_readlane(n, g);
-        acc = add_ones(acc, upto - __builtin_amdgcn_readlane(own, g) - done);
+        acc = t.add(add_ones(acc, upto - __builtin_amdgcn_readlane(own, g) - done));
         done = upto;
-#pragma unroll
-        for (int j = 0; j < 16; j++) {
-          acc += t[j].x;
-          acc += t[j].y;
-          acc += t[j].z;
-          acc += t[j].w;
-        }
       }
       acc = add_ones(acc, __builtin_amdgcn_readlane(n, 63) - done);
     }
     __syncthreads();
   }
   if (threadIdx.x == 0) wout[i] = acc;
+}
+
+constexpr int kWeightWaves = 4;                    // entries of a workgroup of k_weights_w
+
+__global__ __launch_bounds__(64 * kWeightWaves) void k_weights_w(const DevStation* __restrict__ st,
+                                                                 const DevStationSub* __restrict__ ss,
+                                                                 const float* __restrict__ bw, int nblocks,
+                                                                 const DevWTerm* __restrict__ terms, int nterms,
+                                                                 float* __restrict__ wout) {
+  constexpr int NG = 8;
+  __shared__ __align__(16) float lds[kWeightWaves][64 * NG];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i = blockIdx.x * kWeightWaves + wave;
+  if (i >= nterms) return;                         // the whole wavefront; no barrier below
+  WeightTerms<NG, 64> W(st, ss, bw, nblocks, terms[i], lane);
+  float* const term = lds[wave];
+  float acc = 0.0f;
+  W.load(0);
+  for (int t0 = 0; t0 < nblocks; t0 += 64 * NG) {
+    unsigned long long one[NG], odd[NG], any = 0ull;
+#pragma unroll
+    for (int q = 0; q < NG; q++) {
+      const float x = W.term(t0, q);
+      term[q * 64 + lane] = x;
+      one[q] = __ballot(x == 1.0f);
+      odd[q] = __ballot(x != 0.0f) & ~one[q];
+      any |= odd[q];
+    }
+    if (t0 + 64 * NG < nblocks) W.load(t0 + 64 * NG);
+    // a wavefront's own LDS accesses complete in order: this orders the compiler's
+    auto order = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    int n = 0;                                     // ones not yet added
+    if (any != 0ull) order();
+#pragma unroll
+    for (int q = 0; q < NG; q++) {
+      if (odd[q] == 0ull) {
+        n += __popcll(one[q]);
+        continue;
+      }
+      const Terms64 t(term + 64 * q);
+      acc = t.add(add_ones(acc, n));
+      n = 0;
+    }
+    if (any != 0ull) order();
+    acc = add_ones(acc, n);
+  }
+  if (lane == 0) wout[i] = acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -343,7 +431,11 @@ hipError_t launch_zero(float* p, long long n, hipStream_t stream) {
 hipError_t launch_weights(const DevStation* st, const DevStationSub* ss, const float* bw, int nblocks,
                           const DevWTerm* terms, int nterms, float* w, hipStream_t stream) {
   if (nterms == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_weights, dim3(nterms), dim3(256), 0, stream, st, ss, bw, nblocks, terms, nterms, w);
+  if (nblocks > 1024 && nterms <= 1024)
+    hipLaunchKernelGGL(k_weights, dim3(nterms), dim3(256), 0, stream, st, ss, bw, nblocks, terms, nterms, w);
+  else
+    hipLaunchKernelGGL(k_weights_w, dim3((nterms + kWeightWaves - 1) / kWeightWaves), dim3(64 * kWeightWaves), 0, stream, st,
+                       ss, bw, nblocks, terms, nterms, w);
   return hipGetLastError();
 }
 
