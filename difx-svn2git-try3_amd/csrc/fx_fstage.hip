@@ -42,21 +42,22 @@ template <int COUNT>
 __device__ __forceinline__ unsigned valid_samples(const DevStation& S, const DevStationSub& Q,
                                                   const int2* __restrict__ ftab, long long t, long long validend,
                                                   int band) {
+  // sample numbers are below 2^31 + L, so 32-bit divisions do (3 bands of 65536 8-bit
+  // points, five blocks of a lossy stream 49 -> 45 us)
   unsigned m = 0u;
-  const long long end = min(t + COUNT, validend);
-  long long u = t < 0 ? 0 : t;
-  while (u < end) {
-    const long long f = u / S.framesamples;
-    if (f >= Q.nframes) break;
-    const long long base = f * (long long)S.framesamples;
-    const long long fe = min(end, base + S.framesamples);
+  if (t < 0 || t >= validend) return m;
+  const unsigned first = (unsigned)t, end = (unsigned)min(t + COUNT, validend), fs = (unsigned)S.framesamples;
+  for (unsigned u = first; u < end;) {
+    const unsigned f = u / fs, base = f * fs, fe = min(end, base + fs);
+    if ((long long)f >= Q.nframes) break;
     const int2 z = ftab[Q.fbase + f];
     const bool blank = Q.fblank && ((Q.fblank[f] >> band) & 1ull);
     if (z.x < z.y && !blank) {
-      const long long g0 = ((long long)z.x + S.groupbytes - 1) / S.groupbytes;
-      const long long g1 = ((long long)z.y + S.groupbytes - 1) / S.groupbytes;
-      const long long a = max(u, base + g0 * S.groupsamples), b = min(fe, base + g1 * S.groupsamples);
-      if (b > a) m |= (((1u << (int)(b - a)) - 1u) << (int)(a - t));
+      const unsigned gb = (unsigned)S.groupbytes, gs = (unsigned)S.groupsamples;
+      const unsigned g0 = ((unsigned)min(z.x, S.databytes) + gb - 1) / gb;
+      const unsigned g1 = ((unsigned)min(z.y, S.databytes) + gb - 1) / gb;
+      const unsigned a = max(u, base + g0 * gs), b = min(fe, base + g1 * gs);
+      if (b > a) m |= ((1u << (b - a)) - 1u) << (a - first);
     }
     u = fe;
   }

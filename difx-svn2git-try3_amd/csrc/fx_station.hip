@@ -209,14 +209,10 @@ __device__ __forceinline__ DevBlock block_geometry(const DevStation& S, const De
     }
   }
   long long tcut = min(tend, g.validend);
-  while (t < tcut) {
-    long long f = t / S.framesamples;
-    long long fe = min(tcut, (f + 1) * (long long)S.framesamples);
-    if (f < Q.nframes) {
-      int2 z = ftab[Q.fbase + f];
-      long long base = f * (long long)S.framesamples;
-      good += valid_in_frame(S, z, t - base, fe - base);
-    }
+  long long fr = t / S.framesamples;
+  for (long long base = fr * S.framesamples; t < tcut; fr++, base += S.framesamples) {
+    const long long fe = min(tcut, base + S.framesamples);
+    if (fr < Q.nframes) good += valid_in_frame(S, ftab[Q.fbase + fr], t - base, fe - base);
     t = fe;
   }
   g.weight = (float)good / (float)S.L;
