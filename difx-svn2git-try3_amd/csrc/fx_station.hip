@@ -815,6 +815,9 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage(FStageArgs A) {
         for (int i = 0; i < jj; i++) piece = cmulf(piece, qd);
         const float2 rot = cmulf(piece, rstep[jj]);
         v[r] = make_float2(x * rot.x, x * rot.y);
+        // finished before the next point is begun, for registers: gathered, the
+        // points' reads leave four wavefronts a SIMD up to 256 points, not five
+        asm volatile("" : "+v"(v[r].x), "+v"(v[r].y) :: "memory");
       }
     }
     DFT<16>::run(v);
