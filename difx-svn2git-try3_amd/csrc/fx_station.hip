@@ -533,9 +533,10 @@ __device__ __forceinline__ float2 angle_rotator(float x) {
 }
 
 // C: the recorded channels, L/2 (real) or L (complex) -- a compile-time
-// power of two at every call, so the divisions by it are exact products
+// power of two at every call, so the divisions by it are exact products; linear:
+// order 1 (16384 complex channels alone come here with it), else order 2
 __device__ __forceinline__ void rotator_tables(const DevBand& B, const DevStation& S, const DevBlock& G, int L,
-                                               int C, int tid, int NT, float2* rsub,
+                                               int C, bool linear, int tid, int NT, float2* rsub,
                                                float2* rstep, float2* fsub, float2* fstep, float2* rquad) {
 #pragma clang fp contract(off)
   const int s = S.s;
@@ -563,7 +564,7 @@ __device__ __forceinline__ void rotator_tables(const DevBand& B, const DevStatio
     if (e < e1) {
       const int k = e;
       const double subxoff = (double)k / (double)L;
-      double ph = (S.order == 1 ? subxoff * G.a + G.b : subxoff * (G.b + G.a * stepxoff1) + G.c) * lofreq;
+      double ph = (linear ? subxoff * G.a + G.b : subxoff * (G.b + G.a * stepxoff1) + G.c) * lofreq;
       if (S.fractionalLo) ph += (lofreq - (int)lofreq) * (double)G.integerdelay;
       if (looff) {
         ph += ((k * S.sampletime) / 1e6) * (-looffset);
@@ -572,14 +573,14 @@ __device__ __forceinline__ void rotator_tables(const DevBand& B, const DevStatio
       }
       // phase -2 pi frac(ph) (mode.cpp:962-967), as turns
       rsub[k] = turn_rotator((float)((double)(int)ph - ph));
-      if (S.order == 2) {
+      if (!linear) {
         const double qph = (subxoff * (2 * G.a * stepxoff1)) * lofreq;
         rquad[k] = turn_rotator((float)((double)(int)qph - qph));
       }
     } else if (e < e2) {
       const int j = e - e1;
       const double stepxoff = ((double)(j * s)) / (double)L;
-      double ph = (S.order == 1 ? stepxoff * G.a : stepxoff * G.b + (stepxoff * stepxoff) * G.a) * lofreq;
+      double ph = (linear ? stepxoff * G.a : stepxoff * G.b + (stepxoff * stepxoff) * G.a) * lofreq;
       if (looff) ph += (((j * s) * S.sampletime) / 1e6) * (-looffset);
       rstep[j] = turn_rotator((float)((double)(int)ph - ph));
     } else if (e < e3) {
@@ -744,7 +745,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage(FStageArgs A) {
   float2* rquad = fstep + S.nfracsteps;         // order 2 only
 
   // ---- rotator tables: FP64 phase, FP32 residual (mode.cpp:909-978, 1054-1097)
-  rotator_tables(B, S, G, L, L / 2, tid, NT, rsub, rstep, fsub, fstep, rquad);
+  rotator_tables(B, S, G, L, L / 2, false, tid, NT, rsub, rstep, fsub, fstep, rquad);
   ts.store(twlo, twhi, tw256, lut8s, tid);
   if (fast) {
 #pragma unroll
@@ -1004,7 +1005,8 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
   float2* fsub = rstep + S.nfrsteps;
   float2* fstep = fsub + S.s;
   float2* rquad = fstep + S.nfracsteps;
-  rotator_tables(B, S, G, L, L, tid, NT, rsub, rstep, fsub, fstep, rquad);
+  const bool linear = L > kFStageLinCMax && S.order == 1;     // shorter ones: k_fstage_lin_c
+  rotator_tables(B, S, G, L, L, linear, tid, NT, rsub, rstep, fsub, fstep, rquad);
   ts.store(twlo, twhi, tw256, lut8s, tid);
   if (fast) {
 #pragma unroll
@@ -1034,7 +1036,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
       const int k = j & (s - 1), q0 = j >> slog, sstep = NTF >> slog;
       float2 piece = rsub[k];
       float2 qd = make_float2(1.0f, 0.0f);
-      if (S.order == 2) {
+      if (!linear) {
         qd = rquad[k];
         for (int i = 0; i < q0; i++) piece = cmulf(piece, qd);
       }
@@ -1043,10 +1045,10 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
       for (int r = 0; r < 16; r++) {
         const unsigned code = (wp[r * WSTEP] >> sh) & ((1u << UB) - 1u);
         const float2 x = make_float2(lut8s[code & ((1u << NBITS) - 1u)], lut8s[code >> NBITS]);
-        const float2 rot = cmulf(piece, *stp);  // sub[k] step[j] (order 2: piece_j[k] step[j])
+        const float2 rot = cmulf(piece, *stp);  // sub[k] step[j] (quadratic: piece_j[k] step[j])
         stp += sstep;
         v[r] = cmulf(rot, x);
-        if (S.order == 2 && r < 15)
+        if (!linear && r < 15)
           for (int i = 0; i < sstep; i++) piece = cmulf(piece, qd);
       }
     } else {
@@ -1068,7 +1070,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
         const int kk = slog >= 0 ? (n & (s - 1)) : n % s;
         const int jj = slog >= 0 ? (n >> slog) : n / s;
         float2 rot;
-        if (S.order == 1) {
+        if (linear) {
           rot = n < s ? rsub[n] : cmulf(rsub[kk], rstep[jj]);
         } else {
           const float2 qd = rquad[kk];
@@ -1077,6 +1079,7 @@ __global__ __launch_bounds__(FftShape<L>::NT) void k_fstage_c(FStageArgs A) {
           rot = cmulf(piece, rstep[jj]);
         }
         v[r] = cmulf(rot, x);
+        asm volatile("" : "+v"(v[r].x), "+v"(v[r].y) :: "memory");   // as in k_fstage
       }
     }
     DFT<16>::run(v);
@@ -1193,7 +1196,7 @@ __global__ __launch_bounds__(256) void k_rotab(FStageArgs A) {
   const DevBlock G = A.blocks[(long long)B.station * A.nblocks_subint + blk];
   if (G.status != 0) return;
   float2* rt = A.rtab + ((long long)gband * A.zcap + cbl) * A.rtabn;
-  rotator_tables(B, S, G, L, L / 2, threadIdx.x, 256, rt, rt + S.s, rt + 2 * S.s + S.nfrsteps,
+  rotator_tables(B, S, G, L, L / 2, false, threadIdx.x, 256, rt, rt + S.s, rt + 2 * S.s + S.nfrsteps,
                  rt + 3 * S.s + S.nfrsteps, rt + S.s + S.nfrsteps);
 }
 
