@@ -117,7 +117,8 @@ struct fxg_job {
   DBuf d_pairs;                   // band lists of that F stage
   BandLists lists2, lists8;       // its 2-bit and 8-bit bands
   DBuf d_cdesc, d_base, d_quad;   // tables of the F stage with linear rotation (fx_fstage.hip)
-  bool fstage_lin = false;        // that F stage runs: real samples, fringe orders 0 and 1
+  bool fstage_lin = false;        // that F stage runs: real samples, fringe orders 0 and 1; complex ones, order 1,
+                                  // up to kFStageLinCMax
   DBuf d_bandlist;                // global bands grouped by sample size
   int nb2 = 0, nb8 = 0;           // bands of 2-bit and 8-bit datastreams
   std::vector<DBuf> d_raw;        // staged host data per datastream

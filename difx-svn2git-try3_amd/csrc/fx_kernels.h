@@ -11,8 +11,9 @@ namespace fxg {
 // LDS entries for an F-stage workgroup's rotator tables (sub, step,
 // fractional sub and step, quadratic pieces) at FFT length L
 constexpr int fxg_rotator_table_entries(int L) { return L >= 16384 ? 768 : 512; }
-// the largest FFT length of one workgroup; longer ones (to 65536) take
-// several (linear and post-F rotation) or the two-kernel path (quadratic)
+// the largest FFT length of one workgroup with quadratic rotation; longer ones
+// (to 65536) take the two-kernel path.  (Linear and post-F rotation: 8192 points,
+// above that several workgroups a block.)
 constexpr int kFStageMaxL = 16384;
 
 // Spectra layout.  Channel c of the spectrum of one (band, pass block) sits
@@ -154,8 +155,8 @@ hipError_t launch_prologue(const DevStation* st, const DevStationSub* ss, const 
                            const DevRotGroup* groups, DevRot* rots, hipStream_t stream);
 // cplx: complex samples (L = nchan, every output of the transform kept)
 hipError_t launch_fstage(int L, int nbits, int cplx, const FStageArgs& a, int nbands, int nblocks, hipStream_t stream);
-// linear and post-F rotation of real samples; its tables for
-// one length, and the levels of four 2-bit samples by their byte (256 entries)
+// linear and post-F rotation of real samples; the tables of one length (complex
+// samples have the same), and the levels of four 2-bit samples by their byte (256 entries)
 hipError_t launch_fstage_lin(int L, int nbits, const FStageArgs& a, const BandLists& l, int nblocks,
                              hipStream_t stream);
 // complex samples, up to kFStageLinCMax of them a block

@@ -629,8 +629,8 @@ int build_plan(const fxg_job_desc* d, Plan* p, std::string* err) {
     int nin = (int)x.in_station.size();
     DevSeg g{};
     g.kind = SEG_VIS; g.resoff = resoff; g.nchan = nchan; g.avg = avg;
-    // V is accumulated for a <= b tiles and in full inside diagonal tiles;
-    // read the upper triangle and conjugate when the order is swapped
+    // V holds the pairs a <= b alone (the rest is whatever was there): read
+    // those, and conjugate when the order is swapped
     if (a <= b) { g.voff = x.voff + ((long long)a * nin + b) * x.nchan + choff; g.conj = 0; }
     else        { g.voff = x.voff + ((long long)b * nin + a) * x.nchan + choff; g.conj = 1; }
     P.segs.push_back(g);

@@ -7,8 +7,8 @@
 //               Stockham FFT -> sideband select -> fractional-sample rotation
 //               -> spectra (mode.cpp:909-1310); k_fstage_c complex samples (and
 //               linear at 16384 channels); k_bigfft_a/b transforms above
-//               16384 points.  Real samples with
-//               linear or post-F rotation, complex ones with linear: fx_fstage.hip
+//               16384 points.  Real samples with linear or post-F rotation,
+//               complex ones with linear: fx_fstage.hip
 //   k_unpack    standalone Mk5Mode::unpack equivalent
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>

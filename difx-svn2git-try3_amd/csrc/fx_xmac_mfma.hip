@@ -354,8 +354,9 @@ __global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_dl(XmacArgs A,
 // a block and channel for up to 32 inputs and 6 x 64 for up to 64; these
 // 24 (16 inputs), 80 (32), 168 (48), 288 (64).
 // Rows past the last input are not read back (a row of A or B only reaches its
-// own row or column of the tile); they and blocks past the last read a 16-byte
-// zero buffer.  LDS is a ring of stages of 4 or 8 blocks x 16 channels x 16 T
+// own row or column of the tile): an instruction whose rows all lie past it is
+// not issued, and LDS holds there what it held; other such rows and blocks past
+// the last read a 16-byte zero buffer.  LDS is a ring of stages of 4 or 8 blocks x 16 channels x 16 T
 // rows, filled by global_load_lds, as deep as leaves two workgroups on a CU for
 // one and two tiles: there the load stream is the bound, above it the matrix
 // cores.  At 64 inputs two stages of 8 blocks: four of 4 take 382 against 414
