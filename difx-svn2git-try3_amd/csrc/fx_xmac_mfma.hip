@@ -358,10 +358,11 @@ __global__ __launch_bounds__(CROSS ? 512 : 1024) void k_xmac_mfma_dl(XmacArgs A,
 // not issued, and LDS holds there what it held; other such rows and blocks past
 // the last read a 16-byte zero buffer.  LDS is a ring of stages of 4 or 8 blocks x 16 channels x 16 T
 // rows, filled by global_load_lds, as deep as leaves two workgroups on a CU for
-// one and two tiles: there the load stream is the bound, above it the matrix
-// cores.  At 64 inputs two stages of 8 blocks: four of 4 take 382 against 414
-// us at 500 blocks, but 1661 against 1570 at 2000 (4096 channels, constant
-// data).
+// one and two tiles.  One tile is bound by the load stream (16 inputs 4.2 TB/s,
+// the matrix cores 32 % busy); two by both in part (20 inputs 2.5 TB/s and 61 %);
+// four by the matrix cores first.  At 64 inputs two stages of 8 blocks: four of 4
+// take 382 against 414 us at 500 blocks, but 1661 against 1570 at 2000 (4096
+// channels, constant data); the longer integration decides.
 // 10 stations, 1024 channels, 4096 blocks 327 -> 249 us a frequency; 32
 // stations, 4096 channels, 500 blocks 494 -> 440 us, 2000 blocks 1.74 -> 1.67 ms.
 // ---------------------------------------------------------------------------
